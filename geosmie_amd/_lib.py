@@ -97,6 +97,8 @@ SIGNATURES = {
                                          c_i64, c_dbl, c_vp, c_vp, c_vp]),
     "gm_surrogate_post": (ctypes.c_int, [c_vp, c_i64, ctypes.c_int, c_vp, c_dbl, c_vp, c_vp,
                                          c_vp, c_vp, c_vp]),
+    "gm_surrogate_rows": (ctypes.c_int, [c_vp, ctypes.c_int, c_vp, c_i64, c_vp, c_vp, c_vp, c_dbl,
+                                         c_vp, c_vp, c_vp, c_vp]),
     "gm_surrogate_targets": (ctypes.c_int, [c_vp, c_i64, ctypes.c_int, c_vp, c_dbl, c_vp, c_vp,
                                             c_vp, c_vp, c_vp]),
 }

@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "gm_ctx.h"
+#include "gm_surrogate.h"
 
 typedef __bf16 bf16x8_ __attribute__((ext_vector_type(8)));
 typedef float float4_ __attribute__((ext_vector_type(4)));
@@ -273,6 +274,530 @@ __global__ void k_mlp_adam(int64_t n, float* __restrict__ p, const float* __rest
   p[i] -= lr * (mi * c1) / (sqrtf(vi * c2) + eps);
 }
 
+
+// ---- fused network ----------------------------------------------------------
+//
+// Networks whose layers are all at most kFuseWidth wide run whole: a block
+// takes kFuseRows queries through every layer with the activations in LDS (as
+// the BF16 hi and lo planes that the products read), so nothing between the
+// input and the output rows goes through memory.  Layer by layer the 1M-query
+// forward pass wrote and read 10 GB of FP32 activations; what is left is
+// the weights, which every block streams from the L2.
+//
+// The weights are the MFMA's A operand and the activations its B operand:
+// a lane then holds four consecutive features of one query (D[4g + r][j] in
+// lane j + 16g), which it puts back into the planes with 8-byte stores.  The
+// four wavefronts split a layer's features; each multiplies all kFuseRows
+// queries, so a weight fragment it loads (16 bytes a lane, laid out for that
+// by k_mlp_split_weights) feeds four products per term.  64 rows: 67 KB of
+// planes, two blocks per CU, so one block's SiLU (as many VALU cycles as the
+// layer has MFMA cycles) runs under the other's products.
+//
+// Training runs the same block forward and back: dZ_l takes the activations'
+// place in LDS, SiLU'(z) waits in memory in the order the lane reads it, and
+// the planes of every layer's input and dZ are written out with the queries
+// contiguous, in the order the weight gradient's MFMAs (contraction over the
+// batch) load them.
+constexpr int kFuseWidth = 256;
+constexpr int kFuseRows = 64;
+constexpr int kFuseMt = kFuseRows / 16;
+constexpr int kFuseLd = kFuseWidth + 8;   // 528-byte rows: 16-byte fragments on distinct banks
+
+struct FuseNet {
+  int L, n_in, n_out;
+  int kt[kMlpMaxLayers], nt[kMlpMaxLayers];   // 32-wide input and 16-wide output tiles
+  int in[kMlpMaxLayers], out[kMlpMaxLayers];
+  int64_t woff[kMlpMaxLayers], boff[kMlpMaxLayers];   // parameters
+  int64_t wf[kMlpMaxLayers], wb[kMlpMaxLayers];       // fragments (16-byte units)
+  int64_t n_frag;                                     // 64-lane fragments of one term
+};
+
+struct FuseTrain {
+  const float* target;
+  const float* cw;
+  float4* ds;                     // SiLU'(z) [block][hidden tile][m][lane]
+  int ds_tile[kMlpMaxLayers];     // first hidden tile of a layer
+  int ds_tiles;                   // hidden tiles of all layers
+  unsigned short* at[kMlpMaxLayers];   // layer inputs, hi plane [batch / 32][feature][32]
+  unsigned short* gt[kMlpMaxLayers];   // dZ, likewise; the lo plane follows the hi plane
+  float* db;                      // bias gradient parts [bias][block]
+  int db_row[kMlpMaxLayers];
+  double* lpart;                  // loss parts [block]
+  int64_t nb;                     // blocks
+};
+
+struct FusePost {                 // output transform of the surrogate (rows instead of y)
+  const float* q;
+  const float* mean;
+  const float* std;
+  float mw_re;
+  int on;
+};
+
+__device__ __forceinline__ void bf_split(float v, __bf16& h, __bf16& l) {
+  h = (__bf16)v;
+  l = (__bf16)(v - (float)h);
+}
+
+// 1 / (1 + exp(-z)) by the hardware reciprocal and one Newton step (below 1 ulp);
+// the argument is kept where exp() is finite so that the step has no inf * 0.
+__device__ __forceinline__ float sigmoid_nr(float z) {
+  const float d = 1.0f + expf(fminf(-z, 85.0f));
+  const float r = __builtin_amdgcn_rcpf(d);
+  return fmaf(fmaf(-d, r, 1.0f), r, r);
+}
+
+// Weight fragments: forward F[nt][kt] = W[16 nt + i][32 kt + 8 kq + e] and, for
+// training, backward B[nt][kt] = W[32 kt + 8 kq + e][16 nt + i], lane i + 16 kq
+// holding its eight e as one 16-byte word; `terms` words (hi, lo) in turn.
+// Zero outside the layer.
+__global__ __launch_bounds__(256) void k_mlp_split_weights(FuseNet net, int terms, int backward,
+                                                           const float* __restrict__ params,
+                                                           uint4* __restrict__ frag) {
+  const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t per = net.n_frag * 64;
+  if (id >= per * (backward ? 2 : 1)) return;
+  const bool back = id >= per;
+  int64_t f = (back ? id - per : id) >> 6;
+  const int lane = (int)(id & 63), i = lane & 15, kq = lane >> 4;
+  int l = 0;
+  for (; l + 1 < net.L; ++l) {
+    const int64_t here = (int64_t)net.kt[l] * net.nt[l];
+    if (f < here) break;
+    f -= here;
+  }
+  // as many backward as forward fragments: both cover the padded layer
+  const int kts = back ? net.nt[l] / 2 : net.kt[l];
+  const int nt = (int)(f / kts), kt = (int)(f % kts);
+  const float* W = params + net.woff[l];
+  union { uint4 q; __bf16 s[8]; } h, lo;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int a = 16 * nt + i, k = 32 * kt + 8 * kq + e;
+    const int o = back ? k : a, in = back ? a : k;
+    const float v = (o < net.out[l] && in < net.in[l]) ? W[(int64_t)o * net.in[l] + in] : 0.f;
+    bf_split(v, h.s[e], lo.s[e]);
+  }
+  uint4* dst = frag + (back ? net.wb[l] : net.wf[l]) + ((int64_t)(nt * kts + kt) * terms) * 64 + lane;
+  dst[0] = h.q;
+  if (terms == 2) dst[64] = lo.q;
+}
+
+// acc[m][t] += weights tile nt0 + t (of NT) x activations rows 16 m.. over KT
+// steps; products act_hi w_hi, act_lo w_hi, (two terms) act_hi w_lo per step.
+template <int TN, int SB>
+__device__ __forceinline__ void fuse_mm(const uint4* __restrict__ wf, int KT, int NT, int nt0,
+                                        const unsigned short* __restrict__ sH,
+                                        const unsigned short* __restrict__ sL, int lane,
+                                        float4_ (&acc)[kFuseMt][TN]) {
+  union U { uint4 q; bf16x8_ v; };
+  const int i = lane & 15, kq = lane >> 4;
+  const uint4* p[TN];
+#pragma unroll
+  for (int t = 0; t < TN; ++t) {
+    p[t] = wf + (int64_t)min(nt0 + t, NT - 1) * KT * SB * 64 + lane;
+#pragma unroll
+    for (int m = 0; m < kFuseMt; ++m) acc[m][t] = (float4_){0.f, 0.f, 0.f, 0.f};
+  }
+  U wn[TN][SB];
+#pragma unroll
+  for (int t = 0; t < TN; ++t)
+#pragma unroll
+    for (int s = 0; s < SB; ++s) wn[t][s].q = p[t][s * 64];
+  for (int k = 0; k < KT; ++k) {
+    U wc[TN][SB], ah[kFuseMt], al[kFuseMt];
+#pragma unroll
+    for (int t = 0; t < TN; ++t)
+#pragma unroll
+      for (int s = 0; s < SB; ++s) wc[t][s] = wn[t][s];
+    if (k + 1 < KT) {
+#pragma unroll
+      for (int t = 0; t < TN; ++t)
+#pragma unroll
+        for (int s = 0; s < SB; ++s) wn[t][s].q = p[t][((k + 1) * SB + s) * 64];
+    }
+#pragma unroll
+    for (int m = 0; m < kFuseMt; ++m) {
+      const int at = (16 * m + i) * kFuseLd + 32 * k + 8 * kq;
+      ah[m].q = *(const uint4*)&sH[at];
+      al[m].q = *(const uint4*)&sL[at];
+    }
+#pragma unroll
+    for (int m = 0; m < kFuseMt; ++m)
+#pragma unroll
+      for (int t = 0; t < TN; ++t)
+        acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wc[t][0].v, ah[m].v, acc[m][t], 0, 0, 0);
+#pragma unroll
+    for (int m = 0; m < kFuseMt; ++m)
+#pragma unroll
+      for (int t = 0; t < TN; ++t)
+        acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wc[t][0].v, al[m].v, acc[m][t], 0, 0, 0);
+    if (SB == 2) {
+#pragma unroll
+      for (int m = 0; m < kFuseMt; ++m)
+#pragma unroll
+        for (int t = 0; t < TN; ++t)
+          acc[m][t] =
+              __builtin_amdgcn_mfma_f32_16x16x32_bf16(wc[t][SB - 1].v, ah[m].v, acc[m][t], 0, 0, 0);
+    }
+  }
+}
+
+__device__ __forceinline__ void fuse_put(unsigned short* __restrict__ sH,
+                                         unsigned short* __restrict__ sL, int row, int f,
+                                         const float (&v)[4]) {
+  union { uint2 q; __bf16 s[4]; } h, l;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) bf_split(v[r], h.s[r], l.s[r]);
+  *(uint2*)&sH[row * kFuseLd + f] = h.q;
+  *(uint2*)&sL[row * kFuseLd + f] = l.q;
+}
+
+// The planes' first F columns, transposed, to dst[block's two 32-row groups][F][32]
+// (hi; lo follows at lo_off): a thread takes one feature.
+__device__ __forceinline__ void fuse_export(const unsigned short* __restrict__ sH,
+                                            const unsigned short* __restrict__ sL, int F,
+                                            int64_t blk, unsigned short* __restrict__ dst,
+                                            int64_t lo_off) {
+  const int f = threadIdx.x;
+  if (f >= F) return;
+#pragma unroll
+  for (int pl = 0; pl < 2; ++pl) {
+    const unsigned short* src = pl ? sL : sH;
+#pragma unroll
+    for (int g = 0; g < kFuseRows / 32; ++g) {
+      uint4* o = (uint4*)(dst + (pl ? lo_off : 0) + ((blk * (kFuseRows / 32) + g) * F + f) * 32);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        unsigned w[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int b = 32 * g + 8 * c + 2 * e;
+          w[e] = src[b * kFuseLd + f] | ((unsigned)src[(b + 1) * kFuseLd + f] << 16);
+        }
+        o[c] = make_uint4(w[0], w[1], w[2], w[3]);
+      }
+    }
+  }
+}
+
+// One layer of a block, TN feature tiles per wavefront.
+template <int TN, int SB, bool TRAIN>
+__device__ __forceinline__ void fuse_forward(const FuseNet& net, int l, const uint4* __restrict__ frag,
+                                             const float* __restrict__ params, int64_t n,
+                                             int64_t blk, unsigned short* sH, unsigned short* sL,
+                                             float* __restrict__ y, const FuseTrain& tr,
+                                             const FusePost& post, const float* lnb, int wave,
+                                             int lane, double& lsum) {
+  const int NT = net.nt[l], nt0 = wave * TN;
+  const int j = lane & 15, kq = lane >> 4;
+  float4_ acc[kFuseMt][TN];
+  if (nt0 < NT) fuse_mm<TN, SB>(frag + net.wf[l], net.kt[l], NT, nt0, sH, sL, lane, acc);
+  __syncthreads();   // every wavefront has read the layer's input
+  if (nt0 < NT) {
+#pragma unroll
+    for (int t = 0; t < TN; ++t) {
+      if (nt0 + t >= NT) continue;
+      const int f0 = 16 * (nt0 + t) + 4 * kq;
+      float bias[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        bias[r] = f0 + r < net.out[l] ? params[net.boff[l] + f0 + r] : 0.f;
+      if (l + 1 < net.L) {
+#pragma unroll
+        for (int m = 0; m < kFuseMt; ++m) {
+          float a[4], d[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float z = acc[m][t][r] + bias[r];
+            const float s = sigmoid_nr(z);
+            a[r] = z * s;
+            d[r] = s * (1.0f + z * (1.0f - s));
+          }
+          fuse_put(sH, sL, 16 * m + j, f0, a);
+          if (TRAIN)
+            tr.ds[((blk * tr.ds_tiles + tr.ds_tile[l] + nt0 + t) * kFuseMt + m) * 64 + lane] =
+                make_float4(d[0], d[1], d[2], d[3]);
+        }
+      } else if (TRAIN) {
+        // dY = 2 cw (y - t) / n in the planes, the loss and the bias gradient
+        float sum[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int m = 0; m < kFuseMt; ++m) {
+          const int64_t b = blk * kFuseRows + 16 * m + j;
+          float g[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            g[r] = 0.f;
+            if (b < n && f0 + r < net.n_out) {
+              const float d = acc[m][t][r] + bias[r] - tr.target[b * net.n_out + f0 + r];
+              const float c = tr.cw[f0 + r];
+              g[r] = 2.0f * c * d / (float)n;
+              lsum += (double)(c * d * d);
+            }
+            sum[r] += g[r];
+          }
+          fuse_put(sH, sL, 16 * m + j, f0, g);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+#pragma unroll
+          for (int h = 1; h < 16; h <<= 1) sum[r] += __shfl_xor(sum[r], h);
+          if (j == 0 && f0 + r < net.out[l])
+            tr.db[(int64_t)(tr.db_row[l] + f0 + r) * tr.nb + blk] = sum[r];
+        }
+      } else {
+        // output rows through LDS (the planes are free) as [row][n_out] floats
+        float* sy = (float*)sH;
+#pragma unroll
+        for (int m = 0; m < kFuseMt; ++m)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int f = f0 + r;
+            if (f >= net.n_out) continue;
+            float v = acc[m][t][r] + bias[r];
+            if (post.on) v = surr_row_value(f, v * post.std[f] + post.mean[f], lnb[16 * m + j]);
+            sy[(16 * m + j) * net.n_out + f] = v;
+          }
+      }
+    }
+  }
+  __syncthreads();
+  if (!TRAIN && l + 1 == net.L) {
+    const float* sy = (const float*)sH;
+    const int64_t rows = min((int64_t)kFuseRows, n - blk * kFuseRows);
+    float* o = y + blk * kFuseRows * net.n_out;
+    for (int e = threadIdx.x; e < rows * net.n_out; e += 256) o[e] = sy[e];
+  }
+}
+
+// dZ of layer l - 1 from dZ of layer l in the planes.
+template <int TN, int SB>
+__device__ __forceinline__ void fuse_backward(const FuseNet& net, int l,
+                                              const uint4* __restrict__ frag, int64_t blk,
+                                              unsigned short* sH, unsigned short* sL,
+                                              const FuseTrain& tr, int wave, int lane) {
+  const int NT = net.nt[l - 1], nt0 = wave * TN;
+  const int j = lane & 15, kq = lane >> 4;
+  float4_ acc[kFuseMt][TN];
+  if (nt0 < NT) fuse_mm<TN, SB>(frag + net.wb[l], net.nt[l] / 2, NT, nt0, sH, sL, lane, acc);
+  __syncthreads();
+  if (nt0 < NT) {
+#pragma unroll
+    for (int t = 0; t < TN; ++t) {
+      if (nt0 + t >= NT) continue;
+      const int f0 = 16 * (nt0 + t) + 4 * kq;
+      float sum[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int m = 0; m < kFuseMt; ++m) {
+        const float4 d =
+            tr.ds[((blk * tr.ds_tiles + tr.ds_tile[l - 1] + nt0 + t) * kFuseMt + m) * 64 + lane];
+        const float g[4] = {acc[m][t][0] * d.x, acc[m][t][1] * d.y, acc[m][t][2] * d.z,
+                            acc[m][t][3] * d.w};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sum[r] += g[r];
+        fuse_put(sH, sL, 16 * m + j, f0, g);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+#pragma unroll
+        for (int h = 1; h < 16; h <<= 1) sum[r] += __shfl_xor(sum[r], h);
+        if (j == 0 && f0 + r < net.out[l - 1])
+          tr.db[(int64_t)(tr.db_row[l - 1] + f0 + r) * tr.nb + blk] = sum[r];
+      }
+    }
+  }
+  __syncthreads();
+}
+
+template <int SB, bool TRAIN>
+__global__ __launch_bounds__(256, 2) void k_mlp_fused(FuseNet net, int64_t n,
+                                                      const float* __restrict__ params,
+                                                      const uint4* __restrict__ frag,
+                                                      const float* __restrict__ x,
+                                                      float* __restrict__ y, FuseTrain tr,
+                                                      FusePost post) {
+  __shared__ __attribute__((aligned(16))) unsigned short planes[2][kFuseRows * kFuseLd];
+  __shared__ float lnb[kFuseRows];
+  __shared__ double lred[4];
+  unsigned short* sH = planes[0];
+  unsigned short* sL = planes[1];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t blk = blockIdx.x;
+  const int64_t row0 = blk * kFuseRows;
+  const int wide = net.kt[0] * 32;
+  for (int e = threadIdx.x; e < kFuseRows * wide; e += 256) {
+    const int r = e / wide, c = e - r * wide;
+    const float v = (row0 + r < n && c < net.n_in) ? x[(row0 + r) * net.n_in + c] : 0.f;
+    union { __bf16 s; unsigned short u; } h, l;
+    bf_split(v, h.s, l.s);
+    sH[r * kFuseLd + c] = h.u;
+    sL[r * kFuseLd + c] = l.u;
+  }
+  if (!TRAIN && post.on && post.q && threadIdx.x < kFuseRows)
+    lnb[threadIdx.x] = row0 + threadIdx.x < n
+                           ? rayleigh_log_b(post.q + (row0 + threadIdx.x) * kSurrIn, post.mw_re)
+                           : 0.f;
+  else if (!TRAIN && threadIdx.x < kFuseRows)
+    lnb[threadIdx.x] = 0.f;
+  __syncthreads();
+  double lsum = 0.0;
+  for (int l = 0; l < net.L; ++l) {
+    if (TRAIN)
+      fuse_export(sH, sL, net.kt[l] * 32, blk, tr.at[l],
+                  tr.nb * kFuseRows * (int64_t)(net.kt[l] * 32));
+    if (net.nt[l] > 8)
+      fuse_forward<4, SB, TRAIN>(net, l, frag, params, n, blk, sH, sL, y, tr, post, lnb, wave, lane, lsum);
+    else if (net.nt[l] > 4)
+      fuse_forward<2, SB, TRAIN>(net, l, frag, params, n, blk, sH, sL, y, tr, post, lnb, wave, lane, lsum);
+    else
+      fuse_forward<1, SB, TRAIN>(net, l, frag, params, n, blk, sH, sL, y, tr, post, lnb, wave, lane, lsum);
+  }
+  if (!TRAIN) return;
+  for (int h = 32; h > 0; h >>= 1) lsum += __shfl_xor(lsum, h);
+  if (lane == 0) lred[wave] = lsum;
+  for (int l = net.L - 1; l >= 0; --l) {
+    fuse_export(sH, sL, net.nt[l] * 16, blk, tr.gt[l],
+                tr.nb * kFuseRows * (int64_t)(net.nt[l] * 16));
+    if (l == 0) break;
+    if (net.nt[l - 1] > 8)
+      fuse_backward<4, SB>(net, l, frag, blk, sH, sL, tr, wave, lane);
+    else if (net.nt[l - 1] > 4)
+      fuse_backward<2, SB>(net, l, frag, blk, sH, sL, tr, wave, lane);
+    else
+      fuse_backward<1, SB>(net, l, frag, blk, sH, sL, tr, wave, lane);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) tr.lpart[blk] = ((lred[0] + lred[1]) + lred[2]) + lred[3];
+}
+
+// Weight gradients of every layer in one launch: dW_l = dZ_l^T A_l over the
+// batch.  A wavefront takes 64 x 64 of one layer and one batch split; its
+// operands come straight from the exported planes (one 1 KB load per
+// fragment, each used by four products per term), so there is no LDS and no
+// barrier.  Products as the layer-by-layer path: dZ_hi A_hi + dZ_lo A_hi +
+// dZ_hi A_lo.  part[split][parameter].
+struct FuseGrad {
+  int units;                         // 64 x 64 tiles of all layers
+  int first[kMlpMaxLayers + 1];      // first tile of a layer
+  int n_split;
+  int64_t kb;                        // 32-query groups per split
+  int64_t groups;
+};
+
+__global__ __launch_bounds__(256) void k_mlp_fused_dw(FuseNet net, FuseTrain tr, FuseGrad fg,
+                                                      int64_t n_params,
+                                                      float* __restrict__ part) {
+  const int lane = threadIdx.x & 63;
+  const int64_t u = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (u >= (int64_t)fg.units * fg.n_split) return;
+  const int split = (int)(u / fg.units);
+  const int unit = (int)(u - (int64_t)split * fg.units);
+  int l = 0;
+  while (l + 1 < net.L && fg.first[l + 1] <= unit) ++l;
+  const int Fo = net.nt[l] * 16, Fi = net.kt[l] * 32;
+  const int ni = (Fi + 63) / 64;
+  const int o0 = (unit - fg.first[l]) / ni * 64, i0 = (unit - fg.first[l]) % ni * 64;
+  const int i = lane & 15, kq = lane >> 4;
+  const int64_t lo_g = tr.nb * kFuseRows * (int64_t)Fo, lo_a = tr.nb * kFuseRows * (int64_t)Fi;
+  // clamped tiles repeat the last one; their results are not written
+  int64_t go[4], ao[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    go[t] = (int64_t)(min(o0 + 16 * t, Fo - 16) + i) * 32 + 8 * kq;
+    ao[t] = (int64_t)(min(i0 + 16 * t, Fi - 16) + i) * 32 + 8 * kq;
+  }
+  const unsigned short* G = tr.gt[l];
+  const unsigned short* A = tr.at[l];
+  union U { uint4 q; bf16x8_ v; };
+  float4_ acc[4][4];
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) acc[a][b] = (float4_){0.f, 0.f, 0.f, 0.f};
+  const int64_t k1 = min(fg.groups, (split + 1) * fg.kb);
+  U gh[4], gl[4], ah[4], al[4];
+  auto load = [&](int64_t k) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      gh[t].q = *(const uint4*)(G + k * Fo * 32 + go[t]);
+      gl[t].q = *(const uint4*)(G + lo_g + k * Fo * 32 + go[t]);
+      ah[t].q = *(const uint4*)(A + k * Fi * 32 + ao[t]);
+      al[t].q = *(const uint4*)(A + lo_a + k * Fi * 32 + ao[t]);
+    }
+  };
+  int64_t k = split * fg.kb;
+  if (k < k1) load(k);
+  for (; k < k1; ++k) {
+    U ch[4], cl[4], bh[4], bl[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) { ch[t] = gh[t]; cl[t] = gl[t]; bh[t] = ah[t]; bl[t] = al[t]; }
+    if (k + 1 < k1) load(k + 1);
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ch[a].v, bh[b].v, acc[a][b], 0, 0, 0);
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cl[a].v, bh[b].v, acc[a][b], 0, 0, 0);
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ch[a].v, bl[b].v, acc[a][b], 0, 0, 0);
+  }
+  float* dst = part + (int64_t)split * n_params + net.woff[l];
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int o = o0 + 16 * a + 4 * kq + r, c = i0 + 16 * b + i;
+        if (o < net.out[l] && c < net.in[l]) dst[(int64_t)o * net.in[l] + c] = acc[a][b][r];
+      }
+}
+
+// Sums of the parts, in order: weights over the batch splits (a thread each),
+// biases over the blocks and the loss (a wavefront each).
+__global__ __launch_bounds__(256) void k_mlp_fused_reduce(FuseNet net, FuseTrain tr, FuseGrad fg,
+                                                          int64_t n, int64_t n_params, int w_blocks,
+                                                          const float* __restrict__ part,
+                                                          float* __restrict__ grads,
+                                                          float* __restrict__ loss) {
+  if ((int)blockIdx.x < w_blocks) {
+    const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (p >= n_params) return;
+    int l = 0;
+    while (l + 1 < net.L && net.woff[l + 1] <= p) ++l;
+    if (p >= net.boff[l]) return;
+    float s = 0.f;
+#pragma unroll 4
+    for (int q = 0; q < fg.n_split; ++q) s += part[(int64_t)q * n_params + p];
+    grads[p] = s;
+    return;
+  }
+  const int lane = threadIdx.x & 63;
+  const int row = ((int)blockIdx.x - w_blocks) * 4 + (threadIdx.x >> 6);
+  const int n_bias = tr.db_row[net.L - 1] + net.out[net.L - 1];
+  if (row < n_bias) {
+    float s = 0.f;
+    for (int64_t b = lane; b < tr.nb; b += 64) s += tr.db[(int64_t)row * tr.nb + b];
+    for (int h = 32; h > 0; h >>= 1) s += __shfl_xor(s, h);
+    int l = 0;
+    while (l + 1 < net.L && tr.db_row[l + 1] <= row) ++l;
+    if (lane == 0) grads[net.boff[l] + row - tr.db_row[l]] = s;
+  } else if (row == n_bias) {
+    double s = 0.0;
+    for (int64_t b = lane; b < tr.nb; b += 64) s += tr.lpart[b];
+    for (int h = 32; h > 0; h >>= 1) s += __shfl_xor(s, h);
+    if (lane == 0) loss[0] = (float)(s / (double)n);
+  }
+}
+
 }  // namespace gm
 
 namespace {
@@ -355,6 +880,161 @@ int layer_forward(const Net& net, int l, int64_t n, const float* params, const f
   return wterms == 2 ? gemm<2, 2, gm::kEpiFwd>(a, 1, s) : gemm<2, 1, gm::kEpiFwd>(a, 1, s);
 }
 
+// The fused kernels' view of a net, or false where a layer is too wide for them:
+// LDS holds kFuseRows rows of at most kFuseWidth features (the layer-by-layer
+// GEMM takes wider nets).
+bool fuse_net(const Net& net, int terms, gm::FuseNet& f) {
+  if (net.max_width > gm::kFuseWidth) return false;
+  f.L = net.L;
+  f.n_in = net.dims[0];
+  f.n_out = net.dims[net.L];
+  f.n_frag = 0;
+  for (int l = 0; l < net.L; ++l) {
+    f.in[l] = net.dims[l];
+    f.out[l] = net.dims[l + 1];
+    f.kt[l] = (f.in[l] + 31) / 32;
+    f.nt[l] = (f.out[l] + 31) / 32 * 2;
+    f.woff[l] = net.woff[l];
+    f.boff[l] = net.boff[l];
+    f.wf[l] = f.n_frag * 64 * terms;
+    f.n_frag += (int64_t)f.kt[l] * f.nt[l];
+  }
+  for (int l = 0; l < net.L; ++l) f.wb[l] = f.wf[l] + f.n_frag * 64 * terms;
+  return true;
+}
+
+int fuse_split_weights(const gm::FuseNet& f, int terms, int backward, const float* params,
+                       uint4* frag, hipStream_t s) {
+  const int64_t threads = f.n_frag * 64 * (backward ? 2 : 1);
+  hipLaunchKernelGGL(gm::k_mlp_split_weights, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
+                     s, f, terms, backward, params, frag);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return gm_fail(GM_ERUNTIME, "k_mlp_split_weights: %s", hipGetErrorString(e));
+  return GM_OK;
+}
+
+template <bool TRAIN>
+int fuse_launch(const gm::FuseNet& f, int terms, int64_t n, const float* params, const uint4* frag,
+                const float* x, float* y, const gm::FuseTrain& tr, const gm::FusePost& post,
+                hipStream_t s) {
+  const dim3 grid((unsigned)((n + gm::kFuseRows - 1) / gm::kFuseRows));
+  if (terms == 2)
+    hipLaunchKernelGGL((gm::k_mlp_fused<2, TRAIN>), grid, dim3(256), 0, s, f, n, params, frag, x,
+                       y, tr, post);
+  else
+    hipLaunchKernelGGL((gm::k_mlp_fused<1, TRAIN>), grid, dim3(256), 0, s, f, n, params, frag, x,
+                       y, tr, post);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return gm_fail(GM_ERUNTIME, "k_mlp_fused: %s", hipGetErrorString(e));
+  return GM_OK;
+}
+
+// y = net(x), or (post.on) the surrogate's table rows from it.
+int forward_any(gm_ctx* ctx, const Net& net, int64_t n, const float* params, const float* x,
+                float* y, const gm::FusePost& post, bool* posted, hipStream_t s) {
+  int rc;
+  const int terms = ctx->tune_mlp_wterms == 2 ? 2 : 1;
+  gm::FuseNet f;
+  size_t slot;
+  *posted = false;
+  if (fuse_net(net, terms, f)) {
+    if ((rc = ctx->reserve(ctx->mlp_ws, (size_t)f.n_frag * 64 * terms * sizeof(uint4)))) return rc;
+    uint4* frag = (uint4*)ctx->mlp_ws.ptr;
+    ctx->mark_begin(gm::kKMlp, s, &slot);
+    if ((rc = fuse_split_weights(f, terms, 0, params, frag, s))) return rc;
+    if ((rc = fuse_launch<false>(f, terms, n, params, frag, x, y, gm::FuseTrain{}, post, s)))
+      return rc;
+    *posted = post.on != 0;
+  } else {
+    const size_t act = (size_t)n * net.max_width;
+    if ((rc = ctx->reserve(ctx->mlp_ws, 2 * act * sizeof(float)))) return rc;
+    float* buf[2] = {(float*)ctx->mlp_ws.ptr, (float*)ctx->mlp_ws.ptr + act};
+    ctx->mark_begin(gm::kKMlp, s, &slot);
+    const float* in = x;
+    for (int l = 0; l < net.L; ++l) {
+      float* out = l == net.L - 1 ? y : buf[l & 1];
+      if ((rc = layer_forward(net, l, n, params, in, out, nullptr, ctx->tune_mlp_wterms, s)))
+        return rc;
+      in = out;
+    }
+  }
+  ctx->mark_end(slot, s);
+  return GM_OK;
+}
+
+// Loss and gradients through the fused kernels.
+int grad_fused(gm_ctx* ctx, const Net& net, const gm::FuseNet& f, int terms, int64_t n,
+               const float* params, const float* x, const float* target, const float* out_weight,
+               float* grads, float* loss, hipStream_t s) {
+  gm::FuseTrain tr{};
+  gm::FuseGrad fg{};
+  const int64_t nb = (n + gm::kFuseRows - 1) / gm::kFuseRows;
+  tr.target = target;
+  tr.cw = out_weight;
+  tr.nb = nb;
+  int n_bias = 0;
+  for (int l = 0; l < f.L; ++l) {
+    tr.ds_tile[l] = tr.ds_tiles;
+    if (l + 1 < f.L) tr.ds_tiles += f.nt[l];
+    tr.db_row[l] = n_bias;
+    n_bias += f.out[l];
+    fg.first[l] = fg.units;
+    fg.units += ((f.nt[l] * 16 + 63) / 64) * ((f.kt[l] * 32 + 63) / 64);
+  }
+  fg.first[f.L] = fg.units;
+  // about four wavefronts per CU over the weight tiles, at least four K steps each
+  fg.groups = nb * (gm::kFuseRows / 32);
+  const int64_t want = std::max<int64_t>(1, std::min<int64_t>((4 * ctx->n_cu + fg.units - 1) / fg.units,
+                                                              fg.groups / 4));
+  fg.kb = (fg.groups + want - 1) / want;
+  fg.n_split = (int)((fg.groups + fg.kb - 1) / fg.kb);
+  // workspace, every piece 256-byte aligned
+  size_t off = 0;
+  auto take = [&](size_t bytes) {
+    const size_t at = off;
+    off += (bytes + 255) & ~(size_t)255;
+    return at;
+  };
+  const size_t o_frag = take((size_t)f.n_frag * 64 * terms * 2 * sizeof(uint4));
+  const size_t o_ds = take((size_t)nb * tr.ds_tiles * gm::kFuseMt * 64 * sizeof(float4));
+  size_t o_at[gm::kMlpMaxLayers], o_gt[gm::kMlpMaxLayers];
+  for (int l = 0; l < f.L; ++l) {
+    o_at[l] = take((size_t)nb * gm::kFuseRows * f.kt[l] * 32 * 2 * sizeof(unsigned short));
+    o_gt[l] = take((size_t)nb * gm::kFuseRows * f.nt[l] * 16 * 2 * sizeof(unsigned short));
+  }
+  const size_t o_db = take((size_t)n_bias * nb * sizeof(float));
+  const size_t o_lp = take((size_t)nb * sizeof(double));
+  const size_t o_part = take((size_t)fg.n_split * net.n_params * sizeof(float));
+  int rc;
+  if ((rc = ctx->reserve(ctx->mlp_ws, off))) return rc;
+  char* ws = (char*)ctx->mlp_ws.ptr;
+  uint4* frag = (uint4*)(ws + o_frag);
+  tr.ds = (float4*)(ws + o_ds);
+  for (int l = 0; l < f.L; ++l) {
+    tr.at[l] = (unsigned short*)(ws + o_at[l]);
+    tr.gt[l] = (unsigned short*)(ws + o_gt[l]);
+  }
+  tr.db = (float*)(ws + o_db);
+  tr.lpart = (double*)(ws + o_lp);
+  float* part = (float*)(ws + o_part);
+  size_t slot;
+  ctx->mark_begin(gm::kKMlp, s, &slot);
+  if ((rc = fuse_split_weights(f, terms, 1, params, frag, s))) return rc;
+  if ((rc = fuse_launch<true>(f, terms, n, params, frag, x, nullptr, tr, gm::FusePost{}, s)))
+    return rc;
+  const int64_t units = (int64_t)fg.units * fg.n_split;
+  hipLaunchKernelGGL(gm::k_mlp_fused_dw, dim3((unsigned)((units + 3) / 4)), dim3(256), 0, s, f, tr,
+                     fg, net.n_params, part);
+  const int w_blocks = (int)((net.n_params + 255) / 256);
+  hipLaunchKernelGGL(gm::k_mlp_fused_reduce, dim3((unsigned)(w_blocks + (n_bias + 1 + 3) / 4)),
+                     dim3(256), 0, s, f, tr, fg, n, net.n_params, w_blocks, (const float*)part,
+                     grads, loss);
+  ctx->mark_end(slot, s);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return gm_fail(GM_ERUNTIME, "gm_mlp_grad: %s", hipGetErrorString(e));
+  return GM_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -378,19 +1058,36 @@ int gm_mlp_forward(gm_ctx* ctx, int n_layers, const int* dims, int64_t n, const 
   hipError_t e = hipSetDevice(ctx->device);
   if (e != hipSuccess) return gm_fail(GM_ERUNTIME, "hipSetDevice: %s", hipGetErrorString(e));
   hipStream_t s = (hipStream_t)stream;
-  const size_t act = (size_t)n * net.max_width;
-  if ((rc = ctx->reserve(ctx->mlp_ws, 2 * act * sizeof(float)))) return rc;
-  float* buf[2] = {(float*)ctx->mlp_ws.ptr, (float*)ctx->mlp_ws.ptr + act};
-  size_t slot;
-  ctx->mark_begin(gm::kKMlp, s, &slot);
-  const float* in = x;
-  for (int l = 0; l < net.L; ++l) {
-    float* out = l == net.L - 1 ? y : buf[l & 1];
-    if ((rc = layer_forward(net, l, n, params, in, out, nullptr, ctx->tune_mlp_wterms, s))) return rc;
-    in = out;
-  }
-  ctx->mark_end(slot, s);
-  return GM_OK;
+  bool posted;
+  return forward_any(ctx, net, n, params, x, y, gm::FusePost{}, &posted, s);
+}
+
+int gm_surrogate_rows(gm_ctx* ctx, int n_layers, const int* dims, int64_t n, const float* params,
+                      const float* x, const float* q, double m_water_re, const float* tgt_mean,
+                      const float* tgt_std, float* rows, gm_stream stream) {
+  Net net;
+  int rc = make_net(n_layers, dims, net, "gm_surrogate_rows");
+  if (rc) return rc;
+  if (!ctx || n < 0 || net.dims[net.L] < 3)
+    return gm_fail(GM_EINVAL, "gm_surrogate_rows: bad arguments");
+  if (n == 0) return GM_OK;
+  if (n > 0x7fffffffLL / 2) return gm_fail(GM_EINVAL, "gm_surrogate_rows: batch too large");
+  if (!params || !x || !tgt_mean || !tgt_std || !rows)
+    return gm_fail(GM_EINVAL, "gm_surrogate_rows: NULL array");
+  hipError_t e = hipSetDevice(ctx->device);
+  if (e != hipSuccess) return gm_fail(GM_ERUNTIME, "hipSetDevice: %s", hipGetErrorString(e));
+  gm::FusePost post;
+  post.q = q;
+  post.mean = tgt_mean;
+  post.std = tgt_std;
+  post.mw_re = (float)m_water_re;
+  post.on = 1;
+  bool posted;
+  if ((rc = forward_any(ctx, net, n, params, x, rows, post, &posted, (hipStream_t)stream))) return rc;
+  // a net too wide for the fused kernel wrote y: transform it in place
+  return posted ? GM_OK
+                : gm_surrogate_post(ctx, n, net.dims[net.L], q, m_water_re, rows, tgt_mean, tgt_std,
+                                    rows, stream);
 }
 
 int gm_mlp_grad(gm_ctx* ctx, int n_layers, const int* dims, int64_t n, const float* params,
@@ -406,6 +1103,10 @@ int gm_mlp_grad(gm_ctx* ctx, int n_layers, const int* dims, int64_t n, const flo
   hipError_t e = hipSetDevice(ctx->device);
   if (e != hipSuccess) return gm_fail(GM_ERUNTIME, "hipSetDevice: %s", hipGetErrorString(e));
   hipStream_t s = (hipStream_t)stream;
+  gm::FuseNet f;
+  const int terms = ctx->tune_mlp_wterms == 2 ? 2 : 1;
+  if (fuse_net(net, terms, f))
+    return grad_fused(ctx, net, f, terms, n, params, x, target, out_weight, grads, loss, s);
   const int L = net.L;
   // workspace: A_l and Z_l for every layer, two gradient buffers, split-K
   // partials and the loss partials

@@ -32,10 +32,10 @@
 #include <stdint.h>
 
 #include "gm_ctx.h"
+#include "gm_surrogate.h"
 
 namespace gm {
 
-constexpr int kSurrIn = 6;
 constexpr float kGFloor = 1e-8f;
 
 struct Cells {
@@ -77,36 +77,16 @@ __global__ void k_surr_prep(int64_t n, const float* __restrict__ q, const float*
   flags[i] = flag;
 }
 
-// ln B of one query (see the header comment); FP32 throughout, log domain.
-__device__ __forceinline__ float rayleigh_log_b(const float* __restrict__ qi, float mw_re) {
-  const float dry = 1.0f - qi[5];
-  const float lx = qi[0] - logf(qi[4]) + 1.8378770664093453f;   // ln x_eff
-  const float ls = logf(qi[1]);
-  const float mr = mw_re + (qi[2] - mw_re) * dry, mi = expf(qi[3]) * dry;
-  const float a = mr * mr - mi * mi, b = 2.0f * mr * mi;          // m^2 = a + i b
-  const float den = (a + 2.0f) * (a + 2.0f) + b * b;
-  const float k2 = ((a - 1.0f) * (a - 1.0f) + b * b) / den;      // |K|^2
-  const float ln_sca = 0.98082925301172f + logf(k2) + 4.0f * lx + 6.0f * ls * ls;   // ln 8/3
-  const float ln_abs = 1.38629436111989f + logf(3.0f * b / den) + lx;               // ln 4
-  const float hi = fmaxf(ln_sca, ln_abs), lo = fminf(ln_sca, ln_abs);
-  const float lq = hi + log1pf(expf(lo - hi));                   // ln Q_R
-  const float u = lq - 0.69314718055995f;                        // ln(Q_R / 2)
-  return lq - (fmaxf(u, 0.0f) + log1pf(expf(-fabsf(u))));        // ln Q_R - ln(1 + Q_R/2)
-}
-
+// rows may be y (each element is read, then written, by one thread).
 __global__ void k_surr_post(int64_t n, int n_out, const float* __restrict__ q, float mw_re,
-                            const float* __restrict__ y, const float* __restrict__ tmean,
-                            const float* __restrict__ tstd, float* __restrict__ rows) {
+                            const float* y, const float* __restrict__ tmean,
+                            const float* __restrict__ tstd, float* rows) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= n * n_out) return;
   const int j = (int)(e % n_out);
   const float t = y[e] * tstd[j] + tmean[j];
-  float v;
-  if (j == 0) v = expf(q ? t + rayleigh_log_b(q + (e / n_out) * kSurrIn, mw_re) : t);
-  else if (j == 1) v = fminf(expf(t), 1.0f);
-  else if (j == 2) v = expf(t);
-  else v = (float)(2 * (j - 3) + 1) * t;
-  rows[e] = v;
+  rows[e] = surr_row_value(
+      j, t, j == 0 && q ? rayleigh_log_b(q + (e / n_out) * kSurrIn, mw_re) : 0.0f);
 }
 
 __global__ void k_surr_targets(int64_t n, int n_out, const float* __restrict__ q, float mw_re,

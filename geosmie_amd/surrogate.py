@@ -212,11 +212,12 @@ class Surrogate(object):
                                   ptr(d["box_lo"]), ptr(d["box_hi"]), self._ccells,
                                   ptr(self._cell_ok), self._cell_ok.numel(), M_WATER.real,
                                   ptr(x), ptr(flags), s), "gm_surrogate_prep")
-        y = self.mlp.forward(x)
-        rows = t.empty_like(y)
-        check(L.gm_surrogate_post(h, n, self.dims[-1], self._baseline_q(q), M_WATER.real, ptr(y),
-                                  ptr(d["tgt_mean"]), ptr(d["tgt_std"]), ptr(rows), s),
-              "gm_surrogate_post")
+        mlp = self.mlp
+        mlp._precision()
+        rows = t.empty((n, self.dims[-1]), dtype=t.float32, device=dev)
+        check(L.gm_surrogate_rows(h, mlp.n_layers, mlp._cd, n, ptr(mlp.p), ptr(x),
+                                  self._baseline_q(q), M_WATER.real, ptr(d["tgt_mean"]),
+                                  ptr(d["tgt_std"]), ptr(rows), s), "gm_surrogate_rows")
         return rows, flags
 
     def _baseline_q(self, q):

@@ -462,6 +462,13 @@ int gm_surrogate_post(gm_ctx* ctx, int64_t n, int n_out, const float* q, double 
                       const float* y, const float* tgt_mean, const float* tgt_std, float* rows,
                       gm_stream stream);
 
+/* gm_mlp_forward followed by gm_surrogate_post: table rows [n][dims[n_layers]]
+ * of network features x (gm_surrogate_prep) and their queries q, in one pass
+ * where the network is at most 256 wide. */
+int gm_surrogate_rows(gm_ctx* ctx, int n_layers, const int* dims, int64_t n, const float* params,
+                      const float* x, const float* q, double m_water_re, const float* tgt_mean,
+                      const float* tgt_std, float* rows, gm_stream stream);
+
 /* Inverse of gm_surrogate_post: table rows [n][n_out] -> standardised
  * training targets y [n][n_out] (t0 = ln Qext - ln B, t1 = ln SSA, t2 = ln max(g, 1e-8),
  * t_{3+l} = alpha1_l / (2l + 1); y_j = (t_j - tgt_mean[j]) / tgt_std[j]). */
