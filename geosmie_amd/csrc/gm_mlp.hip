@@ -278,7 +278,7 @@ __global__ void k_mlp_adam(int64_t n, float* __restrict__ p, const float* __rest
 // ---- fused network ----------------------------------------------------------
 //
 // Networks whose layers are all at most kFuseWidth wide run whole: a block
-// takes kFuseRows queries through every layer with the activations in LDS (as
+// takes 64 queries (training: 32) through every layer with the activations in LDS (as
 // the BF16 hi and lo planes that the products read), so nothing between the
 // input and the output rows goes through memory.  Layer by layer the 1M-query
 // forward pass wrote and read 10 GB of FP32 activations; what is left is
@@ -287,11 +287,13 @@ __global__ void k_mlp_adam(int64_t n, float* __restrict__ p, const float* __rest
 // The weights are the MFMA's A operand and the activations its B operand:
 // a lane then holds four consecutive features of one query (D[4g + r][j] in
 // lane j + 16g), which it puts back into the planes with 8-byte stores.  The
-// four wavefronts split a layer's features; each multiplies all kFuseRows
+// wavefronts split a layer's features; each multiplies all of the block's
 // queries, so a weight fragment it loads (16 bytes a lane, laid out for that
 // by k_mlp_split_weights) feeds four products per term.  64 rows: 67 KB of
-// planes, two blocks per CU, so one block's SiLU (as many VALU cycles as the
-// layer has MFMA cycles) runs under the other's products.
+// planes, two blocks per CU, so one block's SiLU can run under the other's
+// products.  1M queries (6-256-256-256-256-35, two-term weights): 5284 -> 1460
+// us, MFMA 36% busy, the SiLU and splits about as many VALU cycles as the
+// products take; the products alone are 0.59 ms of matrix-core time.
 //
 // Training runs the same block forward and back: dZ_l takes the activations'
 // place in LDS, SiLU'(z) waits in memory in the order the lane reads it, and
@@ -299,8 +301,6 @@ __global__ void k_mlp_adam(int64_t n, float* __restrict__ p, const float* __rest
 // contiguous, in the order the weight gradient's MFMAs (contraction over the
 // batch) load them.
 constexpr int kFuseWidth = 256;
-constexpr int kFuseRows = 64;
-constexpr int kFuseMt = kFuseRows / 16;
 constexpr int kFuseLd = kFuseWidth + 8;   // 528-byte rows: 16-byte fragments on distinct banks
 
 struct FuseNet {
@@ -339,12 +339,11 @@ __device__ __forceinline__ void bf_split(float v, __bf16& h, __bf16& l) {
   l = (__bf16)(v - (float)h);
 }
 
-// 1 / (1 + exp(-z)) by the hardware reciprocal and one Newton step (below 1 ulp);
-// the argument is kept where exp() is finite so that the step has no inf * 0.
-__device__ __forceinline__ float sigmoid_nr(float z) {
-  const float d = 1.0f + expf(fminf(-z, 85.0f));
-  const float r = __builtin_amdgcn_rcpf(d);
-  return fmaf(fmaf(-d, r, 1.0f), r, r);
+// 1 / (1 + exp(-z)) on the hardware exp2 and reciprocal (1 ulp each; the
+// argument's rounding moves the result by less than an ulp of 1): five
+// instructions a value.  The epilogue is as long as the products otherwise.
+__device__ __forceinline__ float sigmoid_hw(float z) {
+  return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * -1.44269504088896341f));
 }
 
 // Weight fragments: forward F[nt][kt] = W[16 nt + i][32 kt + 8 kq + e] and, for
@@ -383,13 +382,14 @@ __global__ __launch_bounds__(256) void k_mlp_split_weights(FuseNet net, int term
   if (terms == 2) dst[64] = lo.q;
 }
 
-// acc[m][t] += weights tile nt0 + t (of NT) x activations rows 16 m.. over KT
-// steps; products act_hi w_hi, act_lo w_hi, (two terms) act_hi w_lo per step.
-template <int TN, int SB>
+// acc[m][t] = init[t] + weights tile nt0 + t (of NT) x activations rows 16 m.. over
+// KT steps; products act_hi w_hi, act_lo w_hi, (two terms) act_hi w_lo per step.
+template <int MT, int TN, int SB>
 __device__ __forceinline__ void fuse_mm(const uint4* __restrict__ wf, int KT, int NT, int nt0,
                                         const unsigned short* __restrict__ sH,
                                         const unsigned short* __restrict__ sL, int lane,
-                                        float4_ (&acc)[kFuseMt][TN]) {
+                                        const float4_ (&init)[TN],
+                                        float4_ (&acc)[MT][TN]) {
   union U { uint4 q; bf16x8_ v; };
   const int i = lane & 15, kq = lane >> 4;
   const uint4* p[TN];
@@ -397,7 +397,7 @@ __device__ __forceinline__ void fuse_mm(const uint4* __restrict__ wf, int KT, in
   for (int t = 0; t < TN; ++t) {
     p[t] = wf + (int64_t)min(nt0 + t, NT - 1) * KT * SB * 64 + lane;
 #pragma unroll
-    for (int m = 0; m < kFuseMt; ++m) acc[m][t] = (float4_){0.f, 0.f, 0.f, 0.f};
+    for (int m = 0; m < MT; ++m) acc[m][t] = init[t];
   }
   U wn[TN][SB];
 #pragma unroll
@@ -405,7 +405,7 @@ __device__ __forceinline__ void fuse_mm(const uint4* __restrict__ wf, int KT, in
 #pragma unroll
     for (int s = 0; s < SB; ++s) wn[t][s].q = p[t][s * 64];
   for (int k = 0; k < KT; ++k) {
-    U wc[TN][SB], ah[kFuseMt], al[kFuseMt];
+    U wc[TN][SB], ah[MT], al[MT];
 #pragma unroll
     for (int t = 0; t < TN; ++t)
 #pragma unroll
@@ -417,24 +417,24 @@ __device__ __forceinline__ void fuse_mm(const uint4* __restrict__ wf, int KT, in
         for (int s = 0; s < SB; ++s) wn[t][s].q = p[t][((k + 1) * SB + s) * 64];
     }
 #pragma unroll
-    for (int m = 0; m < kFuseMt; ++m) {
+    for (int m = 0; m < MT; ++m) {
       const int at = (16 * m + i) * kFuseLd + 32 * k + 8 * kq;
       ah[m].q = *(const uint4*)&sH[at];
       al[m].q = *(const uint4*)&sL[at];
     }
 #pragma unroll
-    for (int m = 0; m < kFuseMt; ++m)
+    for (int m = 0; m < MT; ++m)
 #pragma unroll
       for (int t = 0; t < TN; ++t)
         acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wc[t][0].v, ah[m].v, acc[m][t], 0, 0, 0);
 #pragma unroll
-    for (int m = 0; m < kFuseMt; ++m)
+    for (int m = 0; m < MT; ++m)
 #pragma unroll
       for (int t = 0; t < TN; ++t)
         acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wc[t][0].v, al[m].v, acc[m][t], 0, 0, 0);
     if (SB == 2) {
 #pragma unroll
-      for (int m = 0; m < kFuseMt; ++m)
+      for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int t = 0; t < TN; ++t)
           acc[m][t] =
@@ -453,36 +453,34 @@ __device__ __forceinline__ void fuse_put(unsigned short* __restrict__ sH,
   *(uint2*)&sL[row * kFuseLd + f] = l.q;
 }
 
-// The planes' first F columns, transposed, to dst[block's two 32-row groups][F][32]
-// (hi; lo follows at lo_off): a thread takes one feature.
+// The planes' first F columns, transposed, to dst[the block's 32-row groups][F][32]
+// (hi; lo follows at lo_off): a thread takes one feature of one group and plane.
+template <int MT, int W>
 __device__ __forceinline__ void fuse_export(const unsigned short* __restrict__ sH,
                                             const unsigned short* __restrict__ sL, int F,
                                             int64_t blk, unsigned short* __restrict__ dst,
                                             int64_t lo_off) {
-  const int f = threadIdx.x;
+  const int f = threadIdx.x & (kFuseWidth - 1);
   if (f >= F) return;
-#pragma unroll
-  for (int pl = 0; pl < 2; ++pl) {
+  for (int c = threadIdx.x / kFuseWidth; c < MT; c += 64 * W / kFuseWidth) {
+    const int g = c >> 1, pl = c & 1;
     const unsigned short* src = pl ? sL : sH;
+    uint4* o = (uint4*)(dst + (pl ? lo_off : 0) + ((blk * (MT / 2) + g) * F + f) * 32);
 #pragma unroll
-    for (int g = 0; g < kFuseRows / 32; ++g) {
-      uint4* o = (uint4*)(dst + (pl ? lo_off : 0) + ((blk * (kFuseRows / 32) + g) * F + f) * 32);
+    for (int q = 0; q < 4; ++q) {
+      unsigned w[4];
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        unsigned w[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int b = 32 * g + 8 * c + 2 * e;
-          w[e] = src[b * kFuseLd + f] | ((unsigned)src[(b + 1) * kFuseLd + f] << 16);
-        }
-        o[c] = make_uint4(w[0], w[1], w[2], w[3]);
+      for (int e = 0; e < 4; ++e) {
+        const int b = 32 * g + 8 * q + 2 * e;
+        w[e] = src[b * kFuseLd + f] | ((unsigned)src[(b + 1) * kFuseLd + f] << 16);
       }
+      o[q] = make_uint4(w[0], w[1], w[2], w[3]);
     }
   }
 }
 
 // One layer of a block, TN feature tiles per wavefront.
-template <int TN, int SB, bool TRAIN>
+template <int MT, int TN, int SB, bool TRAIN, int W>
 __device__ __forceinline__ void fuse_forward(const FuseNet& net, int l, const uint4* __restrict__ frag,
                                              const float* __restrict__ params, int64_t n,
                                              int64_t blk, unsigned short* sH, unsigned short* sL,
@@ -491,46 +489,49 @@ __device__ __forceinline__ void fuse_forward(const FuseNet& net, int l, const ui
                                              int lane, double& lsum) {
   const int NT = net.nt[l], nt0 = wave * TN;
   const int j = lane & 15, kq = lane >> 4;
-  float4_ acc[kFuseMt][TN];
-  if (nt0 < NT) fuse_mm<TN, SB>(frag + net.wf[l], net.kt[l], NT, nt0, sH, sL, lane, acc);
+  float4_ acc[MT][TN], bias[TN];
+#pragma unroll
+  for (int t = 0; t < TN; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int f = 16 * (nt0 + t) + 4 * kq + r;
+      bias[t][r] = f < net.out[l] ? params[net.boff[l] + f] : 0.f;
+    }
+  if (nt0 < NT) fuse_mm<MT, TN, SB>(frag + net.wf[l], net.kt[l], NT, nt0, sH, sL, lane, bias, acc);
   __syncthreads();   // every wavefront has read the layer's input
   if (nt0 < NT) {
 #pragma unroll
     for (int t = 0; t < TN; ++t) {
       if (nt0 + t >= NT) continue;
       const int f0 = 16 * (nt0 + t) + 4 * kq;
-      float bias[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        bias[r] = f0 + r < net.out[l] ? params[net.boff[l] + f0 + r] : 0.f;
       if (l + 1 < net.L) {
 #pragma unroll
-        for (int m = 0; m < kFuseMt; ++m) {
+        for (int m = 0; m < MT; ++m) {
           float a[4], d[4];
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const float z = acc[m][t][r] + bias[r];
-            const float s = sigmoid_nr(z);
+            const float z = acc[m][t][r];
+            const float s = sigmoid_hw(z);
             a[r] = z * s;
             d[r] = s * (1.0f + z * (1.0f - s));
           }
           fuse_put(sH, sL, 16 * m + j, f0, a);
           if (TRAIN)
-            tr.ds[((blk * tr.ds_tiles + tr.ds_tile[l] + nt0 + t) * kFuseMt + m) * 64 + lane] =
+            tr.ds[((blk * tr.ds_tiles + tr.ds_tile[l] + nt0 + t) * MT + m) * 64 + lane] =
                 make_float4(d[0], d[1], d[2], d[3]);
         }
       } else if (TRAIN) {
         // dY = 2 cw (y - t) / n in the planes, the loss and the bias gradient
         float sum[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int m = 0; m < kFuseMt; ++m) {
-          const int64_t b = blk * kFuseRows + 16 * m + j;
+        for (int m = 0; m < MT; ++m) {
+          const int64_t b = blk * (16 * MT) + 16 * m + j;
           float g[4];
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             g[r] = 0.f;
             if (b < n && f0 + r < net.n_out) {
-              const float d = acc[m][t][r] + bias[r] - tr.target[b * net.n_out + f0 + r];
+              const float d = acc[m][t][r] - tr.target[b * net.n_out + f0 + r];
               const float c = tr.cw[f0 + r];
               g[r] = 2.0f * c * d / (float)n;
               lsum += (double)(c * d * d);
@@ -550,12 +551,12 @@ __device__ __forceinline__ void fuse_forward(const FuseNet& net, int l, const ui
         // output rows through LDS (the planes are free) as [row][n_out] floats
         float* sy = (float*)sH;
 #pragma unroll
-        for (int m = 0; m < kFuseMt; ++m)
+        for (int m = 0; m < MT; ++m)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const int f = f0 + r;
             if (f >= net.n_out) continue;
-            float v = acc[m][t][r] + bias[r];
+            float v = acc[m][t][r];
             if (post.on) v = surr_row_value(f, v * post.std[f] + post.mean[f], lnb[16 * m + j]);
             sy[(16 * m + j) * net.n_out + f] = v;
           }
@@ -565,22 +566,24 @@ __device__ __forceinline__ void fuse_forward(const FuseNet& net, int l, const ui
   __syncthreads();
   if (!TRAIN && l + 1 == net.L) {
     const float* sy = (const float*)sH;
-    const int64_t rows = min((int64_t)kFuseRows, n - blk * kFuseRows);
-    float* o = y + blk * kFuseRows * net.n_out;
-    for (int e = threadIdx.x; e < rows * net.n_out; e += 256) o[e] = sy[e];
+    const int64_t rows = min((int64_t)(16 * MT), n - blk * (16 * MT));
+    float* o = y + blk * (16 * MT) * net.n_out;
+    for (int e = threadIdx.x; e < rows * net.n_out; e += 64 * W) o[e] = sy[e];
   }
 }
 
 // dZ of layer l - 1 from dZ of layer l in the planes.
-template <int TN, int SB>
+template <int MT, int TN, int SB>
 __device__ __forceinline__ void fuse_backward(const FuseNet& net, int l,
                                               const uint4* __restrict__ frag, int64_t blk,
                                               unsigned short* sH, unsigned short* sL,
                                               const FuseTrain& tr, int wave, int lane) {
   const int NT = net.nt[l - 1], nt0 = wave * TN;
   const int j = lane & 15, kq = lane >> 4;
-  float4_ acc[kFuseMt][TN];
-  if (nt0 < NT) fuse_mm<TN, SB>(frag + net.wb[l], net.nt[l] / 2, NT, nt0, sH, sL, lane, acc);
+  float4_ acc[MT][TN], zero[TN];
+#pragma unroll
+  for (int t = 0; t < TN; ++t) zero[t] = (float4_){0.f, 0.f, 0.f, 0.f};
+  if (nt0 < NT) fuse_mm<MT, TN, SB>(frag + net.wb[l], net.nt[l] / 2, NT, nt0, sH, sL, lane, zero, acc);
   __syncthreads();
   if (nt0 < NT) {
 #pragma unroll
@@ -589,9 +592,9 @@ __device__ __forceinline__ void fuse_backward(const FuseNet& net, int l,
       const int f0 = 16 * (nt0 + t) + 4 * kq;
       float sum[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int m = 0; m < kFuseMt; ++m) {
+      for (int m = 0; m < MT; ++m) {
         const float4 d =
-            tr.ds[((blk * tr.ds_tiles + tr.ds_tile[l - 1] + nt0 + t) * kFuseMt + m) * 64 + lane];
+            tr.ds[((blk * tr.ds_tiles + tr.ds_tile[l - 1] + nt0 + t) * MT + m) * 64 + lane];
         const float g[4] = {acc[m][t][0] * d.x, acc[m][t][1] * d.y, acc[m][t][2] * d.z,
                             acc[m][t][3] * d.w};
 #pragma unroll
@@ -610,72 +613,78 @@ __device__ __forceinline__ void fuse_backward(const FuseNet& net, int l,
   __syncthreads();
 }
 
-template <int SB, bool TRAIN>
-__global__ __launch_bounds__(256, 2) void k_mlp_fused(FuseNet net, int64_t n,
+template <int SB, bool TRAIN, int W, int MT>
+__global__ __launch_bounds__(64 * W, MT > 4 ? W / 4 : W / 2) void k_mlp_fused(FuseNet net, int64_t n,
                                                       const float* __restrict__ params,
                                                       const uint4* __restrict__ frag,
                                                       const float* __restrict__ x,
                                                       float* __restrict__ y, FuseTrain tr,
                                                       FusePost post) {
-  __shared__ __attribute__((aligned(16))) unsigned short planes[2][kFuseRows * kFuseLd];
-  __shared__ float lnb[kFuseRows];
-  __shared__ double lred[4];
+  __shared__ __attribute__((aligned(16))) unsigned short planes[2][(16 * MT) * kFuseLd];
+  __shared__ float lnb[(16 * MT)];
+  __shared__ double lred[W];
   unsigned short* sH = planes[0];
   unsigned short* sL = planes[1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t blk = blockIdx.x;
-  const int64_t row0 = blk * kFuseRows;
-  const int wide = net.kt[0] * 32;
-  for (int e = threadIdx.x; e < kFuseRows * wide; e += 256) {
-    const int r = e / wide, c = e - r * wide;
+  const int64_t row0 = blk * (16 * MT);
+  for (int e = threadIdx.x; e < (16 * MT) * 32 * net.kt[0]; e += 64 * W) {
+    const int c = (e & 31) + 32 * (e / (32 * 16 * MT)), r = (e >> 5) % (16 * MT);
     const float v = (row0 + r < n && c < net.n_in) ? x[(row0 + r) * net.n_in + c] : 0.f;
     union { __bf16 s; unsigned short u; } h, l;
     bf_split(v, h.s, l.s);
     sH[r * kFuseLd + c] = h.u;
     sL[r * kFuseLd + c] = l.u;
   }
-  if (!TRAIN && post.on && post.q && threadIdx.x < kFuseRows)
+  if (!TRAIN && post.on && post.q && threadIdx.x < (16 * MT))
     lnb[threadIdx.x] = row0 + threadIdx.x < n
                            ? rayleigh_log_b(post.q + (row0 + threadIdx.x) * kSurrIn, post.mw_re)
                            : 0.f;
-  else if (!TRAIN && threadIdx.x < kFuseRows)
+  else if (!TRAIN && threadIdx.x < (16 * MT))
     lnb[threadIdx.x] = 0.f;
   __syncthreads();
   double lsum = 0.0;
   for (int l = 0; l < net.L; ++l) {
     if (TRAIN)
-      fuse_export(sH, sL, net.kt[l] * 32, blk, tr.at[l],
-                  tr.nb * kFuseRows * (int64_t)(net.kt[l] * 32));
-    if (net.nt[l] > 8)
-      fuse_forward<4, SB, TRAIN>(net, l, frag, params, n, blk, sH, sL, y, tr, post, lnb, wave, lane, lsum);
-    else if (net.nt[l] > 4)
-      fuse_forward<2, SB, TRAIN>(net, l, frag, params, n, blk, sH, sL, y, tr, post, lnb, wave, lane, lsum);
+      fuse_export<MT, W>(sH, sL, net.kt[l] * 32, blk, tr.at[l],
+                  tr.nb * (16 * MT) * (int64_t)(net.kt[l] * 32));
+    const int tn = (net.nt[l] + W - 1) / W;   // feature tiles per wavefront
+    if (W == 4 && tn > 2)
+      fuse_forward<MT, 16 / W, SB, TRAIN, W>(net, l, frag, params, n, blk, sH, sL, y, tr, post, lnb, wave, lane, lsum);
+    else if (tn > 1)
+      fuse_forward<MT, 2, SB, TRAIN, W>(net, l, frag, params, n, blk, sH, sL, y, tr, post, lnb, wave, lane, lsum);
     else
-      fuse_forward<1, SB, TRAIN>(net, l, frag, params, n, blk, sH, sL, y, tr, post, lnb, wave, lane, lsum);
+      fuse_forward<MT, 1, SB, TRAIN, W>(net, l, frag, params, n, blk, sH, sL, y, tr, post, lnb, wave, lane, lsum);
   }
   if (!TRAIN) return;
   for (int h = 32; h > 0; h >>= 1) lsum += __shfl_xor(lsum, h);
   if (lane == 0) lred[wave] = lsum;
   for (int l = net.L - 1; l >= 0; --l) {
-    fuse_export(sH, sL, net.nt[l] * 16, blk, tr.gt[l],
-                tr.nb * kFuseRows * (int64_t)(net.nt[l] * 16));
+    fuse_export<MT, W>(sH, sL, net.nt[l] * 16, blk, tr.gt[l],
+                tr.nb * (16 * MT) * (int64_t)(net.nt[l] * 16));
     if (l == 0) break;
-    if (net.nt[l - 1] > 8)
-      fuse_backward<4, SB>(net, l, frag, blk, sH, sL, tr, wave, lane);
-    else if (net.nt[l - 1] > 4)
-      fuse_backward<2, SB>(net, l, frag, blk, sH, sL, tr, wave, lane);
+    const int tn = (net.nt[l - 1] + W - 1) / W;
+    if (W == 4 && tn > 2)
+      fuse_backward<MT, 16 / W, SB>(net, l, frag, blk, sH, sL, tr, wave, lane);
+    else if (tn > 1)
+      fuse_backward<MT, 2, SB>(net, l, frag, blk, sH, sL, tr, wave, lane);
     else
-      fuse_backward<1, SB>(net, l, frag, blk, sH, sL, tr, wave, lane);
+      fuse_backward<MT, 1, SB>(net, l, frag, blk, sH, sL, tr, wave, lane);
   }
   __syncthreads();
-  if (threadIdx.x == 0) tr.lpart[blk] = ((lred[0] + lred[1]) + lred[2]) + lred[3];
+  if (threadIdx.x == 0) {
+    double s = 0.0;
+    for (int w = 0; w < W; ++w) s += lred[w];
+    tr.lpart[blk] = s;
+  }
 }
 
 // Weight gradients of every layer in one launch: dW_l = dZ_l^T A_l over the
 // batch.  A wavefront takes 64 x 64 of one layer and one batch split; its
 // operands come straight from the exported planes (one 1 KB load per
 // fragment, each used by four products per term), so there is no LDS and no
-// barrier.  Products as the layer-by-layer path: dZ_hi A_hi + dZ_lo A_hi +
+// barrier.  All tiles of a split run on one XCD, whose L2 then fetches that
+// part of the planes once (splits in turn over the XCDs).  Products as the layer-by-layer path: dZ_hi A_hi + dZ_lo A_hi +
 // dZ_hi A_lo.  part[split][parameter].
 struct FuseGrad {
   int units;                         // 64 x 64 tiles of all layers
@@ -689,17 +698,18 @@ __global__ __launch_bounds__(256) void k_mlp_fused_dw(FuseNet net, FuseTrain tr,
                                                       int64_t n_params,
                                                       float* __restrict__ part) {
   const int lane = threadIdx.x & 63;
-  const int64_t u = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (u >= (int64_t)fg.units * fg.n_split) return;
-  const int split = (int)(u / fg.units);
-  const int unit = (int)(u - (int64_t)split * fg.units);
+  const int per = (fg.units + 3) / 4;          // blocks of one split
+  const int turn = (int)(blockIdx.x >> 3);     // blocks go to the eight XCDs in turn
+  const int split = turn / per * 8 + (int)(blockIdx.x & 7);
+  const int unit = turn % per * 4 + (int)(threadIdx.x >> 6);
+  if (unit >= fg.units || split >= fg.n_split) return;
   int l = 0;
   while (l + 1 < net.L && fg.first[l + 1] <= unit) ++l;
   const int Fo = net.nt[l] * 16, Fi = net.kt[l] * 32;
   const int ni = (Fi + 63) / 64;
   const int o0 = (unit - fg.first[l]) / ni * 64, i0 = (unit - fg.first[l]) % ni * 64;
   const int i = lane & 15, kq = lane >> 4;
-  const int64_t lo_g = tr.nb * kFuseRows * (int64_t)Fo, lo_a = tr.nb * kFuseRows * (int64_t)Fi;
+  const int64_t lo_g = fg.groups * 32 * Fo, lo_a = fg.groups * 32 * Fi;
   // clamped tiles repeat the last one; their results are not written
   int64_t go[4], ao[4];
 #pragma unroll
@@ -880,8 +890,15 @@ int layer_forward(const Net& net, int l, int64_t n, const float* params, const f
   return wterms == 2 ? gemm<2, 2, gm::kEpiFwd>(a, 1, s) : gemm<2, 1, gm::kEpiFwd>(a, 1, s);
 }
 
+// Wavefronts per block and 16-row tiles per block, measured at 1M queries and at a
+// 16384-row training batch.  Forward: 4 and 4 1481 us (two blocks per CU); 8 and
+// 4 1560, 4 and 8 1867 (one block per CU: its SiLU overlaps nothing), 8 and 8
+// 1571, 4 and 2 1878 (twice the weight traffic).  Training, whose default batch
+// gives 256 blocks of 64 rows: 8 and 2 181 us, 8 and 4 192, 4 and 2 188, 4 and 4 213.
+constexpr int kFuseWavesTrain = 8, kFuseWavesFwd = 4, kFuseMtFwd = 4, kFuseMtTrain = 2;
+
 // The fused kernels' view of a net, or false where a layer is too wide for them:
-// LDS holds kFuseRows rows of at most kFuseWidth features (the layer-by-layer
+// LDS holds a block's rows of at most kFuseWidth features (the layer-by-layer
 // GEMM takes wider nets).
 bool fuse_net(const Net& net, int terms, gm::FuseNet& f) {
   if (net.max_width > gm::kFuseWidth) return false;
@@ -917,13 +934,15 @@ template <bool TRAIN>
 int fuse_launch(const gm::FuseNet& f, int terms, int64_t n, const float* params, const uint4* frag,
                 const float* x, float* y, const gm::FuseTrain& tr, const gm::FusePost& post,
                 hipStream_t s) {
-  const dim3 grid((unsigned)((n + gm::kFuseRows - 1) / gm::kFuseRows));
+  constexpr int W = TRAIN ? kFuseWavesTrain : kFuseWavesFwd;
+  constexpr int MT = TRAIN ? kFuseMtTrain : kFuseMtFwd;
+  const dim3 grid((unsigned)((n + 16 * MT - 1) / (16 * MT)));
   if (terms == 2)
-    hipLaunchKernelGGL((gm::k_mlp_fused<2, TRAIN>), grid, dim3(256), 0, s, f, n, params, frag, x,
-                       y, tr, post);
+    hipLaunchKernelGGL((gm::k_mlp_fused<2, TRAIN, W, MT>), grid, dim3(64 * W), 0, s, f, n, params, frag,
+                       x, y, tr, post);
   else
-    hipLaunchKernelGGL((gm::k_mlp_fused<1, TRAIN>), grid, dim3(256), 0, s, f, n, params, frag, x,
-                       y, tr, post);
+    hipLaunchKernelGGL((gm::k_mlp_fused<1, TRAIN, W, MT>), grid, dim3(64 * W), 0, s, f, n, params, frag,
+                       x, y, tr, post);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return gm_fail(GM_ERUNTIME, "k_mlp_fused: %s", hipGetErrorString(e));
   return GM_OK;
@@ -968,7 +987,7 @@ int grad_fused(gm_ctx* ctx, const Net& net, const gm::FuseNet& f, int terms, int
                float* grads, float* loss, hipStream_t s) {
   gm::FuseTrain tr{};
   gm::FuseGrad fg{};
-  const int64_t nb = (n + gm::kFuseRows - 1) / gm::kFuseRows;
+  const int64_t nb = (n + (16 * kFuseMtTrain) - 1) / (16 * kFuseMtTrain);
   tr.target = target;
   tr.cw = out_weight;
   tr.nb = nb;
@@ -982,12 +1001,13 @@ int grad_fused(gm_ctx* ctx, const Net& net, const gm::FuseNet& f, int terms, int
     fg.units += ((f.nt[l] * 16 + 63) / 64) * ((f.kt[l] * 32 + 63) / 64);
   }
   fg.first[f.L] = fg.units;
-  // about four wavefronts per CU over the weight tiles, at least four K steps each
-  fg.groups = nb * (gm::kFuseRows / 32);
+  // about four wavefronts per CU over the weight tiles, at least four K steps each;
+  // whole rounds of the eight XCDs
+  fg.groups = nb * (kFuseMtTrain / 2);
   const int64_t want = std::max<int64_t>(1, std::min<int64_t>((4 * ctx->n_cu + fg.units - 1) / fg.units,
                                                               fg.groups / 4));
-  fg.kb = (fg.groups + want - 1) / want;
-  fg.n_split = (int)((fg.groups + fg.kb - 1) / fg.kb);
+  fg.n_split = (int)((want + 7) / 8 * 8);
+  fg.kb = (fg.groups + fg.n_split - 1) / fg.n_split;
   // workspace, every piece 256-byte aligned
   size_t off = 0;
   auto take = [&](size_t bytes) {
@@ -996,11 +1016,11 @@ int grad_fused(gm_ctx* ctx, const Net& net, const gm::FuseNet& f, int terms, int
     return at;
   };
   const size_t o_frag = take((size_t)f.n_frag * 64 * terms * 2 * sizeof(uint4));
-  const size_t o_ds = take((size_t)nb * tr.ds_tiles * gm::kFuseMt * 64 * sizeof(float4));
+  const size_t o_ds = take((size_t)nb * tr.ds_tiles * kFuseMtTrain * 64 * sizeof(float4));
   size_t o_at[gm::kMlpMaxLayers], o_gt[gm::kMlpMaxLayers];
   for (int l = 0; l < f.L; ++l) {
-    o_at[l] = take((size_t)nb * gm::kFuseRows * f.kt[l] * 32 * 2 * sizeof(unsigned short));
-    o_gt[l] = take((size_t)nb * gm::kFuseRows * f.nt[l] * 16 * 2 * sizeof(unsigned short));
+    o_at[l] = take((size_t)nb * (16 * kFuseMtTrain) * f.kt[l] * 32 * 2 * sizeof(unsigned short));
+    o_gt[l] = take((size_t)nb * (16 * kFuseMtTrain) * f.nt[l] * 16 * 2 * sizeof(unsigned short));
   }
   const size_t o_db = take((size_t)n_bias * nb * sizeof(float));
   const size_t o_lp = take((size_t)nb * sizeof(double));
@@ -1022,8 +1042,7 @@ int grad_fused(gm_ctx* ctx, const Net& net, const gm::FuseNet& f, int terms, int
   if ((rc = fuse_split_weights(f, terms, 1, params, frag, s))) return rc;
   if ((rc = fuse_launch<true>(f, terms, n, params, frag, x, nullptr, tr, gm::FusePost{}, s)))
     return rc;
-  const int64_t units = (int64_t)fg.units * fg.n_split;
-  hipLaunchKernelGGL(gm::k_mlp_fused_dw, dim3((unsigned)((units + 3) / 4)), dim3(256), 0, s, f, tr,
+  hipLaunchKernelGGL(gm::k_mlp_fused_dw, dim3((unsigned)((fg.units + 3) / 4 * fg.n_split)), dim3(256), 0, s, f, tr,
                      fg, net.n_params, part);
   const int w_blocks = (int)((net.n_params + 255) / 256);
   hipLaunchKernelGGL(gm::k_mlp_fused_reduce, dim3((unsigned)(w_blocks + (n_bias + 1 + 3) / 4)),
