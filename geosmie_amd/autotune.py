@@ -8,20 +8,19 @@ cache per (device, workload name) and reused without timing.
 
 Knobs (include/geosmie.h, enum gm_tune_param):
   mie_grid_mult  persistent Mie grid as a multiple of the resident wavefronts
-  s12_waves      wavefronts (64 angles each) per S1/S2 block
+  s12_waves      wavefronts (64 angles each) per FP32 / split-BF16 S1/S2 block
   psd_chunk      points per split-K chunk of the few-PSD contraction
-  s12_points     points per wavefront of the FP64 S1/S2 kernel
+  s12_points     kept for saved settings; no effect
   mie_waves      register budget of the Mie recurrence kernels (0 unconstrained,
                  3 or 4 resident wavefronts per SIMD)
-  s12_layout     FP64 S1/S2 blocks split angles (0) or points (1) among their waves,
-                 or share LDS-staged angle tables among them (2)
+  s12_layout     kept for saved settings; no effect
   mie_ckpt       coated kernel: downward-chain states kept every 4, 5 or 8 rows and
                  regenerated per block in LDS, or every row kept in scratch (0);
                  non-zero also selects the checkpointed lane-per-point
                  homogeneous kernel (every 4 rows)
   mie_lanes      homogeneous kernel: lanes per point (1, or 16/32/64 with the serial
                  recurrences joined by parallel scans; 0 = chosen by batch)
-  s12_row_tiles  fused S1/S2 row sums: 8-point tiles per work unit (0 = by batch)
+  s12_row_tiles  fused S1/S2 row sums: tiles per work unit (0 = by batch)
   s12_share      split-BF16 fused S1/S2: angle-table tiles shared by four work units
                  through LDS (1) or fetched per wavefront (0)
 (mlp_weight_terms, the BF16 terms per network weight, is a precision

@@ -31,12 +31,12 @@ struct gm_ctx {
   size_t scratch_budget = (size_t)3 << 30;       // bytes of recurrence scratch
   // launch shapes chosen by gm_ctx_tune (an autotuner's knobs)
   int tune_mie_grid_mult = 1;   // persistent Mie grid = multiple of resident wavefronts
-  int tune_s12_waves = 4;       // wavefronts (64 angles each) per S1/S2 block
-  int tune_s12_points = 8;      // points per wavefront of the FP64 S1/S2 kernel (8 or 16)
+  int tune_s12_waves = 4;       // wavefronts (64 angles each) per FP32 / split-BF16 S1/S2 block
+  int tune_s12_points = 8;      // accepted, no effect
   int tune_psd_chunk = 128;     // points per split-K chunk of the few-PSD contraction
   int tune_mlp_wterms = 1;      // BF16 terms per MLP weight (1 = BF16 weights, 2 = hi + lo)
   int tune_mie_waves = 0;       // Mie register variant: 0 unconstrained, 3 or 4 waves per SIMD
-  int tune_s12_layout = 0;      // FP64 S1/S2 block: waves split angles (0) or points (1)
+  int tune_s12_layout = 0;      // accepted, no effect
   int tune_mie_ckpt = 4;        // coated kernel: rows per checkpoint (4, 8) or 0 = every row stored
   int tune_mie_lanes = 0;       // homogeneous kernel: lanes per point (1, 16, 32, 64; 0 = by batch)
   int psd_quirks = 1;           // integratePSD quirks reproduced (GM_PSD_QUIRK_* bits)

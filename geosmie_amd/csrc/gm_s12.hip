@@ -7,9 +7,9 @@
 // real GEMMs  [Re U; Im U](2P x K) x P(K x N_ang)  and the same for V, M, with
 // K = n (ragged per point, zero-padded to the tile maximum).
 //
-// FP64 path: v_mfma_f64_16x16x4_f64.  A wavefront owns 8 points (16 rows =
-// re/im interleaved) x 64 angles (four 16-wide sub-tiles) and walks K in steps
-// of 4.  Operand layouts of v_mfma_f64_16x16x4_f64 (measured on gfx950):
+// FP64 path: v_mfma_f64_16x16x4_f64.  A wavefront owns 16 points (one row tile of
+// real and one of imaginary parts) x 16 TT angles and walks K in steps of 4.
+// Operand layouts of v_mfma_f64_16x16x4_f64 (measured on gfx950):
 // A[i][k] from lane i + 16k, B[k][j] from lane j + 16k, D[g + 4r][j] in lane
 // j + 16g, element r  (the f32/bf16 16x16 variants use D[4g + r][j] instead).
 // Epilogue modes: write S1, S2 (complex), or the four independent Mueller
@@ -26,6 +26,8 @@
 // A row i is then point p0 + (i >> 1), component i & 1, which gives the same
 // per-lane element order as the FP64 kernel: (0,1) = point p0 + 2g (re, im),
 // (2,3) = point p0 + 2g + 1.
+#include <algorithm>
+
 #include "gm_complex.h"
 #include "gm_ctx.h"
 
@@ -50,7 +52,8 @@ __device__ __forceinline__ void s12_store(int mode, int64_t p, int j, int n_ang,
     out1[2 * o] = s2.re;
     out1[2 * o + 1] = s2.im;
   } else if (mode == kOutP11) {
-    out0[o] = 0.5 * (norm2(s1) + norm2(s2));   // s11 only, layout [point][angle]
+    // s11 only, layout [point][angle]: (|S1|^2 + |S2|^2) / 2 = (|sp|^2 + |sm|^2) / 4
+    out0[o] = 0.25 * fma(sp.re, sp.re, fma(sp.im, sp.im, fma(sm.re, sm.re, sm.im * sm.im)));
   } else {
     double a1 = norm2(s1), a2 = norm2(s2);
     cd c = s1 * conj(s2);
@@ -62,274 +65,139 @@ __device__ __forceinline__ void s12_store(int mode, int64_t p, int j, int n_ang,
   }
 }
 
-// MT = M-tiles (8 points each) per wavefront: with MT = 2 every angle-table
-// load feeds twice as many MFMAs.
-template <int MT>
-__global__ __launch_bounds__(256) void k_s12_f64(
-    int64_t n, const int64_t* __restrict__ off, const int32_t* __restrict__ nmax,
-    const double* __restrict__ an, const double* __restrict__ bn, int n_ang,
-    const double* __restrict__ pi_t, const double* __restrict__ tau_t, int nmax_cap, int mode,
-    int wave_points, double* __restrict__ out0, double* __restrict__ out1) {
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int nw = blockDim.x >> 6;
-  // 64 angles x 8 MT points per wavefront.  The waves of a block take
-  // different angles of the same points, or (wave_points) different points of
-  // the same angles, whose angle-table rows they then read through one CU's
-  // cache.
-  const int64_t p0 = wave_points ? ((int64_t)blockIdx.x * nw + wave) * 8 * MT
-                                 : (int64_t)blockIdx.x * 8 * MT;
-  const int j0 = wave_points ? blockIdx.y * 64 : (blockIdx.y * nw + wave) * 64;
-  if (j0 >= n_ang) return;  // whole wavefront past the last angle
-  const int i = lane & 15;   // A row / B column / D column
-  const int kq = lane >> 4;  // k within the 4-step, D row group
-  // The f64 16x16x4 result row of (lane group g, element r) is g + 4r.  A row
-  // i = g + 4r of M-tile mt is assigned to point p0 + 8 mt + 2g + (r >> 1),
-  // component r & 1, so lane group g ends up holding (re, im) of points
-  // p0 + 8 mt + 2g and p0 + 8 mt + 2g + 1.
-  const int comp = (i >> 2) & 1;
-  int nm_a[MT];
-  int64_t oa[MT];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    const int64_t pa = p0 + 8 * mt + 2 * (i & 3) + (i >> 3);
-    const bool ok = pa < n;
-    nm_a[mt] = ok ? nmax[pa] : 0;
-    oa[mt] = ok ? off[pa] : 0;
-  }
-  // tile K = max nmax of the 8 MT points
-  int kmax = 0;
-  for (int q = 0; q < 8 * MT; ++q) {
-    int64_t pq = p0 + q;
-    if (pq < n) kmax = max(kmax, nmax[pq]);
-  }
-  kmax = min(kmax, nmax_cap);
-  double4_ accp[MT][4], accm[MT][4];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      accp[mt][t] = (double4_){0.0, 0.0, 0.0, 0.0};
-      accm[mt][t] = (double4_){0.0, 0.0, 0.0, 0.0};
-    }
-  // Operands of step k0 + 4 are loaded while the MFMAs of step k0 run
-  // (register double buffer), so the loads' latency overlaps the products.
-  double ar_n[MT], br_n[MT], pp_n[4], tt_n[4];
-  auto load_step = [&](int k0) {
-    const int kk = k0 + kq;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      ar_n[mt] = 0.0;
-      br_n[mt] = 0.0;
-      if (kk < nm_a[mt]) {
-        ar_n[mt] = an[2 * (oa[mt] + kk) + comp];
-        br_n[mt] = bn[2 * (oa[mt] + kk) + comp];
-      }
-    }
-    const bool krow = kk < kmax;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int j = j0 + t * 16 + i;
-      pp_n[t] = 0.0;
-      tt_n[t] = 0.0;
-      if (krow && j < n_ang) {
-        pp_n[t] = pi_t[(size_t)kk * n_ang + j];
-        tt_n[t] = tau_t[(size_t)kk * n_ang + j];
-      }
-    }
-  };
-  if (kmax > 0) load_step(0);
-  for (int k0 = 0; k0 < kmax; k0 += 4) {
-    double ua[MT], va[MT], P[4], M[4];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      ua[mt] = ar_n[mt] + br_n[mt];
-      va[mt] = ar_n[mt] - br_n[mt];
-    }
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      P[t] = pp_n[t] + tt_n[t];
-      M[t] = pp_n[t] - tt_n[t];
-    }
-    if (k0 + 4 < kmax) load_step(k0 + 4);
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        accp[mt][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ua[mt], P[t], accp[mt][t], 0, 0, 0);
-        accm[mt][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(va[mt], M[t], accm[mt][t], 0, 0, 0);
-      }
-    }
-  }
-  // epilogue: elements (0,1) = point p0+8mt+2kq (re,im), (2,3) = the next point
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int j = j0 + t * 16 + i;
-      if (j >= n_ang) continue;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int64_t p = p0 + 8 * mt + 2 * kq + h;
-        if (p >= n) continue;
-        s12_store(mode, p, j, n_ang, cd{accp[mt][t][2 * h], accp[mt][t][2 * h + 1]},
-                  cd{accm[mt][t][2 * h], accm[mt][t][2 * h + 1]}, out0, out1);
-      }
-    }
-}
-
-// LDS-staged variant: the kS12LdsWaves wavefronts of a block take 8 points each
-// at the same 64 angles and share the angle tables: every stage of
-// kS12LdsRows K-rows of P = pi' + tau' and M = pi' - tau' (64 angles) is read
-// from global memory once per block into LDS, while the previous stage's
-// MFMAs run (the next stage is held in registers, then stored behind a
-// barrier).  The K loop runs to the block's largest n_max; rows past a
-// point's own n_max multiply zero coefficients.
-constexpr int kS12LdsWaves = 4;
-constexpr int kS12LdsRows = 16;
-constexpr int kS12LdsStride = 64 + 2;   // doubles per LDS row (padding against bank conflicts)
-template <int MT>
-__global__ __launch_bounds__(64 * kS12LdsWaves) void k_s12_f64_lds(
-    int64_t n, const int64_t* __restrict__ off, const int32_t* __restrict__ nmax,
-    const double* __restrict__ an, const double* __restrict__ bn, int n_ang,
-    const double* __restrict__ pi_t, const double* __restrict__ tau_t, int nmax_cap, int mode,
-    double* __restrict__ out0, double* __restrict__ out1) {
-  __shared__ double Ps[2][kS12LdsRows][kS12LdsStride];
-  __shared__ double Ms[2][kS12LdsRows][kS12LdsStride];
-  __shared__ int kmax_w[kS12LdsWaves];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int64_t p0 = ((int64_t)blockIdx.x * kS12LdsWaves + wave) * 8 * MT;
-  const int j0 = blockIdx.y * 64;
-  const int i = lane & 15;
-  const int kq = lane >> 4;
-  const int comp = (i >> 2) & 1;
-  int nm_a[MT];
-  int64_t oa[MT];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    const int64_t pa = p0 + 8 * mt + 2 * (i & 3) + (i >> 3);
-    const bool ok = pa < n;
-    nm_a[mt] = ok ? nmax[pa] : 0;
-    oa[mt] = ok ? off[pa] : 0;
-  }
-  int kw = 0;
-  for (int q = 0; q < 8 * MT; ++q) {
-    const int64_t pq = p0 + q;
-    if (pq < n) kw = max(kw, nmax[pq]);
-  }
-  if (lane == 0) kmax_w[wave] = min(kw, nmax_cap);
-  __syncthreads();
-  int kmax = 0;
-  for (int w = 0; w < kS12LdsWaves; ++w) kmax = max(kmax, kmax_w[w]);
-  // cooperative stage loads: thread tid covers (row, column) pairs tid + 256 e
-  constexpr int kPer = kS12LdsRows * 64 / (64 * kS12LdsWaves);
-  double pn[kPer], mn[kPer];
-  auto load_stage = [&](int s0) {
-#pragma unroll
-    for (int e = 0; e < kPer; ++e) {
-      const int q = tid + 64 * kS12LdsWaves * e;
-      const int r = q >> 6, c = q & 63;
-      const int kk = s0 + r, j = j0 + c;
-      double pp = 0.0, tt = 0.0;
-      if (kk < kmax && j < n_ang) {
-        pp = pi_t[(size_t)kk * n_ang + j];
-        tt = tau_t[(size_t)kk * n_ang + j];
-      }
-      pn[e] = pp + tt;
-      mn[e] = pp - tt;
-    }
-  };
-  auto store_stage = [&](int buf) {
-#pragma unroll
-    for (int e = 0; e < kPer; ++e) {
-      const int q = tid + 64 * kS12LdsWaves * e;
-      const int r = q >> 6, c = q & 63;
-      Ps[buf][r][c] = pn[e];
-      Ms[buf][r][c] = mn[e];
-    }
-  };
-  double4_ accp[MT][4], accm[MT][4];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      accp[mt][t] = (double4_){0.0, 0.0, 0.0, 0.0};
-      accm[mt][t] = (double4_){0.0, 0.0, 0.0, 0.0};
-    }
-  if (kmax > 0) {
-    load_stage(0);
-    store_stage(0);
-  }
-  __syncthreads();
-  int buf = 0;
-  for (int s0 = 0; s0 < kmax; s0 += kS12LdsRows) {
-    const bool more = s0 + kS12LdsRows < kmax;
-    if (more) load_stage(s0 + kS12LdsRows);     // in flight during this stage's MFMAs
-#pragma unroll
-    for (int ks = 0; ks < kS12LdsRows / 4; ++ks) {
-      const int kk = s0 + 4 * ks + kq;
-      double ua[MT], va[MT];
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        ua[mt] = 0.0;
-        va[mt] = 0.0;
-        if (kk < nm_a[mt]) {
-          const double ar = an[2 * (oa[mt] + kk) + comp];
-          const double br = bn[2 * (oa[mt] + kk) + comp];
-          ua[mt] = ar + br;
-          va[mt] = ar - br;
-        }
-      }
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const double P = Ps[buf][4 * ks + kq][t * 16 + i];
-        const double M = Ms[buf][4 * ks + kq][t * 16 + i];
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          accp[mt][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ua[mt], P, accp[mt][t], 0, 0, 0);
-          accm[mt][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(va[mt], M, accm[mt][t], 0, 0, 0);
-        }
-      }
-    }
-    if (more) store_stage(buf ^ 1);
-    __syncthreads();
-    buf ^= 1;
-  }
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int j = j0 + t * 16 + i;
-      if (j >= n_ang) continue;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int64_t p = p0 + 8 * mt + 2 * kq + h;
-        if (p >= n) continue;
-        s12_store(mode, p, j, n_ang, cd{accp[mt][t][2 * h], accp[mt][t][2 * h + 1]},
-                  cd{accm[mt][t][2 * h], accm[mt][t][2 * h + 1]}, out0, out1);
-      }
-    }
-}
-
-// ---- S1/S2 -> Mueller -> weighted point sums, fused --------------------------
+// ---- FP64 tiles of 16 points ---------------------------------------------------
 //
-// integratePSD integrates each Mueller element of rawMie against a row of PSD
-// weights (dointegration.py:1044-1050, 1164-1166: np.dot(s_ij.T, psd)).  When
-// every weight row covers a contiguous range of points and few rows share a
-// point (the runoptics passes: one block of points per (rh, refractive index),
-// one row per mode), the Mueller planes need not exist in memory: each
-// wavefront forms S1/S2 of 8-point tiles x 64 angles on the matrix cores as
-// k_s12_f64 does, turns them into s11, s12, s33, s34 in registers and adds
-// weight x element into per-row sums.  A block takes one chunk (one or two
-// whole 8-point tiles) of one row group (rows with the same range), its four
-// wavefronts taking 64 angles each; the sums go to a partial buffer
-// [chunk][RM][4][n_ang] that k_s12_rows_reduce adds up per row in chunk
-// order (deterministic).  Memory traffic drops from 2 x 32 B per (point,
-// angle) to the partials (8 / RM times less per tile).  Chunks of one or two
-// tiles keep the work units as small as k_s12_f64's, so the long K loops of
-// large size parameters do not end up in a few long waves.
+// A wavefront multiplies 16 points by 16 TT angles.  The two MFMA row tiles are
+// the real and the imaginary parts of the same 16 points, so a lane loads a
+// whole complex a_n and b_n (16 bytes each) and its U and V feed both tiles;
+// with the tables as (P, M) pairs (k_s12_prep_pairs) an angle's two words are
+// one 16-byte load as well: 2 + TT loads per step of 4 TT MFMAs.  Tiles of 8
+// points with one component per lane took 10 8-byte loads for 8 MFMAs (or 12
+// for 16): the texture-address unit was 60-70% busy at 36-53% of the matrix
+// rate.  What bound the loop then was latency: the coefficients stream from
+// memory (each is read by one block, then from its caches), so they are loaded
+// four steps ahead.  Steps below the tile's smallest n_max carry no masks.
+// RAW reads pi', tau' as they are (two 8-byte loads per angle), for calls too
+// small to pay for the pairing pass.  The row of (lane group g, element r) is
+// g + 4r: point p0 + g + 4r, real parts in tile 0, imaginary parts in tile 1.
+// 40k points x 1801 angles with row sums 2.77 -> 2.09 ms (matrix cores 53 ->
+// 74% busy); P11 of 1.2M points x 371 angles 8.8 -> 6.0 ms (36 -> 55%).
+constexpr int kUnitBins = 256;   // series-length bins of the launch order
+
+__global__ __launch_bounds__(256) void k_s12_prep_pairs(int n_ang, int nmax_cap, int apad,
+                                                        int64_t total,
+                                                        const double* __restrict__ pi_t,
+                                                        const double* __restrict__ tau_t,
+                                                        double2* __restrict__ tab,
+                                                        int* __restrict__ hist) {
+  const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (hist && blockIdx.x == 0)
+    for (int b = threadIdx.x; b < 2 * kUnitBins; b += 256) hist[b] = 0;
+  if (id >= total) return;
+  const int k = (int)(id / apad), j = (int)(id - (int64_t)k * apad);
+  double2 v = make_double2(0.0, 0.0);
+  if (k < nmax_cap && j < n_ang) {
+    const double p = pi_t[(size_t)k * n_ang + j], t = tau_t[(size_t)k * n_ang + j];
+    v = make_double2(p + t, p - t);
+  }
+  tab[id] = v;
+}
+
+struct S12Tables {
+  const double* pi_t;
+  const double* tau_t;
+  const double2* tab;   // (P, M) [k][apad], zero padded; NULL: RAW
+  int n_ang, apad, nmax_cap;
+};
+
+// sp = sum U P and sm = sum V M of points p0 .. min(p0 + 16, pend) - 1 at angles
+// j0 + 16 t + i: element r of lane (i, g) is point p0 + g + 4r.
+template <int TT, bool RAW, int kCd, int kTd>
+__device__ __forceinline__ void s12_tile64(const S12Tables& T, int64_t p0, int64_t pend, int j0,
+                                           int lane, const int64_t* __restrict__ off,
+                                           const int32_t* __restrict__ nmax,
+                                           const double* __restrict__ an,
+                                           const double* __restrict__ bn, double4_ (&spr)[TT],
+                                           double4_ (&spi)[TT], double4_ (&smr)[TT],
+                                           double4_ (&smi)[TT]) {
+  const int i = lane & 15, kq = lane >> 4;
+  const int64_t pc = min(p0 + i, pend - 1);   // rows past the end repeat the last point
+  const int nm = min(nmax[pc], T.nmax_cap);
+  const int64_t o = nm > 0 ? off[pc] : 0;
+  int kmax = nm, kmin = nm;
+#pragma unroll
+  for (int h = 1; h < 16; h <<= 1) {
+    kmax = max(kmax, __shfl_xor(kmax, h));
+    kmin = min(kmin, __shfl_xor(kmin, h));
+  }
+  kmax = __builtin_amdgcn_readfirstlane(kmax);
+  kmin = __builtin_amdgcn_readfirstlane(kmin);
+#pragma unroll
+  for (int t = 0; t < TT; ++t) {
+    spr[t] = spi[t] = smr[t] = smi[t] = (double4_){0.0, 0.0, 0.0, 0.0};
+  }
+  if (kmax <= 0) return;
+  const double2* pa = (const double2*)an + o;
+  const double2* pb = (const double2*)bn + o;
+  int col[TT];
+#pragma unroll
+  for (int t = 0; t < TT; ++t)
+    col[t] = RAW ? min(j0 + 16 * t + i, T.n_ang - 1) : j0 + 16 * t + i;
+  // Operands are loaded kCd steps (coefficients, which stream from memory) and kTd
+  // steps (tables, shared through the L2) ahead of their products; a step's
+  // table loads are issued before its coefficient loads, since loads retire in
+  // order.  (4, 1) and (3, 1) measured the same, (4, 2) and (2, 2) 2% slower, (1, 1)
+  // 17%.  Indices past the last term repeat it (never used unmasked).
+  const int last = max(nm - 1, 0), row_last = (kmax + 3) / 4 * 4 - 1;
+  double2 a_n[kCd], b_n[kCd], t_n[kTd][TT];
+  auto load_tab = [&](int k0, double2 (&v)[TT]) {
+    if (RAW) {
+      const size_t row = (size_t)min(k0 + kq, kmax - 1) * T.n_ang;
+#pragma unroll
+      for (int t = 0; t < TT; ++t) v[t] = make_double2(T.pi_t[row + col[t]], T.tau_t[row + col[t]]);
+    } else {
+      const double2* row = T.tab + (size_t)min(k0 + kq, row_last) * T.apad;
+#pragma unroll
+      for (int t = 0; t < TT; ++t) v[t] = row[col[t]];
+    }
+  };
+  auto load_coef = [&](int k0, double2& a, double2& b) {
+    const int kc = min(k0 + kq, last);
+    a = pa[kc];
+    b = pb[kc];
+  };
+#pragma unroll
+  for (int q = 0; q < kTd; ++q) load_tab(4 * q, t_n[q]);
+#pragma unroll
+  for (int q = 0; q < kCd; ++q) load_coef(4 * q, a_n[q], b_n[q]);
+  for (int kb = 0; kb < kmax; kb += 4 * kCd) {
+#pragma unroll
+    for (int q = 0; q < kCd; ++q) {
+      const int k0 = kb + 4 * q;
+      if (k0 >= kmax) break;
+      double ur = a_n[q].x + b_n[q].x, ui = a_n[q].y + b_n[q].y;
+      double vr = a_n[q].x - b_n[q].x, vi = a_n[q].y - b_n[q].y;
+      if (k0 + 4 > kmin && k0 + kq >= nm) ur = ui = vr = vi = 0.0;
+      double P[TT], M[TT];
+#pragma unroll
+      for (int t = 0; t < TT; ++t) {
+        const double2 v = t_n[q % kTd][t];
+        P[t] = RAW ? v.x + v.y : v.x;
+        M[t] = RAW ? v.x - v.y : v.y;
+      }
+      load_tab(k0 + 4 * kTd, t_n[q % kTd]);
+      load_coef(k0 + 4 * kCd, a_n[q], b_n[q]);
+#pragma unroll
+      for (int t = 0; t < TT; ++t) {
+        spr[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ur, P[t], spr[t], 0, 0, 0);
+        spi[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ui, P[t], spi[t], 0, 0, 0);
+        smr[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(vr, M[t], smr[t], 0, 0, 0);
+        smi[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(vi, M[t], smi[t], 0, 0, 0);
+      }
+    }
+  }
+}
+
 constexpr int kRowsPerCall = 64;   // rows per call (range arrays passed by value)
 constexpr int kRowsWaves = 4;      // wavefronts (64 angles each) per block
 
@@ -340,149 +208,242 @@ struct RowGroups {
   int64_t chunk0[kRowsPerCall + 1];   // first chunk of each group; chunk0[n_groups] = total
 };
 
-// RM = most rows of one group this instance accumulates (registers: 16 RM
-// doubles per lane for the sums).  MT = 8-point tiles multiplied together:
-// each angle-table word a lane loads feeds the products of all MT tiles (the
-// table loads, not the matrix cores, bound this kernel at MT = 1); a chunk
-// of chunk_pts points runs as consecutive groups of MT tiles.
-template <int RM, int MT>
-__global__ __launch_bounds__(64 * kRowsWaves) void k_s12_rows_f64(
-    RowGroups g, int chunk_pts, const int64_t* __restrict__ off, const int32_t* __restrict__ nmax,
-    const double* __restrict__ an, const double* __restrict__ bn, int n_ang,
-    const double* __restrict__ pi_t, const double* __restrict__ tau_t, int nmax_cap,
-    const double* __restrict__ w, int64_t ldw, double* __restrict__ part) {
+// Launch order of the work units (tiles or chunks of points) of a large call: the
+// longest series first.  A unit of x ~ 3000 runs 800 steps, 0.4 ms beside one
+// of a few microseconds; in point order (radii ascending) the last units launched
+// were such ones and left the chip a tenth to a sixth of the time idle.  Counting
+// sort by the unit's largest n_max in kUnitBins bins; the place within a bin is
+// whatever order the blocks arrive in, which no result depends on.
+__device__ __forceinline__ int unit_bin(int kmax, int nmax_cap) {
+  const int b = (int)((int64_t)min(kmax, nmax_cap) * (kUnitBins - 1) / nmax_cap);
+  return kUnitBins - 1 - max(b, 0);   // bin 0: the longest
+}
+
+// Points [a, b) of unit u: a chunk of a row group, or (no groups) 16-point tiles.
+__device__ __forceinline__ void unit_range(const RowGroups& g, int unit_pts, int64_t u, int64_t n,
+                                           int64_t& a, int64_t& b) {
+  a = u * unit_pts;
+  b = n;
+  if (g.n_groups) {
+    int gi = 0;
+    while (gi + 1 < g.n_groups && g.chunk0[gi + 1] <= u) ++gi;
+    a = g.start[gi] + (u - g.chunk0[gi]) * unit_pts;
+    b = g.start[gi] + g.count[gi];
+  }
+  b = min(a + unit_pts, b);
+}
+
+__global__ __launch_bounds__(256) void k_s12_unit_bins(RowGroups g, int unit_pts, int64_t units,
+                                                       int64_t n, const int32_t* __restrict__ nmax,
+                                                       int nmax_cap, uint8_t* __restrict__ bin,
+                                                       int* __restrict__ hist) {
+  __shared__ int cnt[kUnitBins];
+  cnt[threadIdx.x] = 0;
+  __syncthreads();
+  const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (u < units) {
+    int64_t a, b;
+    unit_range(g, unit_pts, u, n, a, b);
+    int k = 0;
+    for (int64_t p = a; p < b; ++p) k = max(k, nmax[p]);
+    const int q = unit_bin(k, nmax_cap);
+    bin[u] = (uint8_t)q;
+    atomicAdd(&cnt[q], 1);
+  }
+  __syncthreads();
+  if (cnt[threadIdx.x]) atomicAdd(&hist[threadIdx.x], cnt[threadIdx.x]);
+}
+
+__global__ __launch_bounds__(256) void k_s12_unit_order(int64_t units,
+                                                        const uint8_t* __restrict__ bin,
+                                                        int* __restrict__ hist,
+                                                        int* __restrict__ order) {
+  __shared__ int cnt[kUnitBins], base[kUnitBins], scan[kUnitBins];
+  const int t = threadIdx.x;
+  cnt[t] = 0;
+  scan[t] = hist[t];
+  __syncthreads();
+  for (int h = 1; h < kUnitBins; h <<= 1) {
+    const int v = t >= h ? scan[t - h] : 0;
+    __syncthreads();
+    scan[t] += v;
+    __syncthreads();
+  }
+  const int64_t u = (int64_t)blockIdx.x * 256 + t;
+  int q = 0, rank = 0;
+  if (u < units) {
+    q = bin[u];
+    rank = atomicAdd(&cnt[q], 1);
+  }
+  __syncthreads();
+  if (cnt[t]) base[t] = (t ? scan[t - 1] : 0) + atomicAdd(&hist[kUnitBins + t], cnt[t]);
+  __syncthreads();
+  if (u < units) order[base[q] + rank] = (int)u;
+}
+
+// Unit and first angle of this wavefront.  A unit's angle blocks are launched
+// together, the longest units of all angles first; which angle block comes first
+// moves on by one from unit to unit, so that the eight XCDs, which take the blocks
+// in turn, share the incomplete last one.
+// The grid is one list of units x ablocks blocks, in rows of kGridRow (a launch
+// holds fewer than 2^32 threads in x); false for a block past its end.
+constexpr int kGridRow = 1 << 22;
+__device__ __forceinline__ bool unit_of_block(int64_t units, int ablocks, int wave_angles,
+                                              const int* __restrict__ order, int64_t& unit,
+                                              int& j0) {
+  const int64_t b = (int64_t)blockIdx.y * kGridRow + blockIdx.x;
+  const int64_t u = b / ablocks;
+  if (u >= units) return false;
+  const int ab = (int)((b + u) % ablocks);
+  unit = order ? order[u] : u;
+  j0 = (ab * (int)(blockDim.x >> 6) + (int)(threadIdx.x >> 6)) * wave_angles;
+  return true;
+}
+
+template <int TT, bool RAW>
+__global__ __launch_bounds__(256, 2) void k_s12_tiles(S12Tables T, int64_t n,
+                                                      const int64_t* __restrict__ off,
+                                                      const int32_t* __restrict__ nmax,
+                                                      const double* __restrict__ an,
+                                                      const double* __restrict__ bn, int mode,
+                                                      double* __restrict__ out0,
+                                                      double* __restrict__ out1, int ablocks,
+                                                      const int* __restrict__ order) {
   const int lane = threadIdx.x & 63;
-  const int64_t chunk = blockIdx.x;
-  const int j0 = (blockIdx.y * kRowsWaves + (threadIdx.x >> 6)) * 64;
-  if (j0 >= n_ang) return;   // whole wavefront past the last angle (no barriers below)
+  int64_t p0;
+  int j0;
+  if (!unit_of_block((n + 15) / 16, ablocks, 16 * TT, order, p0, j0)) return;
+  p0 *= 16;
+  if (j0 >= T.n_ang) return;
+  double4_ spr[TT], spi[TT], smr[TT], smi[TT];
+  s12_tile64<TT, RAW, 4, 1>(T, p0, n, j0, lane, off, nmax, an, bn, spr, spi, smr, smi);
+#pragma unroll
+  for (int t = 0; t < TT; ++t) {
+    const int j = j0 + 16 * t + (lane & 15);
+    if (j >= T.n_ang) continue;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int64_t p = p0 + (lane >> 4) + 4 * r;
+      if (p < n)
+        s12_store(mode, p, j, T.n_ang, cd{spr[t][r], spi[t][r]}, cd{smr[t][r], smi[t][r]}, out0,
+                  out1);
+    }
+  }
+}
+
+// ---- S1/S2 -> Mueller -> weighted point sums, fused --------------------------
+//
+// integratePSD integrates each Mueller element of rawMie against a row of PSD
+// weights (dointegration.py:1044-1050, 1164-1166: np.dot(s_ij.T, psd)).  When
+// every weight row covers a contiguous range of points and few rows share a
+// point (the runoptics passes: one block of points per (rh, refractive index),
+// one row per mode), the Mueller planes need not exist in memory: each
+// wavefront forms S1/S2 of 16-point tiles on the matrix cores as k_s12_tiles
+// does, turns them into s11, s12, s33, s34 in registers and adds
+// weight x element into per-row sums.  A block takes one chunk (one or more
+// whole tiles) of one row group (rows with the same range), its wavefronts
+// taking different angles; the sums go to a partial buffer
+// [chunk][RM][4][n_ang] that k_s12_rows_reduce adds up per row in chunk
+// order (deterministic).  Memory traffic drops from 2 x 32 B per (point,
+// angle) to the partials (16 / RM times less per tile).  Chunks of one tile keep
+// the work units small, so the long K loops of large size parameters do not end
+// up in a few long waves; short series take several tiles per chunk.
+
+
+// RM = most rows of one group this instance accumulates.  Per point and angle the
+// weighted sums are of |sp|^2, |sm|^2 and the two parts of sp conj(sm), from
+// which the elements follow once per chunk:
+//   s11 = (|sp|^2 + |sm|^2) / 4, s33 = (|sp|^2 - |sm|^2) / 4,
+//   s12 = -Re(sp conj sm) / 2,   s34 = -Im(sp conj sm) / 2
+// (S1 = (sp + sm) / 2, S2 = (sp - sm) / 2).
+template <int RM, int TT, bool RAW, bool MANY>
+__global__ __launch_bounds__(64 * kRowsWaves, 2) void k_s12_rows_f64(
+    RowGroups g, int chunk_pts, S12Tables T, const int64_t* __restrict__ off,
+    const int32_t* __restrict__ nmax, const double* __restrict__ an,
+    const double* __restrict__ bn, const double* __restrict__ w, int64_t ldw,
+    double* __restrict__ part, int ablocks, const int* __restrict__ order) {
+  const int lane = threadIdx.x & 63;
+  int64_t chunk;
+  int j0;
+  if (!unit_of_block(g.chunk0[g.n_groups], ablocks, 16 * TT, order, chunk, j0)) return;
+  if (j0 >= T.n_ang) return;   // whole wavefront past the last angle (no barriers below)
   int gi = 0;
   while (gi + 1 < g.n_groups && g.chunk0[gi + 1] <= chunk) ++gi;
   const int64_t cstart = g.start[gi] + (chunk - g.chunk0[gi]) * chunk_pts;
   const int64_t cend = min(cstart + (int64_t)chunk_pts, g.start[gi] + g.count[gi]);
   const int nr = g.nrow[gi];
   const double* wr = w + (size_t)g.row0[gi] * ldw;
-  const int i = lane & 15;
-  const int kq = lane >> 4;
-  const int comp = (i >> 2) & 1;
-  double sum[RM][4][4];   // [row][angle sub-tile t][element]
+  const int i = lane & 15, kq = lane >> 4;
+  double* dst = part + (size_t)chunk * RM * 4 * T.n_ang;
+  double4_ spr[TT], spi[TT], smr[TT], smi[TT];
+  // add the weighted products of point q of the lane's four at sub-tile t to s
+  auto add = [&](int t, int q, double wv, double (&s)[4]) {
+    const double pr = spr[t][q], pi = spi[t][q], mr = smr[t][q], mi = smi[t][q];
+    s[0] = fma(wv, fma(pr, pr, pi * pi), s[0]);
+    s[1] = fma(wv, fma(mr, mr, mi * mi), s[1]);
+    s[2] = fma(wv, fma(pr, mr, pi * mi), s[2]);
+    s[3] = fma(wv, fma(pi, mr, -(pr * mi)), s[3]);
+  };
+  // add the four lane groups (lanes i + 16 kq); lane group kq writes element kq
+  auto finish = [&](int r, int t, double (&v)[4]) {
 #pragma unroll
-  for (int r = 0; r < RM; ++r)
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) sum[r][t][e] = 0.0;
-  for (int64_t p0 = cstart; p0 < cend; p0 += 8 * MT) {
-    int nm_a[MT];
-    int64_t oa[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int64_t pa = p0 + 8 * mt + 2 * (i & 3) + (i >> 3);
-      const bool ok = pa < cend;
-      nm_a[mt] = ok ? nmax[pa] : 0;
-      oa[mt] = ok ? off[pa] : 0;
+    for (int e = 0; e < 4; ++e) {
+      v[e] += __shfl_xor(v[e], 16);
+      v[e] += __shfl_xor(v[e], 32);
     }
-    int kmax = 0;
-    for (int q = 0; q < 8 * MT; ++q)
-      if (p0 + q < cend) kmax = max(kmax, nmax[p0 + q]);
-    kmax = min(kmax, nmax_cap);
-    double4_ accp[MT][4], accm[MT][4];
+    const double mine = kq == 0   ? 0.25 * (v[0] + v[1])
+                        : kq == 1 ? -0.5 * v[2]
+                        : kq == 2 ? 0.25 * (v[0] - v[1])
+                                  : -0.5 * v[3];
+    const int j = j0 + 16 * t + i;
+    if (r < nr && j < T.n_ang) dst[((size_t)r * 4 + kq) * T.n_ang + j] = mine;
+  };
+  if (MANY) {
+    // the sums stay in registers from tile to tile
+    double sum[RM][TT][4];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+    for (int r = 0; r < RM; ++r)
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        accp[mt][t] = (double4_){0.0, 0.0, 0.0, 0.0};
-        accm[mt][t] = (double4_){0.0, 0.0, 0.0, 0.0};
-      }
-    double ar_n[MT], br_n[MT], pp_n[4], tt_n[4];
-    auto load_step = [&](int k0) {
-      const int kk = k0 + kq;
+      for (int t = 0; t < TT; ++t)
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        ar_n[mt] = 0.0;
-        br_n[mt] = 0.0;
-        if (kk < nm_a[mt]) {
-          ar_n[mt] = an[2 * (oa[mt] + kk) + comp];
-          br_n[mt] = bn[2 * (oa[mt] + kk) + comp];
+        for (int e = 0; e < 4; ++e) sum[r][t][e] = 0.0;
+    for (int64_t p0 = cstart; p0 < cend; p0 += 16) {
+      s12_tile64<TT, RAW, 2, 2>(T, p0, cend, j0, lane, off, nmax, an, bn, spr, spi, smr, smi);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int64_t p = p0 + kq + 4 * q;
+#pragma unroll
+        for (int r = 0; r < RM; ++r) {
+          const double wv = (r < nr && p < cend) ? wr[(size_t)r * ldw + p] : 0.0;
+#pragma unroll
+          for (int t = 0; t < TT; ++t) add(t, q, wv, sum[r][t]);
         }
       }
-      const bool krow = kk < kmax;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int j = j0 + t * 16 + i;
-        pp_n[t] = 0.0;
-        tt_n[t] = 0.0;
-        if (krow && j < n_ang) {
-          pp_n[t] = pi_t[(size_t)kk * n_ang + j];
-          tt_n[t] = tau_t[(size_t)kk * n_ang + j];
-        }
-      }
-    };
-    if (kmax > 0) load_step(0);
-    for (int k0 = 0; k0 < kmax; k0 += 4) {
-      double ua[MT], va[MT], P[4], M[4];
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        ua[mt] = ar_n[mt] + br_n[mt];
-        va[mt] = ar_n[mt] - br_n[mt];
-      }
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        P[t] = pp_n[t] + tt_n[t];
-        M[t] = pp_n[t] - tt_n[t];
-      }
-      if (k0 + 4 < kmax) load_step(k0 + 4);
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          accp[mt][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ua[mt], P[t], accp[mt][t], 0, 0, 0);
-          accm[mt][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(va[mt], M[t], accm[mt][t], 0, 0, 0);
-        }
     }
-    // lane (i, kq) holds angle j0 + 16 t + i of points p0 + 8 mt + 2 kq + h
-    // (h = 0, 1)
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+    for (int r = 0; r < RM; ++r)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int64_t p = p0 + 8 * mt + 2 * kq + h;
-        double wv[RM];
+      for (int t = 0; t < TT; ++t) finish(r, t, sum[r][t]);
+  } else {
+    // one tile per chunk: no sums in registers while the products run
+    s12_tile64<TT, RAW, 4, 1>(T, cstart, cend, j0, lane, off, nmax, an, bn, spr, spi, smr, smi);
 #pragma unroll
-        for (int r = 0; r < RM; ++r)
-          wv[r] = (r < nr && p < cend) ? wr[(size_t)r * ldw + p] : 0.0;
+    for (int r = 0; r < RM; ++r) {
+      double wv[4];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const cd sp = cd{accp[mt][t][2 * h], accp[mt][t][2 * h + 1]};
-          const cd sm = cd{accm[mt][t][2 * h], accm[mt][t][2 * h + 1]};
-          const cd s1 = (sp + sm) * 0.5, s2 = (sp - sm) * 0.5;
-          const double a1 = norm2(s1), a2 = norm2(s2);
-          const cd c = s1 * conj(s2);
-          const double el[4] = {0.5 * (a1 + a2), 0.5 * (a2 - a1), c.re, c.im};
-#pragma unroll
-          for (int r = 0; r < RM; ++r)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) sum[r][t][e] = fma(wv[r], el[e], sum[r][t][e]);
-        }
+      for (int q = 0; q < 4; ++q) {
+        const int64_t p = cstart + kq + 4 * q;
+        wv[q] = (r < nr && p < cend) ? wr[(size_t)r * ldw + p] : 0.0;
       }
+#pragma unroll
+      for (int t = 0; t < TT; ++t) {
+        double v[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) add(t, q, wv[q], v);
+        finish(r, t, v);
+      }
+    }
   }
-  // add the four point pairs (lanes i + 16 kq) and write; lane group kq
-  // writes element kq
-  double* dst = part + (size_t)chunk * RM * 4 * n_ang;
-#pragma unroll
-  for (int r = 0; r < RM; ++r)
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      double mine = 0.0;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        double v = sum[r][t][e];
-        v += __shfl_xor(v, 16);
-        v += __shfl_xor(v, 32);
-        if (e == kq) mine = v;
-      }
-      const int j = j0 + t * 16 + i;
-      if (r < nr && j < n_ang) dst[((size_t)r * 4 + kq) * n_ang + j] = mine;
-    }
 }
 
 // out[row][e][j] = sum over the row group's chunks of the partials.  A block
@@ -1163,6 +1124,79 @@ __global__ __launch_bounds__(64 * kShChunks) void k_s12_rows_bf16s(
 
 namespace {
 
+// Wavefronts a call should have at least before a wavefront takes more angles
+// (20k points x 181 angles: 158 us a step with 16 angles each, 183 at 32, 213 at
+// 64; 40k x 1801 the same time from 2k to 16k), tiles from which the pairing pass
+// pays (8 to 13 us; 40k points x 1801 angles 3.25 against 3.61 ms, 1.2M x 371
+// 13.7 against 14.5; below 256 tiles the launch costs more than it saves), and the
+// table rows from which units are sorted by length (1.2M points, n_max to 3400:
+// 11.60 against 11.86 ms; 20k points, n_max to 449: 178 us against 168 unsorted).
+constexpr int64_t kS12Want = 8192;
+constexpr int64_t kS12PairTiles = 256;
+constexpr int kS12SortRows = 512;
+
+// The FP64 tiles' shape for `tiles` tiles of 16 points at n_ang angles: 16-angle
+// sub-tiles per wavefront (as many as leave `want` wavefronts), wavefronts per
+// block, and whether the (P, M) pairs are built.
+struct S12Shape {
+  int tt, wpb, ablocks;
+  bool raw;
+};
+S12Shape s12_shape(int64_t tiles, int n_ang, int64_t want, int max_tt = 4) {
+  S12Shape h;
+  const int64_t sub = (n_ang + 15) / 16;
+  h.tt = max_tt;
+  while (h.tt > 1 && tiles * ((sub + h.tt - 1) / h.tt) < want) h.tt >>= 1;
+  const int waves = (int)((sub + h.tt - 1) / h.tt);
+  h.ablocks = (waves + 3) / 4;
+  h.wpb = (waves + h.ablocks - 1) / h.ablocks;
+  h.raw = tiles < kS12PairTiles;
+  return h;
+}
+
+dim3 s12_grid(int64_t blocks) {
+  return dim3((unsigned)std::min<int64_t>(blocks, gm::kGridRow),
+              (unsigned)((blocks + gm::kGridRow - 1) / gm::kGridRow));
+}
+
+// The (P, M) pairs, and the launch order of `units` units of unit_pts points
+// (*order, NULL where the series are too short or the units too few for a long
+// unit at the end to matter: sorting costs two launches, about 10 us).
+int s12_pairs(gm_ctx* ctx, const S12Shape& h, int n_ang, const double* pi_t, const double* tau_t,
+              int nmax_cap, gm::S12Tables& T, const gm::RowGroups& g, int unit_pts, int64_t units,
+              int64_t n, const int32_t* nmax, const int** order, hipStream_t s) {
+  *order = nullptr;
+  T.pi_t = pi_t;
+  T.tau_t = tau_t;
+  T.tab = nullptr;
+  T.n_ang = n_ang;
+  T.apad = (n_ang + 63) / 64 * 64;
+  T.nmax_cap = nmax_cap;
+  if (h.raw) return GM_OK;
+  const int64_t total = (int64_t)((nmax_cap + 3) / 4 * 4) * T.apad;
+  const bool sorted = nmax_cap >= kS12SortRows && units >= 1024 && units <= 0x7fffffffLL;
+  // pairs, then (sorted) the histogram and its cursors, the order and the bins
+  const size_t o_hist = (size_t)total * sizeof(double2);
+  const size_t o_ord = o_hist + 2 * gm::kUnitBins * sizeof(int);
+  const size_t o_bin = o_ord + (size_t)units * sizeof(int);
+  int rc = ctx->reserve(ctx->tab_lp, sorted ? o_bin + (size_t)units : o_hist);
+  if (rc) return rc;
+  char* ws = (char*)ctx->tab_lp.ptr;
+  int* hist = sorted ? (int*)(ws + o_hist) : nullptr;
+  T.tab = (const double2*)ws;
+  hipLaunchKernelGGL(gm::k_s12_prep_pairs, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s,
+                     n_ang, nmax_cap, T.apad, total, pi_t, tau_t, (double2*)ws, hist);
+  if (sorted) {
+    const dim3 gu((unsigned)((units + 255) / 256));
+    hipLaunchKernelGGL(gm::k_s12_unit_bins, gu, dim3(256), 0, s, g, unit_pts, units, n, nmax,
+                       nmax_cap, (uint8_t*)(ws + o_bin), hist);
+    hipLaunchKernelGGL(gm::k_s12_unit_order, gu, dim3(256), 0, s, units,
+                       (const uint8_t*)(ws + o_bin), hist, (int*)(ws + o_ord));
+    *order = (const int*)(ws + o_ord);
+  }
+  return GM_OK;
+}
+
 // Launch the S1/S2 contraction at the requested precision.  Tables for the
 // reduced-precision paths are rebuilt on every call (one pass over pi, tau:
 // small next to the contraction itself).
@@ -1178,35 +1212,24 @@ int launch_s12(gm_ctx* ctx, const char* who, int64_t n, const int64_t* off, cons
   const int wpb = ctx->tune_s12_waves;
   dim3 grid((unsigned)((n + 7) / 8), (unsigned)((n_ang + 64 * wpb - 1) / (64 * wpb)));
   dim3 block(64 * wpb);
-  const int wave_points = ctx->tune_s12_layout;   // FP64 kernel only
   size_t slot;
   if (precision == GM_PREC_FP64) {
     ctx->mark_begin(gm::kKS12, s, &slot);
-    const int pts = ctx->tune_s12_points == 16 ? 16 : 8;
-    if (wave_points == 2) {   // LDS-staged angle tables, 8 or 16 points per wavefront
-      const int64_t per_block = (int64_t)pts * gm::kS12LdsWaves;
-      dim3 gl((unsigned)((n + per_block - 1) / per_block), (unsigned)((n_ang + 63) / 64));
-      if (pts == 16)
-        hipLaunchKernelGGL(gm::k_s12_f64_lds<2>, gl, dim3(64 * gm::kS12LdsWaves), 0, s, n, off,
-                           nmax, an, bn, n_ang, pi_t, tau_t, nmax_cap, mode, out0, out1);
-      else
-        hipLaunchKernelGGL(gm::k_s12_f64_lds<1>, gl, dim3(64 * gm::kS12LdsWaves), 0, s, n, off,
-                           nmax, an, bn, n_ang, pi_t, tau_t, nmax_cap, mode, out0, out1);
-      ctx->mark_end(slot, s);
-      e = hipGetLastError();
-      if (e != hipSuccess) return gm_fail(GM_ERUNTIME, "%s: %s", who, hipGetErrorString(e));
-      return GM_OK;
-    }
-    dim3 g = wave_points
-                 ? dim3((unsigned)((n + (int64_t)pts * wpb - 1) / ((int64_t)pts * wpb)),
-                        (unsigned)((n_ang + 63) / 64))
-                 : dim3((unsigned)((n + pts - 1) / pts), grid.y);
-    if (pts == 16)
-      hipLaunchKernelGGL(gm::k_s12_f64<2>, g, block, 0, s, n, off, nmax, an, bn, n_ang, pi_t,
-                         tau_t, nmax_cap, mode, wave_points, out0, out1);
-    else
-      hipLaunchKernelGGL(gm::k_s12_f64<1>, g, block, 0, s, n, off, nmax, an, bn, n_ang, pi_t,
-                         tau_t, nmax_cap, mode, wave_points, out0, out1);
+    const S12Shape h = s12_shape((n + 15) / 16, n_ang, kS12Want);
+    gm::S12Tables T;
+    const int* order;
+    gm::RowGroups none{};
+    const int rc = s12_pairs(ctx, h, n_ang, pi_t, tau_t, nmax_cap, T, none, 16, (n + 15) / 16, n,
+                             nmax, &order, s);
+    if (rc) return rc;
+    const dim3 g = s12_grid((n + 15) / 16 * h.ablocks);
+#define GM_TILES(T_, R_)                                                                       \
+  hipLaunchKernelGGL((gm::k_s12_tiles<T_, R_>), g, dim3(64 * h.wpb), 0, s, T, n, off, nmax, an, \
+                     bn, mode, out0, out1, h.ablocks, order)
+    if (h.tt == 4) { if (h.raw) GM_TILES(4, true); else GM_TILES(4, false); }
+    else if (h.tt == 2) { if (h.raw) GM_TILES(2, true); else GM_TILES(2, false); }
+    else { if (h.raw) GM_TILES(1, true); else GM_TILES(1, false); }
+#undef GM_TILES
     ctx->mark_end(slot, s);
   } else {
     const int kpad = (nmax_cap + gm::kLpK - 1) / gm::kLpK * gm::kLpK;
@@ -1303,33 +1326,31 @@ int gm_s12_contract_rows(gm_ctx* ctx, int64_t n, const int64_t* coef_off, const 
                                     "coefficients of gm_s12_split_coef (coef_lp)");
   if (nmax_cap < 1) return gm_fail(GM_EINVAL, "gm_s12_contract_rows: nmax_cap must be >= 1");
   // rows with the same range form a group (at most 4 rows; a longer run of
-  // equal ranges is split, its points then contracted once per group).  One
-  // 8-point tile per chunk, two when that still leaves >= 16k wavefronts.
-  int64_t tiles = 0;
+  // rows with the same range form a group (at most 4 rows; a longer run of
+  // equal ranges is split, its points then contracted once per group).
   for (int r = 0; r < n_rows; ++r)
     if (count_host[r] > 0) tiles += (count_host[r] + 7) / 8;
   const int64_t ablocks = (n_ang + 64 * gm::kRowsWaves - 1) / (64 * gm::kRowsWaves);
-  // most rows of one group (consecutive rows with the same range, at most 4)
-  int rm_pre = 1;
-  for (int r = 1, run = 1; r < n_rows; ++r) {
-    run = (start_host[r] == start_host[r - 1] && count_host[r] == count_host[r - 1] && run < 4)
-              ? run + 1 : 1;
-    rm_pre = max(rm_pre, run);
-  }
-  // tiles per chunk.  The kernels multiply two tiles together, sharing each
-  // angle-table fetch (FP64 with one row sum per group; otherwise FP64 walks
-  // the tiles one after the other, which pays for short series only: fewer
-  // work units and half the partial sums where the K loop is short).  Two
-  // when that still leaves >= 16k wavefronts at FP64, >= 8k at FP32 and
-  // split-BF16.
+  // FP32 and split-BF16: 8-point tiles multiplied together per chunk, two when that
+  // still leaves >= 8k wavefronts.
   const int64_t waves2 = (tiles / 2) * ablocks * gm::kRowsWaves;
-  const int row_tiles =
-      ctx->tune_s12_row_tiles
-          ? ctx->tune_s12_row_tiles
-          : (precision == GM_PREC_FP64
-                 ? ((rm_pre == 1 || nmax_cap <= 256) && waves2 >= 16384 ? 2 : 1)
-                 : (waves2 >= 8192 ? 2 : 1));
-  const int chunk_pts = 8 * row_tiles;
+  const int row_tiles = ctx->tune_s12_row_tiles ? ctx->tune_s12_row_tiles : (waves2 >= 8192 ? 2 : 1);
+  // FP64: 16-point tiles; for short series several one after the other (fewer
+  // partial sums) while that leaves work for the whole chip
+  bool many = false;   // a group of several rows
+  for (int r = 1; r < n_rows; ++r)
+    many |= start_host[r] == start_host[r - 1] && count_host[r] == count_host[r - 1];
+  S12Shape h64 = s12_shape((tiles + 1) / 2, n_ang, kS12Want);
+  int64_t per = 1;
+  while (per < 8 && nmax_cap <= 256 &&
+         (tiles / 2) / (2 * per) * h64.ablocks * h64.wpb >= 2 * kS12Want)
+    per *= 2;
+  if (ctx->tune_s12_row_tiles) per = ctx->tune_s12_row_tiles;
+  if (per > 1) {   // the sums of all rows take registers: fewer sub-tiles for several rows
+    h64 = s12_shape(tiles, n_ang, 0, many ? 2 : 4);
+    h64.raw = false;
+  }
+  const int chunk_pts = precision == GM_PREC_FP64 ? (int)(16 * per) : 8 * row_tiles;
   gm::RowGroups g;
   g.n_groups = 0;
   g.chunk0[0] = 0;
@@ -1371,19 +1392,25 @@ int gm_s12_contract_rows(gm_ctx* ctx, int64_t n, const int64_t* coef_off, const 
   size_t slot;
   if (precision == GM_PREC_FP64) {
     ctx->mark_begin(gm::kKS12, s, &slot);
-    // two tiles multiplied together where a chunk has two and one row sum per
-    // group (one table load feeds both tiles; with more row sums two tiles
-    // leave one wavefront per SIMD)
-#define GM_ROWS_F64(R_, M_)                                                                    \
-  hipLaunchKernelGGL((gm::k_s12_rows_f64<R_, M_>), grid, block, 0, s, g, chunk_pts, coef_off, \
-                     nmax, an, bn, n_ang, pi_t, tau_t, nmax_cap, w, n, part)
-    if (RM == 1) {
-      if (row_tiles >= 2) GM_ROWS_F64(1, 2); else GM_ROWS_F64(1, 1);
-    } else if (RM == 2) {
-      GM_ROWS_F64(2, 1);
-    } else {
-      GM_ROWS_F64(4, 1);
-    }
+    gm::S12Tables T;
+    const int* order;
+    if ((rc = s12_pairs(ctx, h64, n_ang, pi_t, tau_t, nmax_cap, T, g, chunk_pts, chunks, n, nmax,
+                        &order, s)))
+      return rc;
+    const dim3 g64 = s12_grid(chunks * h64.ablocks);
+#define GM_ROWS_F64(R_, T_, W_, M_)                                                              \
+  hipLaunchKernelGGL((gm::k_s12_rows_f64<R_, T_, W_, M_>), g64, dim3(64 * h64.wpb), 0, s, g,        \
+                     chunk_pts, T, coef_off, nmax, an, bn, w, n, part, h64.ablocks, order)
+#define GM_ROWS_F64_T(R_)                                                                      \
+  if (per > 1) GM_ROWS_F64(R_, (R_ == 1 ? 4 : 2), false, true);                                 \
+  else if (h64.tt == 4 && h64.raw) GM_ROWS_F64(R_, 4, true, false);                             \
+  else if (h64.tt == 4) GM_ROWS_F64(R_, 4, false, false);                                       \
+  else if (h64.tt == 2 && h64.raw) GM_ROWS_F64(R_, 2, true, false);                             \
+  else if (h64.tt == 2) GM_ROWS_F64(R_, 2, false, false);                                       \
+  else if (h64.raw) GM_ROWS_F64(R_, 1, true, false);                                            \
+  else GM_ROWS_F64(R_, 1, false, false);
+    if (RM == 1) { GM_ROWS_F64_T(1) } else if (RM == 2) { GM_ROWS_F64_T(2) } else { GM_ROWS_F64_T(4) }
+#undef GM_ROWS_F64_T
 #undef GM_ROWS_F64
     ctx->mark_end(slot, s);
   } else {

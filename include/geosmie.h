@@ -85,18 +85,18 @@ int gm_ctx_check(gm_ctx* ctx, gm_stream stream, int32_t* flags_host);
  * budgets let the compiler fuse a different set of multiply-adds. */
 enum gm_tune_param {
   GM_TUNE_MIE_GRID_MULT = 0,  /* persistent Mie grid = this x resident wavefronts (1..16; 1) */
-  GM_TUNE_S12_WAVES = 1,      /* wavefronts of 64 angles per S1/S2 block (1, 2, 4; 4) */
+  GM_TUNE_S12_WAVES = 1,      /* wavefronts of 64 angles per S1/S2 block at FP32 and split-BF16
+                                   (1, 2, 4; 4); FP64 chooses from the sizes */
   GM_TUNE_PSD_CHUNK = 2,      /* points per split-K chunk, few-PSD contraction (16..2^20; 128) */
   GM_TUNE_MLP_WEIGHT_TERMS = 3, /* precision, not shape: BF16 terms per MLP weight on the matrix
                                    cores, 1 = BF16 weights (default), 2 = hi + lo BF16 pair */
-  GM_TUNE_S12_POINTS = 4,       /* points per wavefront of the FP64 S1/S2 kernel (8, 16; 8) */
+  GM_TUNE_S12_POINTS = 4,       /* accepted (8, 16; 8), no effect: the FP64 S1/S2 kernel takes 16
+                                   points per wavefront */
   GM_TUNE_MIE_WAVES = 5         /* Mie recurrence kernels' register budget: 0 = unconstrained
                                    (default), 3 or 4 = at least that many resident wavefronts
                                    per SIMD (fewer registers, a few spills) */,
-  GM_TUNE_S12_LAYOUT = 6        /* FP64 S1/S2 blocks: 0 = the block's wavefronts take different
-                                   angles of the same points (default), 1 = different points
-                                   of the same 64 angles (angle-table rows shared in cache),
-                                   2 = as 1 with the angle tables staged through LDS */,
+  GM_TUNE_S12_LAYOUT = 6        /* accepted (0, 1, 2; 0), no effect: the FP64 S1/S2 kernel has one
+                                   block layout */,
   GM_TUNE_MIE_CKPT = 7          /* coated kernel (real / weakly absorbing shells): the downward
                                    chains' states kept every 4, 5 or 8 rows and each block of rows
                                    regenerated in LDS before use (4, the default), or 0 = every
@@ -112,10 +112,10 @@ enum gm_tune_param {
   GM_TUNE_PSD_QUIRKS = 9,       /* a behaviour setting, not tuned for speed: the integratePSD
                                    quirks gm_integrate_psd[_rows] reproduce (GM_PSD_QUIRK_* bits;
                                    default GM_PSD_QUIRK_ALIAS) */
-  GM_TUNE_S12_ROW_TILES = 10,   /* gm_s12_contract_rows: 8-point tiles per work unit (1, 2, 4): at
-                                   FP64 one after the other, at FP32 / split-BF16 multiplied
-                                   together, sharing each angle-table fetch; 0 (default) = by
-                                   batch size.  Results agree to rounding */
+  GM_TUNE_S12_ROW_TILES = 10,   /* gm_s12_contract_rows: tiles per work unit (1, 2, 4): at FP64
+                                   16-point tiles one after the other, at FP32 / split-BF16
+                                   8-point tiles multiplied together, sharing each angle-table
+                                   fetch; 0 (default) = by batch size.  Results agree to rounding */
   GM_TUNE_S12_SHARE = 11        /* gm_s12_contract_rows at split-BF16 with one tile per work
                                    unit: 1 (default) = four work units per block share each
                                    K-step's angle-table tile through LDS; 0 = each wavefront

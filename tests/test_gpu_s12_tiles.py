@@ -1,0 +1,89 @@
+"""FP64 S1/S2 tiles (16 points x 16, 32 or 64 angles per wavefront, angle tables
+paired or read as they are, units in point order or longest first) against the
+same sums by dense FP64 products of the same coefficients and tables.
+
+The kernel adds the K terms in groups of four, the reference in torch's order:
+both are FP64 sums of n_max <= 60 terms, so they agree within n_max * 2^-53 of
+the sum of the terms' magnitudes; 1e-13 of max|S| (S at 0 degrees is that sum
+up to a factor of a few) leaves an order of magnitude.  P11 and the row sums
+are quadratic in S: twice that of their largest value.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _setup(n, n_ang, cap):
+    import torch
+    from geosmie_amd.lut import _DevMie
+    from geosmie_amd.s12 import angle_tables_dev
+    rng = np.random.default_rng(n + n_ang)
+    dm = _DevMie(10 ** rng.uniform(-1.5, 1.5, n), complex(1.5, 0.01))
+    cost = np.cos(np.radians(np.linspace(0.0, 180.0, n_ang))) if n_ang > 1 else np.array([0.3])
+    pi_t, tau_t = angle_tables_dev(cost, max(cap, dm.nmax_max))
+    k = dm.nmax_max
+    idx = torch.arange(k, device="cuda")
+    live = idx[None, :] < dm.d_nmax[:, None]
+    at = (dm.d_off[:-1, None] + idx[None, :]).clamp(max=dm.d_an.numel() // 2 - 1)
+    a, b = (torch.where(live, torch.view_as_complex(c.view(-1, 2))[at], 0) for c in
+            (dm.d_an, dm.d_bn))
+
+    def mul(c, t):
+        return torch.complex(c.real.contiguous() @ t[:k], c.imag.contiguous() @ t[:k])
+    return dm, pi_t, tau_t, mul(a, pi_t) + mul(b, tau_t), mul(a, tau_t) + mul(b, pi_t)
+
+
+# one point and angle; ragged tiles; wavefronts of 16, 32 and 64 angles; 4100 points
+# for the paired tables; 17000 with a 520-row table for the sorted order
+@pytest.mark.parametrize("n,n_ang,cap", [(1, 1, 0), (15, 17, 0), (17, 371, 0), (4100, 16, 0),
+                                         (4100, 371, 0), (4097, 1801, 0), (17000, 130, 520)])
+def test_amplitudes_and_p11(gpu, n, n_ang, cap):
+    import torch
+    from geosmie_amd import _lib
+    from geosmie_amd._lib import check, ptr
+    dm, pi_t, tau_t, s1, s2 = _setup(n, n_ang, cap)
+    d1, d2 = dm.s12(pi_t, tau_t)
+    scale = max(float(s1.abs().max()), float(s2.abs().max()))
+    for d, s in ((d1, s1), (d2, s2)):
+        got = torch.view_as_complex(d.view(n, n_ang, 2))
+        assert float((got - s).abs().max()) <= 1e-13 * scale
+    p11 = torch.empty((n, n_ang), dtype=torch.float64, device="cuda")
+    check(_lib.lib().gm_s12_p11(_lib.ctx(), n, ptr(dm.d_off), ptr(dm.d_nmax), ptr(dm.d_an),
+                                ptr(dm.d_bn), n_ang, ptr(pi_t), ptr(tau_t), int(pi_t.shape[0]),
+                                ptr(p11), 0, _lib.stream()), "gm_s12_p11")
+    ref = (s1.abs() ** 2 + s2.abs() ** 2) / 2
+    assert float((p11 - ref).abs().max()) <= 2e-13 * float(ref.max())
+
+
+# rows with their own ranges and rows sharing one (1, 2 and 4 sums per group), one
+# tile per chunk and several (short series, many points), sorted chunks
+@pytest.mark.parametrize("n,n_ang,cap,share", [(33, 19, 0, 1), (5000, 371, 0, 2),
+                                               (60000, 371, 0, 1), (60000, 371, 0, 4),
+                                               (17000, 130, 520, 2)])
+def test_row_sums(gpu, n, n_ang, cap, share):
+    import torch
+    from geosmie_amd import _lib
+    from geosmie_amd._lib import check, ptr
+    dm, pi_t, tau_t, s1, s2 = _setup(n, n_ang, cap)
+    cut = n // 3 + 1
+    ranges = [(0, cut)] * share + [(cut, n - cut)] * share
+    w = torch.zeros((len(ranges), n), dtype=torch.float64, device="cuda")
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    for r, (a, c) in enumerate(ranges):
+        w[r, a:a + c] = torch.rand(c, generator=gen, dtype=torch.float64, device="cuda")
+    k = len(ranges)
+    out = torch.empty((k, 4, n_ang), dtype=torch.float64, device="cuda")
+    st = (ctypes.c_int64 * k)(*[a for a, _ in ranges])
+    ct = (ctypes.c_int64 * k)(*[c for _, c in ranges])
+    check(_lib.lib().gm_s12_contract_rows(_lib.ctx(), n, ptr(dm.d_off), ptr(dm.d_nmax),
+                                          ptr(dm.d_an), ptr(dm.d_bn), n_ang, ptr(pi_t), ptr(tau_t),
+                                          int(pi_t.shape[0]), k, st, ct, ptr(w), ptr(out), 0, None,
+                                          _lib.stream()), "gm_s12_contract_rows")
+    a1, a2, c = s1.abs() ** 2, s2.abs() ** 2, s1 * s2.conj()
+    for e, v in enumerate(((a1 + a2) / 2, (a2 - a1) / 2, c.real, c.imag)):
+        ref = w @ v.contiguous()
+        bound = 2e-13 * float((w @ ((a1 + a2) / 2)).max())
+        assert float((out[:, e] - ref).abs().max()) <= bound, e
