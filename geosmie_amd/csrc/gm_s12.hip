@@ -1326,8 +1326,8 @@ int gm_s12_contract_rows(gm_ctx* ctx, int64_t n, const int64_t* coef_off, const 
                                     "coefficients of gm_s12_split_coef (coef_lp)");
   if (nmax_cap < 1) return gm_fail(GM_EINVAL, "gm_s12_contract_rows: nmax_cap must be >= 1");
   // rows with the same range form a group (at most 4 rows; a longer run of
-  // rows with the same range form a group (at most 4 rows; a longer run of
   // equal ranges is split, its points then contracted once per group).
+  int64_t tiles = 0;
   for (int r = 0; r < n_rows; ++r)
     if (count_host[r] > 0) tiles += (count_host[r] + 7) / 8;
   const int64_t ablocks = (n_ang + 64 * gm::kRowsWaves - 1) / (64 * gm::kRowsWaves);
