@@ -27,6 +27,7 @@
 // per-lane element order as the FP64 kernel: (0,1) = point p0 + 2g (re, im),
 // (2,3) = point p0 + 2g + 1.
 #include <algorithm>
+#include <type_traits>
 
 #include "gm_complex.h"
 #include "gm_ctx.h"
@@ -103,10 +104,32 @@ __global__ __launch_bounds__(256) void k_s12_prep_pairs(int n_ang, int nmax_cap,
   tab[id] = v;
 }
 
+// The same as FP32 pairs; total counts pairs.
+__global__ __launch_bounds__(256) void k_s12_prep_pairs32(int n_ang, int nmax_cap, int apad,
+                                                          int64_t total,
+                                                          const double* __restrict__ pi_t,
+                                                          const double* __restrict__ tau_t,
+                                                          float2* __restrict__ tab,
+                                                          int* __restrict__ hist) {
+  const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (hist && blockIdx.x == 0)
+    for (int b = threadIdx.x; b < 2 * kUnitBins; b += 256) hist[b] = 0;
+  if (id >= total) return;
+  const int k = (int)(id / apad), j = (int)(id - (int64_t)k * apad);
+  double P = 0.0, M = 0.0;
+  if (k < nmax_cap && j < n_ang) {
+    const double p = pi_t[(size_t)k * n_ang + j], t = tau_t[(size_t)k * n_ang + j];
+    P = p + t;
+    M = p - t;
+  }
+  tab[id] = make_float2((float)P, (float)M);
+}
+
 struct S12Tables {
   const double* pi_t;
   const double* tau_t;
   const double2* tab;   // (P, M) [k][apad], zero padded; NULL: RAW
+  const float2* tab32;  // FP32 (P, M)
   int n_ang, apad, nmax_cap;
 };
 
@@ -281,6 +304,103 @@ __global__ __launch_bounds__(256) void k_s12_unit_order(int64_t units,
   if (u < units) order[base[q] + rank] = (int)u;
 }
 
+// The same sums at FP32 (v_mfma_f32_16x16x4_f32, results in FP32): U, V rounded from
+// FP64 sums, tables FP32 pairs.  A lane loads the pairs of two neighbouring angles
+// as 16 bytes: sub-tiles t and t + 1 (t even) are the even and odd columns of 32
+// angles, column i of sub-tile t being angle j0 + 16 (t & ~1) + 2 i + (t & 1).
+// Element r of lane (i, g) is point p0 + 4 g + r.  LP: the coefficients come from
+// gm_s12_split_coef, 16 bytes {U.re, V.re, U.im, V.im} a term.  Tiles of 8 points and
+// 64 angles spent 8 8-byte or 4-byte loads and two coefficient loads on 8 MFMAs of
+// half the FP64 length: 40k points x 1801 angles with row sums 1.51 -> 1.02 ms, P11
+// of 1.5M points x 371 angles 6.2 -> 4.6 ms.
+template <int TT, bool LP, int kCd>
+__device__ __forceinline__ void s12_tile32(const S12Tables& T, int64_t p0, int64_t pend, int j0,
+                                           int lane, const int64_t* __restrict__ off,
+                                           const int32_t* __restrict__ nmax,
+                                           const double* __restrict__ an,
+                                           const double* __restrict__ bn,
+                                           const float4* __restrict__ cf, float4_ (&spr)[TT],
+                                           float4_ (&spi)[TT], float4_ (&smr)[TT],
+                                           float4_ (&smi)[TT]) {
+  const int i = lane & 15, kq = lane >> 4;
+  const int64_t pc = min(p0 + i, pend - 1);
+  const int nm = min(nmax[pc], T.nmax_cap);
+  const int64_t o = nm > 0 ? off[pc] : 0;
+  int kmax = nm, kmin = nm;
+#pragma unroll
+  for (int h = 1; h < 16; h <<= 1) {
+    kmax = max(kmax, __shfl_xor(kmax, h));
+    kmin = min(kmin, __shfl_xor(kmin, h));
+  }
+  kmax = __builtin_amdgcn_readfirstlane(kmax);
+  kmin = __builtin_amdgcn_readfirstlane(kmin);
+#pragma unroll
+  for (int t = 0; t < TT; ++t) spr[t] = spi[t] = smr[t] = smi[t] = (float4_){0.f, 0.f, 0.f, 0.f};
+  if (kmax <= 0) return;
+  const double2* pa = (const double2*)an + o;
+  const double2* pb = (const double2*)bn + o;
+  const float4* pc4 = cf + o;
+  const int last = max(nm - 1, 0), row_last = (kmax + 3) / 4 * 4 - 1;
+  double2 a_n[LP ? 1 : kCd], b_n[LP ? 1 : kCd];
+  float4 c_n[LP ? kCd : 1], t_n[TT / 2];
+  auto load_tab = [&](int k0) {
+    const float2* row = T.tab32 + (size_t)min(k0 + kq, row_last) * T.apad + j0 + 2 * i;
+#pragma unroll
+    for (int h = 0; h < TT / 2; ++h) t_n[h] = *(const float4*)(row + 32 * h);
+  };
+  auto load_coef = [&](int k0, int q) {
+    const int kc = min(k0 + kq, last);
+    if (LP) {
+      c_n[LP ? q : 0] = pc4[kc];
+    } else {
+      a_n[LP ? 0 : q] = pa[kc];
+      b_n[LP ? 0 : q] = pb[kc];
+    }
+  };
+  load_tab(0);
+#pragma unroll
+  for (int q = 0; q < kCd; ++q) load_coef(4 * q, q);
+  for (int kb = 0; kb < kmax; kb += 4 * kCd) {
+#pragma unroll
+    for (int q = 0; q < kCd; ++q) {
+      const int k0 = kb + 4 * q;
+      if (k0 >= kmax) break;
+      float ur, ui, vr, vi;
+      if (LP) {
+        const float4 c = c_n[LP ? q : 0];
+        ur = c.x;
+        vr = c.y;
+        ui = c.z;
+        vi = c.w;
+      } else {
+        const double2 a = a_n[LP ? 0 : q], b = b_n[LP ? 0 : q];
+        ur = (float)(a.x + b.x);
+        ui = (float)(a.y + b.y);
+        vr = (float)(a.x - b.x);
+        vi = (float)(a.y - b.y);
+      }
+      if (k0 + 4 > kmin && k0 + kq >= nm) ur = ui = vr = vi = 0.f;
+      float P[TT], M[TT];
+#pragma unroll
+      for (int h = 0; h < TT / 2; ++h) {
+        P[2 * h] = t_n[h].x;
+        M[2 * h] = t_n[h].y;
+        P[2 * h + 1] = t_n[h].z;
+        M[2 * h + 1] = t_n[h].w;
+      }
+      load_tab(k0 + 4);
+      load_coef(k0 + 4 * kCd, q);
+#pragma unroll
+      for (int t = 0; t < TT; ++t) {
+        spr[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(ur, P[t], spr[t], 0, 0, 0);
+        spi[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(ui, P[t], spi[t], 0, 0, 0);
+        smr[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr, M[t], smr[t], 0, 0, 0);
+        smi[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(vi, M[t], smi[t], 0, 0, 0);
+      }
+    }
+  }
+}
+
 // Unit and first angle of this wavefront.  A unit's angle blocks are launched
 // together, the longest units of all angles first; which angle block comes first
 // moves on by one from unit to unit, so that the eight XCDs, which take the blocks
@@ -331,6 +451,37 @@ __global__ __launch_bounds__(256, 2) void k_s12_tiles(S12Tables T, int64_t n,
   }
 }
 
+template <int TT>
+__global__ __launch_bounds__(256, 2) void k_s12_tiles32(S12Tables T, int64_t n,
+                                                        const int64_t* __restrict__ off,
+                                                        const int32_t* __restrict__ nmax,
+                                                        const double* __restrict__ an,
+                                                        const double* __restrict__ bn, int mode,
+                                                        double* __restrict__ out0,
+                                                        double* __restrict__ out1, int ablocks,
+                                                        const int* __restrict__ order) {
+  const int lane = threadIdx.x & 63;
+  int64_t p0;
+  int j0;
+  if (!unit_of_block((n + 15) / 16, ablocks, 16 * TT, order, p0, j0)) return;
+  p0 *= 16;
+  if (j0 >= T.n_ang) return;
+  float4_ spr[TT], spi[TT], smr[TT], smi[TT];
+  s12_tile32<TT, false, 4>(T, p0, n, j0, lane, off, nmax, an, bn, nullptr, spr, spi, smr, smi);
+#pragma unroll
+  for (int t = 0; t < TT; ++t) {
+    const int j = j0 + 16 * (t & ~1) + 2 * (lane & 15) + (t & 1);
+    if (j >= T.n_ang) continue;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int64_t p = p0 + 4 * (lane >> 4) + r;
+      if (p < n)
+        s12_store(mode, p, j, T.n_ang, cd{(double)spr[t][r], (double)spi[t][r]},
+                  cd{(double)smr[t][r], (double)smi[t][r]}, out0, out1);
+    }
+  }
+}
+
 // ---- S1/S2 -> Mueller -> weighted point sums, fused --------------------------
 //
 // integratePSD integrates each Mueller element of rawMie against a row of PSD
@@ -356,11 +507,12 @@ __global__ __launch_bounds__(256, 2) void k_s12_tiles(S12Tables T, int64_t n,
 //   s11 = (|sp|^2 + |sm|^2) / 4, s33 = (|sp|^2 - |sm|^2) / 4,
 //   s12 = -Re(sp conj sm) / 2,   s34 = -Im(sp conj sm) / 2
 // (S1 = (sp + sm) / 2, S2 = (sp - sm) / 2).
-template <int RM, int TT, bool RAW, bool MANY>
-__global__ __launch_bounds__(64 * kRowsWaves, 2) void k_s12_rows_f64(
+template <int PREC, int RM, int TT, bool RAW, bool MANY>
+__global__ __launch_bounds__(64 * kRowsWaves, 2) void k_s12_rows(
     RowGroups g, int chunk_pts, S12Tables T, const int64_t* __restrict__ off,
     const int32_t* __restrict__ nmax, const double* __restrict__ an,
-    const double* __restrict__ bn, const double* __restrict__ w, int64_t ldw,
+    const double* __restrict__ bn, const float4* __restrict__ cf, const double* __restrict__ w,
+    int64_t ldw,
     double* __restrict__ part, int ablocks, const int* __restrict__ order) {
   const int lane = threadIdx.x & 63;
   int64_t chunk;
@@ -375,7 +527,18 @@ __global__ __launch_bounds__(64 * kRowsWaves, 2) void k_s12_rows_f64(
   const double* wr = w + (size_t)g.row0[gi] * ldw;
   const int i = lane & 15, kq = lane >> 4;
   double* dst = part + (size_t)chunk * RM * 4 * T.n_ang;
-  double4_ spr[TT], spi[TT], smr[TT], smi[TT];
+  constexpr bool F64 = PREC == GM_PREC_FP64;
+  using Acc = std::conditional_t<F64, double4_, float4_>;
+  Acc spr[TT], spi[TT], smr[TT], smi[TT];
+  auto tile = [&](int64_t p0, auto depth, auto ahead) {
+    if constexpr (F64)
+      s12_tile64<TT, RAW, depth(), ahead()>(T, p0, cend, j0, lane, off, nmax, an, bn, spr, spi,
+                                            smr, smi);
+    else
+      s12_tile32<TT, true, 4>(T, p0, cend, j0, lane, off, nmax, an, bn, cf, spr, spi, smr, smi);
+  };
+  // point q of the lane's four
+  auto point = [&](int64_t p0, int q) { return p0 + (F64 ? kq + 4 * q : 4 * kq + q); };
   // add the weighted products of point q of the lane's four at sub-tile t to s
   auto add = [&](int t, int q, double wv, double (&s)[4]) {
     const double pr = spr[t][q], pi = spi[t][q], mr = smr[t][q], mi = smi[t][q];
@@ -395,7 +558,7 @@ __global__ __launch_bounds__(64 * kRowsWaves, 2) void k_s12_rows_f64(
                         : kq == 1 ? -0.5 * v[2]
                         : kq == 2 ? 0.25 * (v[0] - v[1])
                                   : -0.5 * v[3];
-    const int j = j0 + 16 * t + i;
+    const int j = F64 ? j0 + 16 * t + i : j0 + 16 * (t & ~1) + 2 * i + (t & 1);
     if (r < nr && j < T.n_ang) dst[((size_t)r * 4 + kq) * T.n_ang + j] = mine;
   };
   if (MANY) {
@@ -408,10 +571,10 @@ __global__ __launch_bounds__(64 * kRowsWaves, 2) void k_s12_rows_f64(
 #pragma unroll
         for (int e = 0; e < 4; ++e) sum[r][t][e] = 0.0;
     for (int64_t p0 = cstart; p0 < cend; p0 += 16) {
-      s12_tile64<TT, RAW, 2, 2>(T, p0, cend, j0, lane, off, nmax, an, bn, spr, spi, smr, smi);
+      tile(p0, std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{});
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int64_t p = p0 + kq + 4 * q;
+        const int64_t p = point(p0, q);
 #pragma unroll
         for (int r = 0; r < RM; ++r) {
           const double wv = (r < nr && p < cend) ? wr[(size_t)r * ldw + p] : 0.0;
@@ -426,13 +589,13 @@ __global__ __launch_bounds__(64 * kRowsWaves, 2) void k_s12_rows_f64(
       for (int t = 0; t < TT; ++t) finish(r, t, sum[r][t]);
   } else {
     // one tile per chunk: no sums in registers while the products run
-    s12_tile64<TT, RAW, 4, 1>(T, cstart, cend, j0, lane, off, nmax, an, bn, spr, spi, smr, smi);
+    tile(cstart, std::integral_constant<int, 4>{}, std::integral_constant<int, 1>{});
 #pragma unroll
     for (int r = 0; r < RM; ++r) {
       double wv[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int64_t p = cstart + kq + 4 * q;
+        const int64_t p = point(cstart, q);
         wv[q] = (r < nr && p < cend) ? wr[(size_t)r * ldw + p] : 0.0;
       }
 #pragma unroll
@@ -496,14 +659,13 @@ __device__ __forceinline__ void bf16_split(double x, unsigned short& hi, unsigne
   lo = bf16_rne((float)(x - (double)bf16_val(hi)));
 }
 
-// P = pi + tau and M = pi - tau from the FP64 tables [k][angle] (k < nmax_cap).
-//   FP32 : t32[2][kpad][apad]            (plane 0 P, plane 1 M)
-//   BF16 : t16[4][kpad / 8][apad][8]     (planes P_hi, P_lo, M_hi, M_lo)
-// Zero outside k < nmax_cap, j < n_ang.
+// P = pi + tau and M = pi - tau from the FP64 tables [k][angle] (k < nmax_cap) as
+// BF16 terms t16[4][kpad / 8][apad][8] (planes P_hi, P_lo, M_hi, M_lo), zero
+// outside k < nmax_cap, j < n_ang.
 __global__ void k_s12_prep_tables(int n_ang, int nmax_cap, int kpad, int apad,
                                   const double* __restrict__ pi_t,
-                                  const double* __restrict__ tau_t, int precision,
-                                  float* __restrict__ t32, unsigned short* __restrict__ t16) {
+                                  const double* __restrict__ tau_t,
+                                  unsigned short* __restrict__ t16) {
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= (int64_t)kpad * apad) return;
   const int k = (int)(idx / apad), j = (int)(idx % apad);
@@ -513,20 +675,15 @@ __global__ void k_s12_prep_tables(int n_ang, int nmax_cap, int kpad, int apad,
     P = pv + tv;
     M = pv - tv;
   }
-  if (precision == GM_PREC_FP32) {
-    t32[(size_t)k * apad + j] = (float)P;
-    t32[((size_t)kpad + k) * apad + j] = (float)M;
-  } else {
-    const size_t plane = (size_t)kpad * apad;
-    const size_t o = ((size_t)(k >> 3) * apad + j) * 8 + (k & 7);
-    unsigned short h, l;
-    bf16_split(P, h, l);
-    t16[o] = h;
-    t16[plane + o] = l;
-    bf16_split(M, h, l);
-    t16[2 * plane + o] = h;
-    t16[3 * plane + o] = l;
-  }
+  const size_t plane = (size_t)kpad * apad;
+  const size_t o = ((size_t)(k >> 3) * apad + j) * 8 + (k & 7);
+  unsigned short h, l;
+  bf16_split(P, h, l);
+  t16[o] = h;
+  t16[plane + o] = l;
+  bf16_split(M, h, l);
+  t16[2 * plane + o] = h;
+  t16[3 * plane + o] = l;
 }
 
 // K extent of the tile of 8 points starting at p0, rounded up to a whole step.
@@ -539,78 +696,6 @@ __device__ __forceinline__ int tile_kmax(int64_t n, int64_t p0, const int32_t* _
   }
   kmax = min(kmax, nmax_cap);
   return (kmax + step - 1) / step * step;
-}
-
-__global__ __launch_bounds__(256) void k_s12_f32(
-    int64_t n, const int64_t* __restrict__ off, const int32_t* __restrict__ nmax,
-    const double* __restrict__ an, const double* __restrict__ bn, int n_ang, int apad, int kpad,
-    const float* __restrict__ t32, int nmax_cap, int mode, double* __restrict__ out0,
-    double* __restrict__ out1) {
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int64_t p0 = (int64_t)blockIdx.x * 8;
-  const int j0 = (blockIdx.y * (blockDim.x >> 6) + wave) * 64;  // 64 angles per wavefront
-  if (j0 >= n_ang) return;
-  const int i = lane & 15, kq = lane >> 4;
-  const int64_t pa = p0 + (i >> 1);
-  const int comp = i & 1;
-  const bool pa_ok = pa < n;
-  const int nm_a = pa_ok ? nmax[pa] : 0;
-  const int64_t oa = pa_ok ? off[pa] : 0;
-  const int kmax = tile_kmax(n, p0, nmax, nmax_cap, 4);
-  const float* Pt = t32;
-  const float* Mt = t32 + (size_t)kpad * apad;
-  float4_ accp[4], accm[4];
-  for (int t = 0; t < 4; ++t) {
-    accp[t] = (float4_){0.f, 0.f, 0.f, 0.f};
-    accm[t] = (float4_){0.f, 0.f, 0.f, 0.f};
-  }
-  // register double buffer: step k0 + 4's operands load during step k0's MFMAs
-  double ar_n = 0.0, br_n = 0.0;
-  float p_n[4], m_n[4];
-  auto load_step = [&](int k0) {
-    const int kk = k0 + kq;
-    ar_n = 0.0;
-    br_n = 0.0;
-    if (kk < nm_a) {
-      ar_n = an[2 * (oa + kk) + comp];
-      br_n = bn[2 * (oa + kk) + comp];
-    }
-    const size_t row = (size_t)kk * apad + j0 + i;   // rows < kpad: zero padded
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      p_n[t] = Pt[row + 16 * t];
-      m_n[t] = Mt[row + 16 * t];
-    }
-  };
-  if (kmax > 0) load_step(0);
-  for (int k0 = 0; k0 < kmax; k0 += 4) {
-    const float ua = (float)(ar_n + br_n), va = (float)(ar_n - br_n);
-    float P[4], M[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      P[t] = p_n[t];
-      M[t] = m_n[t];
-    }
-    if (k0 + 4 < kmax) load_step(k0 + 4);
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      accp[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(ua, P[t], accp[t], 0, 0, 0);
-      accm[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(va, M[t], accm[t], 0, 0, 0);
-    }
-  }
-#pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int j = j0 + t * 16 + i;
-    if (j >= n_ang) continue;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int64_t p = p0 + 2 * kq + h;
-      if (p >= n) continue;
-      s12_store(mode, p, j, n_ang, cd{(double)accp[t][2 * h], (double)accp[t][2 * h + 1]},
-                cd{(double)accm[t][2 * h], (double)accm[t][2 * h + 1]}, out0, out1);
-    }
-  }
 }
 
 __global__ __launch_bounds__(256) void k_s12_bf16x3(
@@ -808,7 +893,7 @@ __device__ __forceinline__ void rows_lp_epilogue(const float4_ (&accp)[MT][4],
 // angle-table word fetched feeds the products of all MT tiles, and the row
 // sums are formed once, after the K loop, so they hold no registers while
 // it runs.
-template <int PREC, int MT, int RM>
+template <int MT, int RM>
 __global__ __launch_bounds__(64 * kRowsWaves) void k_s12_rows_lp(
     RowGroups g, const int64_t* __restrict__ off, const int32_t* __restrict__ nmax,
     const uint4* __restrict__ coef, int n_ang, int apad, int kpad, const void* __restrict__ tab,
@@ -826,7 +911,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_s12_rows_lp(
   const int i = lane & 15;
   const int kq = lane >> 4;
   const int comp = i & 1;   // A row i of tile mt: point p0 + 8 mt + (i >> 1), component i & 1
-  constexpr int kStep = PREC == GM_PREC_FP32 ? 4 : kLpK;
+  constexpr int kStep = kLpK;
   int nm_a[MT];
   int64_t oa[MT];
 #pragma unroll
@@ -848,47 +933,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void k_s12_rows_lp(
       accp[mt][t] = (float4_){0.f, 0.f, 0.f, 0.f};
       accm[mt][t] = (float4_){0.f, 0.f, 0.f, 0.f};
     }
-  if constexpr (PREC == GM_PREC_FP32) {
-    const float2* cf = (const float2*)coef;
-    const float* Pt = (const float*)tab;
-    const float* Mt = Pt + (size_t)kpad * apad;
-    float2 uv_n[MT];
-    float p_n[4], m_n[4];
-    auto load_step = [&](int k0) {
-      const int kk = k0 + kq;
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-        uv_n[mt] = kk < nm_a[mt] ? cf[2 * (oa[mt] + kk) + comp] : make_float2(0.f, 0.f);
-      const size_t row = (size_t)kk * apad + j0 + i;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        p_n[t] = Pt[row + 16 * t];
-        m_n[t] = Mt[row + 16 * t];
-      }
-    };
-    if (kmax > 0) load_step(0);
-    for (int k0 = 0; k0 < kmax; k0 += 4) {
-      float ua[MT], va[MT], P[4], M[4];
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        ua[mt] = uv_n[mt].x;
-        va[mt] = uv_n[mt].y;
-      }
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        P[t] = p_n[t];
-        M[t] = m_n[t];
-      }
-      if (k0 + 4 < kmax) load_step(k0 + 4);
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          accp[mt][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(ua[mt], P[t], accp[mt][t], 0, 0, 0);
-          accm[mt][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[mt], M[t], accm[mt][t], 0, 0, 0);
-        }
-    }
-  } else {
+  {
     const uint2* cb = (const uint2*)coef;
     const uint4* tb = (const uint4*)tab;   // 8 BF16 (one K-octet) per uint4
     const size_t plane4 = (size_t)kpad * apad / 8;
@@ -1132,6 +1177,10 @@ namespace {
 // table rows from which units are sorted by length (1.2M points, n_max to 3400:
 // 11.60 against 11.86 ms; 20k points, n_max to 449: 178 us against 168 unsorted).
 constexpr int64_t kS12Want = 8192;
+// FP32: up to 128 angles per wavefront where a and b are read as FP64 (1.5M points x
+// 371 angles 10.49 against 11.03 ms at 64; 60k points, 11k wavefronts, 1.97 against
+// 1.87), 64 where they come converted (40k x 1801 1.73 against 1.75 ms at 128).
+constexpr int64_t kS12Want32 = 16384;
 constexpr int64_t kS12PairTiles = 256;
 constexpr int kS12SortRows = 512;
 
@@ -1154,6 +1203,19 @@ S12Shape s12_shape(int64_t tiles, int n_ang, int64_t want, int max_tt = 4) {
   return h;
 }
 
+// FP32: 32, 64 or 128 angles per wavefront, always on the paired tables.
+S12Shape s12_shape32(int64_t tiles, int n_ang, int max_tt) {
+  S12Shape h = s12_shape(tiles, n_ang, kS12Want32, max_tt);
+  if (h.tt < 2) {
+    h.tt = 2;
+    const int waves = (n_ang + 31) / 32;
+    h.ablocks = (waves + 3) / 4;
+    h.wpb = (waves + h.ablocks - 1) / h.ablocks;
+  }
+  h.raw = false;
+  return h;
+}
+
 dim3 s12_grid(int64_t blocks) {
   return dim3((unsigned)std::min<int64_t>(blocks, gm::kGridRow),
               (unsigned)((blocks + gm::kGridRow - 1) / gm::kGridRow));
@@ -1162,21 +1224,23 @@ dim3 s12_grid(int64_t blocks) {
 // The (P, M) pairs, and the launch order of `units` units of unit_pts points
 // (*order, NULL where the series are too short or the units too few for a long
 // unit at the end to matter: sorting costs two launches, about 10 us).
-int s12_pairs(gm_ctx* ctx, const S12Shape& h, int n_ang, const double* pi_t, const double* tau_t,
-              int nmax_cap, gm::S12Tables& T, const gm::RowGroups& g, int unit_pts, int64_t units,
+int s12_pairs(gm_ctx* ctx, int precision, const S12Shape& h, int n_ang, const double* pi_t,
+              const double* tau_t, int nmax_cap, gm::S12Tables& T, const gm::RowGroups& g, int unit_pts, int64_t units,
               int64_t n, const int32_t* nmax, const int** order, hipStream_t s) {
   *order = nullptr;
   T.pi_t = pi_t;
   T.tau_t = tau_t;
   T.tab = nullptr;
+  T.tab32 = nullptr;
   T.n_ang = n_ang;
-  T.apad = (n_ang + 63) / 64 * 64;
+  T.apad = (n_ang + 127) / 128 * 128;
   T.nmax_cap = nmax_cap;
   if (h.raw) return GM_OK;
   const int64_t total = (int64_t)((nmax_cap + 3) / 4 * 4) * T.apad;
   const bool sorted = nmax_cap >= kS12SortRows && units >= 1024 && units <= 0x7fffffffLL;
   // pairs, then (sorted) the histogram and its cursors, the order and the bins
-  const size_t o_hist = (size_t)total * sizeof(double2);
+  const bool f64 = precision == GM_PREC_FP64;
+  const size_t o_hist = (size_t)total * (f64 ? sizeof(double2) : sizeof(float2));
   const size_t o_ord = o_hist + 2 * gm::kUnitBins * sizeof(int);
   const size_t o_bin = o_ord + (size_t)units * sizeof(int);
   int rc = ctx->reserve(ctx->tab_lp, sorted ? o_bin + (size_t)units : o_hist);
@@ -1184,8 +1248,14 @@ int s12_pairs(gm_ctx* ctx, const S12Shape& h, int n_ang, const double* pi_t, con
   char* ws = (char*)ctx->tab_lp.ptr;
   int* hist = sorted ? (int*)(ws + o_hist) : nullptr;
   T.tab = (const double2*)ws;
-  hipLaunchKernelGGL(gm::k_s12_prep_pairs, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s,
-                     n_ang, nmax_cap, T.apad, total, pi_t, tau_t, (double2*)ws, hist);
+  T.tab32 = (const float2*)ws;
+  const dim3 gp((unsigned)((total + 255) / 256));
+  if (f64)
+    hipLaunchKernelGGL(gm::k_s12_prep_pairs, gp, dim3(256), 0, s, n_ang, nmax_cap, T.apad, total,
+                       pi_t, tau_t, (double2*)ws, hist);
+  else
+    hipLaunchKernelGGL(gm::k_s12_prep_pairs32, gp, dim3(256), 0, s, n_ang, nmax_cap, T.apad, total,
+                       pi_t, tau_t, (float2*)ws, hist);
   if (sorted) {
     const dim3 gu((unsigned)((units + 255) / 256));
     hipLaunchKernelGGL(gm::k_s12_unit_bins, gu, dim3(256), 0, s, g, unit_pts, units, n, nmax,
@@ -1209,26 +1279,33 @@ int launch_s12(gm_ctx* ctx, const char* who, int64_t n, const int64_t* off, cons
   if (nmax_cap < 1) return gm_fail(GM_EINVAL, "%s: nmax_cap must be >= 1", who);
   hipError_t e = hipSetDevice(ctx->device);
   if (e != hipSuccess) return gm_fail(GM_ERUNTIME, "hipSetDevice: %s", hipGetErrorString(e));
-  const int wpb = ctx->tune_s12_waves;
-  dim3 grid((unsigned)((n + 7) / 8), (unsigned)((n_ang + 64 * wpb - 1) / (64 * wpb)));
-  dim3 block(64 * wpb);
   size_t slot;
-  if (precision == GM_PREC_FP64) {
+  if (precision != GM_PREC_BF16X3) {
     ctx->mark_begin(gm::kKS12, s, &slot);
-    const S12Shape h = s12_shape((n + 15) / 16, n_ang, kS12Want);
+    const int64_t units = (n + 15) / 16;
+    const S12Shape h = precision == GM_PREC_FP64 ? s12_shape(units, n_ang, kS12Want)
+                                                 : s12_shape32(units, n_ang, 8);
     gm::S12Tables T;
     const int* order;
     gm::RowGroups none{};
-    const int rc = s12_pairs(ctx, h, n_ang, pi_t, tau_t, nmax_cap, T, none, 16, (n + 15) / 16, n,
+    const int rc = s12_pairs(ctx, precision, h, n_ang, pi_t, tau_t, nmax_cap, T, none, 16, units, n,
                              nmax, &order, s);
     if (rc) return rc;
-    const dim3 g = s12_grid((n + 15) / 16 * h.ablocks);
-#define GM_TILES(T_, R_)                                                                       \
-  hipLaunchKernelGGL((gm::k_s12_tiles<T_, R_>), g, dim3(64 * h.wpb), 0, s, T, n, off, nmax, an, \
-                     bn, mode, out0, out1, h.ablocks, order)
-    if (h.tt == 4) { if (h.raw) GM_TILES(4, true); else GM_TILES(4, false); }
-    else if (h.tt == 2) { if (h.raw) GM_TILES(2, true); else GM_TILES(2, false); }
-    else { if (h.raw) GM_TILES(1, true); else GM_TILES(1, false); }
+    const dim3 g = s12_grid(units * h.ablocks);
+#define GM_TILES(...)                                                                          \
+  hipLaunchKernelGGL((gm::__VA_ARGS__), g, dim3(64 * h.wpb), 0, s, T, n, off, nmax, an, bn, mode, \
+                     out0, out1, h.ablocks, order)
+    if (precision == GM_PREC_FP32) {
+      if (h.tt == 8) GM_TILES(k_s12_tiles32<8>);
+      else if (h.tt == 4) GM_TILES(k_s12_tiles32<4>);
+      else GM_TILES(k_s12_tiles32<2>);
+    } else if (h.tt == 4) {
+      if (h.raw) GM_TILES(k_s12_tiles<4, true>); else GM_TILES(k_s12_tiles<4, false>);
+    } else if (h.tt == 2) {
+      if (h.raw) GM_TILES(k_s12_tiles<2, true>); else GM_TILES(k_s12_tiles<2, false>);
+    } else {
+      if (h.raw) GM_TILES(k_s12_tiles<1, true>); else GM_TILES(k_s12_tiles<1, false>);
+    }
 #undef GM_TILES
     ctx->mark_end(slot, s);
   } else {
@@ -1236,21 +1313,17 @@ int launch_s12(gm_ctx* ctx, const char* who, int64_t n, const int64_t* off, cons
     // whole 256-angle blocks: every wavefront with j0 < n_ang reads 64 padded columns
     const int apad = (n_ang + 255) / 256 * 256;
     const size_t elems = (size_t)kpad * apad;
-    const size_t bytes = precision == GM_PREC_FP32 ? 2 * elems * sizeof(float)
-                                                   : 4 * elems * sizeof(unsigned short);
-    int rc = ctx->reserve(ctx->tab_lp, bytes);
+    int rc = ctx->reserve(ctx->tab_lp, 4 * elems * sizeof(unsigned short));
     if (rc) return rc;
-    float* t32 = (float*)ctx->tab_lp.ptr;
     unsigned short* t16 = (unsigned short*)ctx->tab_lp.ptr;
     hipLaunchKernelGGL(gm::k_s12_prep_tables, dim3((unsigned)((elems + 255) / 256)), dim3(256), 0,
-                       s, n_ang, nmax_cap, kpad, apad, pi_t, tau_t, precision, t32, t16);
+                       s, n_ang, nmax_cap, kpad, apad, pi_t, tau_t, t16);
+    const int wpb = ctx->tune_s12_waves;
     ctx->mark_begin(gm::kKS12, s, &slot);
-    if (precision == GM_PREC_FP32)
-      hipLaunchKernelGGL(gm::k_s12_f32, grid, block, 0, s, n, off, nmax, an, bn, n_ang, apad,
-                         kpad, (const float*)t32, nmax_cap, mode, out0, out1);
-    else
-      hipLaunchKernelGGL(gm::k_s12_bf16x3, grid, block, 0, s, n, off, nmax, an, bn, n_ang,
-                         apad, kpad, (const unsigned short*)t16, nmax_cap, mode, out0, out1);
+    hipLaunchKernelGGL(gm::k_s12_bf16x3,
+                       dim3((unsigned)((n + 7) / 8), (unsigned)((n_ang + 64 * wpb - 1) / (64 * wpb))),
+                       dim3(64 * wpb), 0, s, n, off, nmax, an, bn, n_ang, apad, kpad,
+                       (const unsigned short*)t16, nmax_cap, mode, out0, out1);
     ctx->mark_end(slot, s);
   }
   e = hipGetLastError();
@@ -1331,16 +1404,17 @@ int gm_s12_contract_rows(gm_ctx* ctx, int64_t n, const int64_t* coef_off, const 
   for (int r = 0; r < n_rows; ++r)
     if (count_host[r] > 0) tiles += (count_host[r] + 7) / 8;
   const int64_t ablocks = (n_ang + 64 * gm::kRowsWaves - 1) / (64 * gm::kRowsWaves);
-  // FP32 and split-BF16: 8-point tiles multiplied together per chunk, two when that
-  // still leaves >= 8k wavefronts.
+  // Split-BF16: 8-point tiles multiplied together per chunk, two when that still
+  // leaves >= 8k wavefronts.
   const int64_t waves2 = (tiles / 2) * ablocks * gm::kRowsWaves;
   const int row_tiles = ctx->tune_s12_row_tiles ? ctx->tune_s12_row_tiles : (waves2 >= 8192 ? 2 : 1);
-  // FP64: 16-point tiles; for short series several one after the other (fewer
+  // FP64 and FP32: 16-point tiles; for short series several one after the other (fewer
   // partial sums) while that leaves work for the whole chip
   bool many = false;   // a group of several rows
   for (int r = 1; r < n_rows; ++r)
     many |= start_host[r] == start_host[r - 1] && count_host[r] == count_host[r - 1];
-  S12Shape h64 = s12_shape((tiles + 1) / 2, n_ang, kS12Want);
+  S12Shape h64 = precision == GM_PREC_FP64 ? s12_shape((tiles + 1) / 2, n_ang, kS12Want)
+                                           : s12_shape32((tiles + 1) / 2, n_ang, 4);
   int64_t per = 1;
   while (per < 8 && nmax_cap <= 256 &&
          (tiles / 2) / (2 * per) * h64.ablocks * h64.wpb >= 2 * kS12Want)
@@ -1350,7 +1424,7 @@ int gm_s12_contract_rows(gm_ctx* ctx, int64_t n, const int64_t* coef_off, const 
     h64 = s12_shape(tiles, n_ang, 0, many ? 2 : 4);
     h64.raw = false;
   }
-  const int chunk_pts = precision == GM_PREC_FP64 ? (int)(16 * per) : 8 * row_tiles;
+  const int chunk_pts = precision != GM_PREC_BF16X3 ? (int)(16 * per) : 8 * row_tiles;
   gm::RowGroups g;
   g.n_groups = 0;
   g.chunk0[0] = 0;
@@ -1390,56 +1464,60 @@ int gm_s12_contract_rows(gm_ctx* ctx, int64_t n, const int64_t* coef_off, const 
   const dim3 rgrid((unsigned)((int64_t)n_rows * ((4 * (int64_t)n_ang + 63) / 64)));
   const dim3 rblock(64 * gm::kReduceWaves);
   size_t slot;
-  if (precision == GM_PREC_FP64) {
+  if (precision != GM_PREC_BF16X3) {
     ctx->mark_begin(gm::kKS12, s, &slot);
     gm::S12Tables T;
     const int* order;
-    if ((rc = s12_pairs(ctx, h64, n_ang, pi_t, tau_t, nmax_cap, T, g, chunk_pts, chunks, n, nmax,
+    const float4* cf = (const float4*)coef_lp;
+    if ((rc = s12_pairs(ctx, precision, h64, n_ang, pi_t, tau_t, nmax_cap, T, g, chunk_pts, chunks, n, nmax,
                         &order, s)))
       return rc;
     const dim3 g64 = s12_grid(chunks * h64.ablocks);
-#define GM_ROWS_F64(R_, T_, W_, M_)                                                              \
-  hipLaunchKernelGGL((gm::k_s12_rows_f64<R_, T_, W_, M_>), g64, dim3(64 * h64.wpb), 0, s, g,        \
-                     chunk_pts, T, coef_off, nmax, an, bn, w, n, part, h64.ablocks, order)
-#define GM_ROWS_F64_T(R_)                                                                      \
-  if (per > 1) GM_ROWS_F64(R_, (R_ == 1 ? 4 : 2), false, true);                                 \
-  else if (h64.tt == 4 && h64.raw) GM_ROWS_F64(R_, 4, true, false);                             \
-  else if (h64.tt == 4) GM_ROWS_F64(R_, 4, false, false);                                       \
-  else if (h64.tt == 2 && h64.raw) GM_ROWS_F64(R_, 2, true, false);                             \
-  else if (h64.tt == 2) GM_ROWS_F64(R_, 2, false, false);                                       \
-  else if (h64.raw) GM_ROWS_F64(R_, 1, true, false);                                            \
-  else GM_ROWS_F64(R_, 1, false, false);
-    if (RM == 1) { GM_ROWS_F64_T(1) } else if (RM == 2) { GM_ROWS_F64_T(2) } else { GM_ROWS_F64_T(4) }
-#undef GM_ROWS_F64_T
+#define GM_ROWS(P_, R_, T_, W_, M_)                                                            \
+  hipLaunchKernelGGL((gm::k_s12_rows<P_, R_, T_, W_, M_>), g64, dim3(64 * h64.wpb), 0, s, g,     \
+                     chunk_pts, T, coef_off, nmax, an, bn, cf, w, n, part, h64.ablocks, order)
+#define GM_ROWS_F64(R_)                                                                        \
+  if (per > 1) GM_ROWS(GM_PREC_FP64, R_, (R_ == 1 ? 4 : 2), false, true);                       \
+  else if (h64.tt == 4 && h64.raw) GM_ROWS(GM_PREC_FP64, R_, 4, true, false);                   \
+  else if (h64.tt == 4) GM_ROWS(GM_PREC_FP64, R_, 4, false, false);                             \
+  else if (h64.tt == 2 && h64.raw) GM_ROWS(GM_PREC_FP64, R_, 2, true, false);                   \
+  else if (h64.tt == 2) GM_ROWS(GM_PREC_FP64, R_, 2, false, false);                             \
+  else if (h64.raw) GM_ROWS(GM_PREC_FP64, R_, 1, true, false);                                  \
+  else GM_ROWS(GM_PREC_FP64, R_, 1, false, false);
+#define GM_ROWS_F32(R_)                                                                        \
+  if (per > 1) GM_ROWS(GM_PREC_FP32, R_, (R_ == 1 ? 4 : 2), false, true);                       \
+  else if (h64.tt == 4) GM_ROWS(GM_PREC_FP32, R_, 4, false, false);                             \
+  else GM_ROWS(GM_PREC_FP32, R_, 2, false, false);
+    if (precision == GM_PREC_FP64) {
+      if (RM == 1) { GM_ROWS_F64(1) } else if (RM == 2) { GM_ROWS_F64(2) } else { GM_ROWS_F64(4) }
+    } else {
+      if (RM == 1) { GM_ROWS_F32(1) } else if (RM == 2) { GM_ROWS_F32(2) } else { GM_ROWS_F32(4) }
+    }
+#undef GM_ROWS_F32
 #undef GM_ROWS_F64
+#undef GM_ROWS
     ctx->mark_end(slot, s);
   } else {
     // P, M tables of this precision (padded to whole K-steps and 256 angles)
     const int kpad = (nmax_cap + gm::kLpK - 1) / gm::kLpK * gm::kLpK;
     const int apad = (n_ang + 255) / 256 * 256;
     const size_t elems = (size_t)kpad * apad;
-    const size_t bytes = precision == GM_PREC_FP32 ? 2 * elems * sizeof(float)
-                                                   : 4 * elems * sizeof(unsigned short);
-    rc = ctx->reserve(ctx->tab_lp, bytes);
+    rc = ctx->reserve(ctx->tab_lp, 4 * elems * sizeof(unsigned short));
     if (rc) return rc;
     ctx->mark_begin(gm::kKS12, s, &slot);
     hipLaunchKernelGGL(gm::k_s12_prep_tables, dim3((unsigned)((elems + 255) / 256)), dim3(256), 0,
-                       s, n_ang, nmax_cap, kpad, apad, pi_t, tau_t, precision,
-                       (float*)ctx->tab_lp.ptr, (unsigned short*)ctx->tab_lp.ptr);
+                       s, n_ang, nmax_cap, kpad, apad, pi_t, tau_t,
+                       (unsigned short*)ctx->tab_lp.ptr);
     const uint4* cf = (const uint4*)coef_lp;
     const void* tb = ctx->tab_lp.ptr;
-#define GM_ROWS_LP(P_, M_, R_)                                                                \
-  hipLaunchKernelGGL((gm::k_s12_rows_lp<P_, M_, R_>), grid, block, 0, s, g, coef_off, nmax, cf,  \
+#define GM_ROWS_LP(M_, R_)                                                                   \
+  hipLaunchKernelGGL((gm::k_s12_rows_lp<M_, R_>), grid, block, 0, s, g, coef_off, nmax, cf,  \
                      n_ang, apad, kpad, tb, nmax_cap, w, n, part)
-#define GM_ROWS_LP_RM(P_, M_)        \
-  if (RM == 1) GM_ROWS_LP(P_, M_, 1); \
-  else if (RM == 2) GM_ROWS_LP(P_, M_, 2); \
-  else GM_ROWS_LP(P_, M_, 4)
-    if (precision == GM_PREC_FP32) {
-      if (row_tiles == 4) { GM_ROWS_LP_RM(GM_PREC_FP32, 4); }
-      else if (row_tiles == 2) { GM_ROWS_LP_RM(GM_PREC_FP32, 2); }
-      else { GM_ROWS_LP_RM(GM_PREC_FP32, 1); }
-    } else if (ctx->tune_s12_share && row_tiles == 1) {
+#define GM_ROWS_LP_RM(M_)        \
+  if (RM == 1) GM_ROWS_LP(M_, 1); \
+  else if (RM == 2) GM_ROWS_LP(M_, 2); \
+  else GM_ROWS_LP(M_, 4)
+    if (ctx->tune_s12_share && row_tiles == 1) {
       // kShChunks work units per block share the angle-table tiles (LDS)
       const dim3 sgrid((unsigned)((chunks + gm::kShChunks - 1) / gm::kShChunks),
                        (unsigned)((n_ang + 63) / 64));
@@ -1454,9 +1532,9 @@ int gm_s12_contract_rows(gm_ctx* ctx, int64_t n, const int64_t* coef_off, const 
 #undef GM_ROWS_SH_RM
 #undef GM_ROWS_SH
     } else {
-      if (row_tiles == 4) { GM_ROWS_LP_RM(GM_PREC_BF16X3, 4); }
-      else if (row_tiles == 2) { GM_ROWS_LP_RM(GM_PREC_BF16X3, 2); }
-      else { GM_ROWS_LP_RM(GM_PREC_BF16X3, 1); }
+      if (row_tiles == 4) { GM_ROWS_LP_RM(4); }
+      else if (row_tiles == 2) { GM_ROWS_LP_RM(2); }
+      else { GM_ROWS_LP_RM(1); }
     }
 #undef GM_ROWS_LP_RM
 #undef GM_ROWS_LP
