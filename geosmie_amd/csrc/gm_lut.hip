@@ -51,75 +51,107 @@ __global__ void k_lut_points(int64_t n_slab, int n_r, const double* __restrict__
 //   [PSD rows x n_r radii] x [n_r x (n_ang + 4) columns]
 // on the FP64 matrix cores (v_mfma_f64_16x16x4_f64: A[i][k] from lane
 // i + 16k, B[k][j] from lane j + 16k, D[g + 4r][j] in lane j + 16g element r).
-// One wavefront per (slab, 64 columns, 48 PSD rows): three 16-row tiles x four
+// One wavefront per (slab, 64 columns, 16 RT PSD rows): RT 16-row tiles x four
 // 16-column tiles, walking the radii four at a time; every plane element is
 // read once, the weights (shared by the slabs) come from the cache, and each
-// sum is formed in one fixed order.
+// sum is formed in one fixed order.  Bound by the planes' bytes; operands are
+// loaded kLutAhead steps ahead (2; 3 to 8 at fewer wavefronts per SIMD were
+// slower) and RT = 1 where 16 rows are enough.  400 slabs x 40 PSDs (3.6 GB of
+// planes) 2.16 -> 1.76 ms, 512 slabs x 1 PSD (4.6 GB) 2.14 -> 1.52 ms.
 typedef double double4_ __attribute__((ext_vector_type(4)));
-constexpr int kLutRowTiles = 3;   // 48 PSD rows per wavefront
-__global__ __launch_bounds__(64) void k_lut_contract(
+constexpr int kLutAhead = 2;
+
+// wt[p][k] = w[k][p], k < ldt (zero past n_psd).
+__global__ __launch_bounds__(256) void k_lut_transpose(int n_r, int n_psd, int ldt,
+                                                       const double* __restrict__ w,
+                                                       double* __restrict__ wt) {
+  const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (id >= (int64_t)n_r * ldt) return;
+  const int p = (int)(id / ldt), k = (int)(id - (int64_t)p * ldt);
+  wt[id] = k < n_psd ? w[(size_t)k * n_r + p] : 0.0;
+}
+
+// Weight of PSD k at radius p: w[slab stride + k sk + p sp].
+template <int RT>
+__global__ __launch_bounds__(64, 3) void k_lut_contract(
     int64_t n_slab, int n_r, int n_ang, int n_psd, const double* __restrict__ w,
-    int64_t w_slab_stride, const double* __restrict__ x, const double* __restrict__ lam,
+    int64_t w_slab_stride, int64_t sk, int64_t sp, const double* __restrict__ x, const double* __restrict__ lam,
     const double* __restrict__ props, const double* __restrict__ p11, double* __restrict__ sums) {
   const int ncol = n_ang + kLutFeat;
   const int ncb = (ncol + 63) / 64;
-  const int64_t s = blockIdx.x / ncb;
-  const int c0 = (int)(blockIdx.x - s * ncb) * 64;
-  const int k0 = blockIdx.y * 16 * kLutRowTiles;
+  // all column blocks of a slab on one XCD (blocks go to the eight in turn): the
+  // lines at their edges, which rows of 8 n_ang bytes do not end on, are fetched once
+  const int64_t turn = blockIdx.x >> 3;
+  const int64_t s = turn / ncb * 8 + (blockIdx.x & 7);
+  if (s >= n_slab) return;
+  const int c0 = (int)(turn % ncb) * 64;
+  const int k0 = blockIdx.y * 16 * RT;
   const int lane = threadIdx.x;
   const int i = lane & 15, kq = lane >> 4;
   const int64_t n_all = n_slab * n_r;
   const double* wb = w + s * w_slab_stride;
   const double rscale = lam[s] / (2.0 * 3.14159265358979323846);
-  double4_ acc[kLutRowTiles][4];
+  double4_ acc[RT][4];
 #pragma unroll
-  for (int mt = 0; mt < kLutRowTiles; ++mt)
+  for (int mt = 0; mt < RT; ++mt)
 #pragma unroll
     for (int t = 0; t < 4; ++t) acc[mt][t] = (double4_){0.0, 0.0, 0.0, 0.0};
   // operands of radius p = p0 + kq: the weight of PSD k0 + 16 mt + i and the
-  // column c0 + 16 t + i (a P11 value or, past n_ang, a feature of point p)
-  auto load = [&](int p0, double* a, double* bv) {
-    const int p = p0 + kq;
-    const bool pok = p < n_r;
+  // column c0 + 16 t + i (a P11 value or, past n_ang, a feature of point p).
+  // Radii past the end repeat the last one with weight 0; rows and columns past
+  // the end repeat the last one (not written).
+  const double* wrow[RT];
 #pragma unroll
-    for (int mt = 0; mt < kLutRowTiles; ++mt) {
-      const int k = k0 + 16 * mt + i;
-      a[mt] = (pok && k < n_psd) ? wb[(size_t)k * n_r + p] : 0.0;
-    }
-    const int64_t pt = s * n_r + p;
+  for (int mt = 0; mt < RT; ++mt) wrow[mt] = wb + min(k0 + 16 * mt + i, n_psd - 1) * sk;
+  const bool plain = c0 + 64 <= n_ang;   // no feature column in this wavefront
+  const double* plane = p11 + s * n_r * (int64_t)n_ang;
+  int col[4];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int c = c0 + 16 * t + i;
-      double v = 0.0;
-      if (pok && c < n_ang) {
-        v = p11[pt * n_ang + c];
-      } else if (pok && c < ncol) {
-        const double r = x[pt] * rscale, r2 = r * r;
-        const int f = c - n_ang;
-        const double qext = props[pt], qsca = props[n_all + pt], g = props[4 * n_all + pt];
-        v = f == 0 ? r2 : (f == 1 ? qext * r2 : (f == 2 ? qsca * r2 : g * qsca * r2));
+  for (int t = 0; t < 4; ++t) col[t] = min(c0 + 16 * t + i, n_ang - 1);
+  double a_n[kLutAhead][RT], b_n[kLutAhead][4];
+  auto load = [&](int p0, double (&a)[RT], double (&bv)[4]) {
+    const int p = p0 + kq, pc = min(p, n_r - 1);
+    const double* row = plane + (int64_t)pc * n_ang;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) bv[t] = row[col[t]];
+#pragma unroll
+    for (int mt = 0; mt < RT; ++mt) a[mt] = wrow[mt][pc * sp];
+    if (!plain) {
+      const int64_t pt = s * n_r + pc;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int f = c0 + 16 * t + i - n_ang;
+        if (f >= 0 && f < kLutFeat) {
+          const double r = x[pt] * rscale, r2 = r * r;
+          const double qext = props[pt], qsca = props[n_all + pt], g = props[4 * n_all + pt];
+          bv[t] = f == 0 ? r2 : (f == 1 ? qext * r2 : (f == 2 ? qsca * r2 : g * qsca * r2));
+        }
       }
-      bv[t] = v;
     }
   };
-  double a_n[kLutRowTiles], b_n[4];
-  load(0, a_n, b_n);
-  for (int p0 = 0; p0 < n_r; p0 += 4) {
-    double a_c[kLutRowTiles], b_c[4];
 #pragma unroll
-    for (int mt = 0; mt < kLutRowTiles; ++mt) a_c[mt] = a_n[mt];
+  for (int q = 0; q < kLutAhead; ++q) load(4 * q, a_n[q], b_n[q]);
+  for (int pb = 0; pb < n_r; pb += 4 * kLutAhead) {
 #pragma unroll
-    for (int t = 0; t < 4; ++t) b_c[t] = b_n[t];
-    if (p0 + 4 < n_r) load(p0 + 4, a_n, b_n);
+    for (int q = 0; q < kLutAhead; ++q) {
+      const int p0 = pb + 4 * q;
+      if (p0 >= n_r) break;
+      double a_c[RT], b_c[4];
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+      for (int mt = 0; mt < RT; ++mt) a_c[mt] = p0 + kq < n_r ? a_n[q][mt] : 0.0;
 #pragma unroll
-      for (int mt = 0; mt < kLutRowTiles; ++mt)
-        acc[mt][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a_c[mt], b_c[t], acc[mt][t], 0, 0, 0);
+      for (int t = 0; t < 4; ++t) b_c[t] = b_n[q][t];
+      load(p0 + 4 * kLutAhead, a_n[q], b_n[q]);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int mt = 0; mt < RT; ++mt)
+          acc[mt][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a_c[mt], b_c[t], acc[mt][t], 0, 0, 0);
+    }
   }
   // lane (i, kq) element r of acc[mt][t]: PSD k0 + 16 mt + kq + 4 r, column c0 + 16 t + i
 #pragma unroll
-  for (int mt = 0; mt < kLutRowTiles; ++mt)
+  for (int mt = 0; mt < RT; ++mt)
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const int c = c0 + 16 * t + i;
@@ -131,27 +163,49 @@ __global__ __launch_bounds__(64) void k_lut_contract(
     }
 }
 
-// One wavefront per entry: lane l forms alpha1_l from the GSF table G1[a][l].
-__global__ __launch_bounds__(64) void k_lut_finish(int n_ang, int ng, int n_mom,
+// Lane l forms alpha1_l of kLutFinish entries from the GSF table G1[a][l] (two
+// groups of entries per wavefront where 32 lanes hold the moments): the table is
+// read from the L2 by every wavefront, so each word of it serves several entries.
+// 16000 entries x 371 angles x 32 moments: 222 us with one entry per wavefront.
+constexpr int kLutFinish = 4;
+__global__ __launch_bounds__(64) void k_lut_finish(int64_t n_ent, int n_ang, int ng, int n_mom,
                                                    const double* __restrict__ G1,
                                                    const double* __restrict__ sums,
                                                    float* __restrict__ out) {
-  const int64_t e = blockIdx.x;
-  const int l = threadIdx.x;
+  const int lane = threadIdx.x;
+  const bool halves = n_mom <= 32;
+  const int l = halves ? lane & 31 : lane;
+  const int64_t e0 =
+      ((int64_t)blockIdx.x * (halves ? 2 : 1) + (halves ? lane >> 5 : 0)) * kLutFinish;
   const int ncol = n_ang + kLutFeat;
-  const double* S = sums + e * ncol;
-  double acc = 0.0;
-  if (l < n_mom)
-    for (int a = 0; a < n_ang; ++a) acc = fma(G1[(size_t)a * ng + l], S[a], acc);
-  const double alpha = acc * ((double)l + 0.5);
-  const double a0 = __shfl(alpha, 0);
-  float* o = out + e * (3 + n_mom);
-  if (l < n_mom) o[3 + l] = (float)(alpha / a0);
-  if (l == 0) {
-    const double sr2 = S[n_ang], sext = S[n_ang + 1], ssca = S[n_ang + 2], sg = S[n_ang + 3];
-    o[0] = (float)(sext / sr2);
-    o[1] = (float)(ssca / sext);
-    o[2] = (float)(sg / ssca);
+  const double* S[kLutFinish];
+  double acc[kLutFinish];
+#pragma unroll
+  for (int q = 0; q < kLutFinish; ++q) {
+    S[q] = sums + min(e0 + q, n_ent - 1) * ncol;   // entries past the end repeat the last
+    acc[q] = 0.0;
+  }
+  const double* g = G1 + min(l, n_mom - 1);
+#pragma unroll 4
+  for (int a = 0; a < n_ang; ++a) {
+    const double w = g[(size_t)a * ng];
+#pragma unroll
+    for (int q = 0; q < kLutFinish; ++q) acc[q] = fma(w, S[q][a], acc[q]);
+  }
+#pragma unroll
+  for (int q = 0; q < kLutFinish; ++q) {
+    const double alpha = acc[q] * ((double)l + 0.5);
+    const double a0 = __shfl(alpha, halves ? lane & 32 : 0);
+    if (e0 + q >= n_ent) continue;
+    float* o = out + (e0 + q) * (3 + n_mom);
+    if (l < n_mom) o[3 + l] = (float)(alpha / a0);
+    if (l == 0) {
+      const double sr2 = S[q][n_ang], sext = S[q][n_ang + 1], ssca = S[q][n_ang + 2],
+                   sg = S[q][n_ang + 3];
+      o[0] = (float)(sext / sr2);
+      o[1] = (float)(ssca / sext);
+      o[2] = (float)(sg / ssca);
+    }
   }
 }
 
@@ -296,24 +350,45 @@ int gm_lut_bulk(gm_ctx* ctx, int64_t n_slab, int n_r, int n_ang, int n_psd, cons
       return gm_fail(GM_EINVAL, "gm_lut_bulk: angles must increase");
   const int64_t ncb = (n_ang + gm::kLutFeat + 63) / 64;
   const int64_t n_ent = n_slab * n_psd;
-  if (n_slab * ncb > 0x7fffffffLL || n_ent > 0x7fffffffLL)
+  if ((n_slab + 7) * ncb > 0x7fffffffLL || n_ent > 0x7fffffffLL)
     return gm_fail(GM_EINVAL, "gm_lut_bulk: too many slabs for one call");
   hipError_t e = hipSetDevice(ctx->device);
   if (e != hipSuccess) return gm_fail(GM_ERUNTIME, "hipSetDevice: %s", hipGetErrorString(e));
   hipStream_t s = (hipStream_t)stream;
   int rc = gm::gsf_tables(ctx, ng, n_ang, ang_deg_host, s);
   if (rc) return rc;
-  rc = ctx->reserve(ctx->lut_tmp, sizeof(double) * (size_t)n_ent * (n_ang + gm::kLutFeat));
+  // Weights shared by the slabs are transposed once: a step then reads 16 PSDs of
+  // one radius from one line instead of 16 lines, 32 bytes of each (48 rows and nine
+  // wavefronts per CU: more lines than the CU's cache holds)
+  const bool turn = !w_per_slab && n_psd > 1 && n_slab > 1;
+  const int ldt = (n_psd + 15) / 16 * 16;
+  const size_t n_sums = (size_t)n_ent * (n_ang + gm::kLutFeat);
+  rc = ctx->reserve(ctx->lut_tmp, sizeof(double) * (n_sums + (turn ? (size_t)n_r * ldt : 0)));
   if (rc) return rc;
   double* sums = (double*)ctx->lut_tmp.ptr;
+  const double* wc = w;
+  int64_t wss = w_per_slab ? (int64_t)n_psd * n_r : 0, sk = n_r, sp = 1;
+  if (turn) {
+    double* wt = sums + n_sums;
+    hipLaunchKernelGGL(gm::k_lut_transpose, dim3((unsigned)(((int64_t)n_r * ldt + 255) / 256)),
+                       dim3(256), 0, s, n_r, n_psd, ldt, w, wt);
+    wc = wt;
+    sk = 1;
+    sp = ldt;
+  }
   size_t slot;
   ctx->mark_begin(gm::kKLut, s, &slot);
-  hipLaunchKernelGGL(gm::k_lut_contract,
-                     dim3((unsigned)(n_slab * ncb),
-                          (unsigned)((n_psd + 16 * gm::kLutRowTiles - 1) / (16 * gm::kLutRowTiles))),
-                     dim3(64), 0, s, n_slab, n_r, n_ang, n_psd, w,
-                     w_per_slab ? (int64_t)n_psd * n_r : (int64_t)0, x, lam, props, p11, sums);
-  hipLaunchKernelGGL(gm::k_lut_finish, dim3((unsigned)n_ent), dim3(64), 0, s, n_ang, ng, n_mom,
+  const unsigned blocks = (unsigned)((n_slab + 7) / 8 * 8 * ncb);
+  if (n_psd <= 16)
+    hipLaunchKernelGGL(gm::k_lut_contract<1>, dim3(blocks, 1), dim3(64), 0, s,
+                       n_slab, n_r, n_ang, n_psd, wc, wss, sk, sp, x, lam, props, p11, sums);
+  else
+    hipLaunchKernelGGL(gm::k_lut_contract<3>,
+                       dim3(blocks, (unsigned)((n_psd + 47) / 48)), dim3(64), 0,
+                       s, n_slab, n_r, n_ang, n_psd, wc, wss, sk, sp, x, lam, props, p11, sums);
+  const int per = gm::kLutFinish * (n_mom <= 32 ? 2 : 1);
+  hipLaunchKernelGGL(gm::k_lut_finish, dim3((unsigned)((n_ent + per - 1) / per)), dim3(64), 0, s,
+                     n_ent, n_ang, ng, n_mom,
                      (const double*)ctx->gsf_tab.ptr, sums, out);
   ctx->mark_end(slot, s);
   e = hipGetLastError();
