@@ -135,7 +135,23 @@ struct MieGrids {
   int lanes = 1;      // homogeneous kernel: lanes per point
   int lcap = 0;       // rows per lane segment (lanes > 1)
   int64_t small_grid = 0;   // grid of the 4-lane kernel for the short series (lanes > 1)
+  int long_lcap = 0;        // lanes = 1: rows per lane of the long series' kernel (0: none)
+  int64_t long_grid = 0;
 };
+
+// Long series of a batch that otherwise runs one point per lane (sorted, series of
+// at least kLongRows rows possible): points that cost more than kLongCost (cost =
+// nmx + 2 n_max, about 300 rows) and more than a lane's even share of the batch
+// (k_plan_scan) take a wavefront each.  One point per lane walks its rows serially, so a
+// point of x = 3400 held its wavefront for the whole 3.0 ms of a 1.2M-point LUT
+// batch whose CUs were 46% busy.  That batch: 2.97 ms serial; 2.35 with 16 lanes
+// for the long points, 2.25 with 32, 2.15 with 64, bounds of 1024 and 2048 alike.
+// Splitting points over lanes costs about twice the instructions: 300k points of x
+// uniform in 1..1500, where it saves no tail, took 2.9 ms serial and 3.6 with a
+// bound of half the share.
+constexpr int kLongLanes = 64;
+constexpr int kLongCost = 1024;
+constexpr int kLongRows = 512;
 
 // Lanes per point of the homogeneous kernel: the tuned value, or by batch:
 // one point per lane once the batch fills the GPU (64 points per wavefront,
@@ -178,6 +194,22 @@ MieGrids mie_grids(const gm_ctx* ctx, int64_t n, int rows_cap, size_t budget) {
     g.homog = std::make_pair(gg, (size_t)gg * slot_bytes);
   } else if (g.lanes == 1) {
     g.homog = grid_for(ctx->occ_homog[var], gm::kHomogRowDoubles);
+  }
+  if (g.lanes == 1) {
+    if (!ctx->tune_mie_lanes && rows_cap >= kLongRows) {
+      // the long series run first, on the same slots
+      const int lcap = (rows_cap + kLongLanes - 1) / kLongLanes;
+      const size_t slot_bytes = (size_t)lcap * 64 * gm::kHomogRowDoubles * sizeof(double);
+      const int64_t per_wave = 64 / kLongLanes;
+      int64_t gg = std::min<int64_t>((n + per_wave - 1) / per_wave,
+                                     (int64_t)ctx->n_cu * std::max(ctx->occ_coop, 1));
+      gg = std::min<int64_t>(gg, (int64_t)(budget / slot_bytes));
+      if (gg >= 1) {
+        g.long_lcap = lcap;
+        g.long_grid = gg;
+        g.homog.second = std::max(g.homog.second, (size_t)gg * slot_bytes);
+      }
+    }
   } else {
     g.lcap = (rows_cap + g.lanes - 1) / g.lanes;
     const size_t slot_bytes = (size_t)g.lcap * 64 * gm::kHomogRowDoubles * sizeof(double);
@@ -256,7 +288,8 @@ int mie_batch_run(gm_ctx* ctx, int64_t n, const double* x, const double* y, cons
     hipLaunchKernelGGL(gm::k_plan_keys, dim3(pblk), dim3(256), 0, s, n, x, y, eps, mu, eps2,
                        ws.key, nmax_out, hist, ws.status, per);
     hipLaunchKernelGGL(gm::k_plan_scan, dim3(1), dim3(256), 0, s, hist, cursor, range,
-                       gm::kSmallCost >> gm::kBucketShift, ab);
+                       (g.long_lcap ? kLongCost : gm::kSmallCost) >> gm::kBucketShift,
+                       g.long_lcap ? g.homog.first : (int64_t)0, ab);
     hipLaunchKernelGGL(gm::k_plan_scatter, dim3(pblk), dim3(256), 0, s, n,
                        (const int32_t*)ws.key, cursor, ws.order, per);
   } else {
@@ -281,6 +314,12 @@ int mie_batch_run(gm_ctx* ctx, int64_t n, const double* x, const double* y, cons
             : g.lanes == 32 ? gm::k_mie_homog_coop<32> : gm::k_mie_homog_coop<64>;
     cap_arg = g.lcap;
     hrange = ab;
+  }
+  if (g.long_lcap && (flags & GM_MIE_SORT)) {
+    hipLaunchKernelGGL(gm::k_mie_homog_coop<kLongLanes>, dim3((unsigned)g.long_grid), dim3(64), 0,
+                       s, order, ab, n, x, y, eps, mu, eps2, coef_off, an, bn, props, ws.status,
+                       ws.slots, g.long_lcap, dn_extra);
+    hrange = ab + 2;
   }
   hipLaunchKernelGGL(homog, dim3((unsigned)g.homog.first), dim3(64), 0, s, order, hrange, n, x, y,
                      eps, mu, eps2, coef_off, an, bn, props, ws.status, ws.slots, cap_arg,

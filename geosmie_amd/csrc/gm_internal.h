@@ -20,7 +20,7 @@ __global__ void k_plan_keys(int64_t n, const double* x, const double* y, const d
                             const double* mu, const double* eps2, int32_t* key,
                             int32_t* nmax_out, int64_t* hist, int32_t* status, int per);
 __global__ void k_plan_scan(const int64_t* hist, int64_t* cursor, int64_t* range, int small_b,
-                            int64_t* ab);
+                            int64_t slots, int64_t* ab);
 __global__ void k_plan_scatter(int64_t n, const int32_t* key, int64_t* cursor, int64_t* order,
                                int per);
 __global__ void k_plan_identity(int64_t n, int64_t* order, int64_t* range, int64_t* ab);

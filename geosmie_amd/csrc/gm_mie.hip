@@ -173,11 +173,14 @@ __global__ __launch_bounds__(256) void k_plan_keys(
 // class boundaries that fall in it.
 // Also splits the homogeneous class at the first bucket of cost below
 // small_b (buckets descend along the order): ab = {begin, split, split, end},
-// the points run with many lanes per point and those run with few.
+// the points run with many lanes per point and those run with few.  slots > 0
+// (the wavefronts of the lane-per-point kernel) raises the bound to the cost that
+// an even share of the batch puts on a lane of one of them: only points that would
+// keep a wavefront running after the others have finished are split over lanes.
 __global__ __launch_bounds__(256) void k_plan_scan(const int64_t* __restrict__ hist,
                                                    int64_t* __restrict__ cursor,
                                                    int64_t* __restrict__ range, int small_b,
-                                                   int64_t* __restrict__ ab) {
+                                                   int64_t slots, int64_t* __restrict__ ab) {
   __shared__ int64_t part[256];
   constexpr int per = (kClasses * kBuckets) / 256;
   static_assert(per * 256 == kClasses * kBuckets, "histogram must split into 256 runs");
@@ -210,6 +213,24 @@ __global__ __launch_bounds__(256) void k_plan_scan(const int64_t* __restrict__ h
     acc += h[i];
   }
   if (t == 255) range[2 * kClasses - 1] = acc;
+  if (slots > 0) {
+    // cost of the homogeneous class (keys 0 .. kBuckets - 1, cost descending)
+    int64_t c = 0;
+#pragma unroll
+    for (int i = 0; i < per; ++i) {
+      const int j = t * per + i;
+      if (j < kBuckets) c += h[i] * (kBuckets - 1 - j);
+    }
+    __syncthreads();
+    part[t] = c;
+    __syncthreads();
+    for (int off = 128; off > 0; off >>= 1) {
+      if (t < off) part[t] += part[t + off];
+      __syncthreads();
+    }
+    const int64_t share = part[0] / (64 * slots);
+    if (share > small_b) small_b = (int)min(share, (int64_t)kBuckets);
+  }
   __syncthreads();
   if (t == 0 && ab) {
     const int key = kBuckets - min(max(small_b, 0), kBuckets);   // class 0's first small key

@@ -108,7 +108,8 @@ enum gm_tune_param {
                                    (large batches); 16, 32, 64 = each point's rows split over that
                                    many lanes, its serial recurrences joined by parallel scans
                                    (batches too small to fill the GPU); 0 (default) = chosen from
-                                   the batch size and series length.  Results agree to rounding */,
+                                   the batch size and series length, a large batch's longest
+                                   points with 64 lanes each.  Results agree to rounding */,
   GM_TUNE_PSD_QUIRKS = 9,       /* a behaviour setting, not tuned for speed: the integratePSD
                                    quirks gm_integrate_psd[_rows] reproduce (GM_PSD_QUIRK_* bits;
                                    default GM_PSD_QUIRK_ALIAS) */
