@@ -357,7 +357,13 @@ int gm_psd_contract(gm_ctx* ctx, int n_psd, int64_t n_pts, int n_cols, const dou
   hipStream_t s = (hipStream_t)stream;
   size_t slot;
   ctx->mark_begin(gm::kKPsd, s, &slot);
-  if (n_psd <= gm::kSmallPsd) {
+  // columns that fit one MFMA tile (the integratePSD features) go to the narrow
+  // kernel whatever the rows: the few-row kernel has one thread per column, 13 of
+  // a block's 256 here (8 rows x 40k points x 13 columns: 97 + 76 us with its
+  // reduction against 14 + 5)
+  const int64_t narrow_splits = (n_pts + gm::kNarrowChunk - 1) / gm::kNarrowChunk;
+  const bool narrow = n_cols <= 16 && narrow_splits <= 65535;
+  if (n_psd <= gm::kSmallPsd && !narrow) {
     const int chunk = ctx->tune_psd_chunk;
     int nsplit = (int)std::max<int64_t>(1, (n_pts + chunk - 1) / chunk);
     size_t bytes = sizeof(double) * (size_t)nsplit * n_psd * n_cols;
