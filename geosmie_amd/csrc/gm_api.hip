@@ -134,6 +134,8 @@ struct MieGrids {
   std::pair<int64_t, size_t> homog, stable, literal;
   int lanes = 1;      // homogeneous kernel: lanes per point
   int lcap = 0;       // rows per lane segment (lanes > 1)
+  int coated_lanes = 1;     // coated class (real / weakly absorbing shells): lanes per point
+  int coated_lcap = 0;      // rows per lane segment (coated_lanes > 1)
   int64_t small_grid = 0;   // grid of the 4-lane kernel for the short series (lanes > 1)
   int long_lcap = 0;        // lanes = 1: rows per lane of the long series' kernel (0: none)
   int64_t long_grid = 0;
@@ -164,6 +166,20 @@ int mie_lanes(const gm_ctx* ctx, int64_t n, int rows_cap) {
   if (n >= (int64_t)64 * ctx->n_cu * 4 * 4) return 1;
   if (rows_cap <= 64 && n >= (int64_t)64 * ctx->n_cu * 4) return 1;
   return rows_cap <= 300 ? 16 : rows_cap <= 1200 ? 32 : 64;
+}
+
+// Lanes per point of the coated kernel (real / weakly absorbing shells): P lanes
+// while the batch leaves SIMDs idle at one point per lane, as few as still fill
+// them.  Times in us, serial / 16 / 32 / 64 lanes, shells y in 100..209: 512 points
+// 281 / 59 / 51 / 48, 2048 points 282 / 64 / 55 / 76, 8192 points 278 / 106, 24576
+// points 289 / 245, 32768 points 295 / 318; y in 800..1000: 24576 points 1217 / 745.
+// Short series gain less (y in 1..20: 2048 points 68 / 46, 8192 points 68 / 72),
+// so the bound falls with the series length.  A caller who sets the checkpoint
+// knob or a register budget chooses among the lane-per-point forms.
+int coated_lanes(const gm_ctx* ctx, int64_t n, int rows_cap) {
+  if (ctx->mie_ckpt_set || ctx->tune_mie_waves != 0) return 1;
+  if (n > (int64_t)ctx->n_cu * std::min(96, std::max(24, rows_cap / 2))) return 1;
+  return n <= (int64_t)ctx->n_cu * 4 ? 64 : n <= (int64_t)ctx->n_cu * 8 ? 32 : 16;
 }
 
 // The lane-per-point homogeneous kernel in its checkpointed form: with the
@@ -227,7 +243,17 @@ MieGrids mie_grids(const gm_ctx* ctx, int64_t n, int rows_cap, size_t budget) {
   }
   g.literal = grid_for(ctx->occ_literal, gm::kCoatedRowDoubles);
   const int ck = ctx->tune_mie_ckpt;
-  if (ck == 0) {
+  g.coated_lanes = coated_lanes(ctx, n, rows_cap);
+  if (g.coated_lanes > 1) {
+    g.coated_lcap = (rows_cap + g.coated_lanes - 1) / g.coated_lanes;
+    const size_t slot_bytes =
+        (size_t)g.coated_lcap * 64 * gm::kCoatedRowDoubles * sizeof(double);
+    const int64_t per_wave = 64 / g.coated_lanes;
+    int64_t gg = std::min<int64_t>((n + per_wave - 1) / per_wave,
+                                   (int64_t)ctx->n_cu * std::max(ctx->occ_coated_coop, 1));
+    gg = std::min<int64_t>(gg, std::max<int64_t>(1, (int64_t)(budget / slot_bytes)));
+    g.stable = std::make_pair(gg, (size_t)gg * slot_bytes);
+  } else if (ck == 0) {
     g.stable = grid_for(ctx->occ_stable[var], gm::kCoatedRowDoubles);
   } else {
     // a checkpointed slot: coated_ckpt_lane_doubles per lane (no per-row planes
@@ -343,8 +369,15 @@ int mie_batch_run(gm_ctx* ctx, int64_t n, const double* x, const double* y, cons
       stable = gm::k_mie_coated_ckpt<1, 5>;
     else if (ctx->tune_mie_ckpt == 8)
       stable = gm::k_mie_coated_ckpt<1, 8>;
+    int coated_cap = rows_cap;
+    if (g.coated_lanes > 1) {
+      stable = g.coated_lanes == 16   ? gm::k_mie_coated_coop<16>
+               : g.coated_lanes == 32 ? gm::k_mie_coated_coop<32>
+                                      : gm::k_mie_coated_coop<64>;
+      coated_cap = g.coated_lcap;
+    }
     hipLaunchKernelGGL(stable, dim3((unsigned)g.stable.first), dim3(64), 0, s, order, range, n, x,
-                       y, eps, mu, eps2, coef_off, an, bn, props, ws.status, ws.slots, rows_cap,
+                       y, eps, mu, eps2, coef_off, an, bn, props, ws.status, ws.slots, coated_cap,
                        dn_extra);
     ctx->mark_end(slot, s);
     HIP_OK(hipGetLastError());
@@ -417,6 +450,9 @@ int gm_ctx_create(int device, gm_ctx** out) {
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, gm::k_mie_homog_coop<16>, 64, 0) ==
       hipSuccess)
     c->occ_coop = occ;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, gm::k_mie_coated_coop<16>, 64, 0) ==
+      hipSuccess)
+    c->occ_coated_coop = occ;
   int rc = noalloc_init(device);
   if (!rc) rc = c->reserve(c->status, 64);
   if (rc) {
@@ -487,6 +523,7 @@ int gm_ctx_tune(gm_ctx* ctx, int param, int value) {
       if (value != 0 && value != 4 && value != 5 && value != 8)
         return gm_fail(GM_EINVAL, "gm_ctx_tune: rows per checkpoint must be 0, 4, 5 or 8");
       ctx->tune_mie_ckpt = value;
+      ctx->mie_ckpt_set = true;
       return GM_OK;
     case GM_TUNE_MIE_LANES:
       if (value != 0 && value != 1 && value != 16 && value != 32 && value != 64)

@@ -26,6 +26,7 @@ struct gm_ctx {
   // (unconstrained, >= 3 waves per SIMD) and K = 8
   int occ_ckpt4[2] = {8, 8}, occ_ckpt5 = 8, occ_ckpt8 = 5;
   int occ_coop = 8;             // the homogeneous kernel with P lanes per point
+  int occ_coated_coop = 4;      // the coated kernel with P lanes per point
   int occ_homog_ckpt = 8;       // the checkpointed homogeneous kernel (K = 4)
 
   size_t scratch_budget = (size_t)3 << 30;       // bytes of recurrence scratch
@@ -38,6 +39,7 @@ struct gm_ctx {
   int tune_mie_waves = 0;       // Mie register variant: 0 unconstrained, 3 or 4 waves per SIMD
   int tune_s12_layout = 0;      // accepted, no effect
   int tune_mie_ckpt = 4;        // coated kernel: rows per checkpoint (4, 8) or 0 = every row stored
+  bool mie_ckpt_set = false;    // tune_mie_ckpt chosen by the caller: one coated point per lane
   int tune_mie_lanes = 0;       // homogeneous kernel: lanes per point (1, 16, 32, 64; 0 = by batch)
   int psd_quirks = 1;           // integratePSD quirks reproduced (GM_PSD_QUIRK_* bits)
   int tune_s12_share = 1;        // split-BF16 fused S1/S2: angle-table tiles shared through LDS

@@ -700,25 +700,28 @@ __device__ __forceinline__ cm2 cm2_eye() {
   return cm2{cd{1.0, 0.0}, cd{0.0, 0.0}, cd{0.0, 0.0}, cd{1.0, 0.0}};
 }
 __device__ __forceinline__ rm2 rm2_eye() { return rm2{1.0, 0.0, 0.0, 1.0}; }
-// scale by a power of two so the largest component is in [0.5, 1) (exact)
-__device__ __forceinline__ void renorm(cm2& m) {
+// scale by a power of two so the largest component is in [0.5, 1) (exact);
+// returns the exponent taken out
+__device__ __forceinline__ int renorm(cm2& m) {
   double mx = fmax(fmax(fmax(fabs(m.a.re), fabs(m.a.im)), fmax(fabs(m.b.re), fabs(m.b.im))),
                    fmax(fmax(fabs(m.c.re), fabs(m.c.im)), fmax(fabs(m.d.re), fabs(m.d.im))));
-  if (mx == 0.0) return;
+  if (mx == 0.0) return 0;
   const int e = __builtin_amdgcn_frexp_exp(mx);
   m.a = cd{ldexp(m.a.re, -e), ldexp(m.a.im, -e)};
   m.b = cd{ldexp(m.b.re, -e), ldexp(m.b.im, -e)};
   m.c = cd{ldexp(m.c.re, -e), ldexp(m.c.im, -e)};
   m.d = cd{ldexp(m.d.re, -e), ldexp(m.d.im, -e)};
+  return e;
 }
-__device__ __forceinline__ void renorm(rm2& m) {
+__device__ __forceinline__ int renorm(rm2& m) {
   double mx = fmax(fmax(fabs(m.a), fabs(m.b)), fmax(fabs(m.c), fabs(m.d)));
-  if (mx == 0.0) return;
+  if (mx == 0.0) return 0;
   const int e = __builtin_amdgcn_frexp_exp(mx);
   m.a = ldexp(m.a, -e);
   m.b = ldexp(m.b, -e);
   m.c = ldexp(m.c, -e);
   m.d = ldexp(m.d, -e);
+  return e;
 }
 // shuffles within a group of P lanes (source lane index relative to the group)
 template <int P>
@@ -1088,40 +1091,58 @@ struct CoatedPt {
   int nmax, nsw_v, nsw_w, nsw_y;
   bool ddv_on, ddw_on;
 };
+// psi_{n-1}, psi_{n-2} and chi_{n-1}, chi_{n-2} of a chain before row n
+template <class T>
+struct RbPair {
+  T psi_p, psi_pp, chi_p, chi_pp;
+};
+struct CoatedState {
+  RbPair<cd> v, w;
+  RbPair<double> y;
+};
+__device__ __forceinline__ CoatedState coated_state1(cd v, cd w, double y) {
+  CoatedState s;
+  csincos_(v, s.v.psi_p, s.v.psi_pp);   // psi_0 = sin, psi_{-1} = cos
+  s.v.chi_pp = -s.v.psi_p;              // chi_{-1}, chi_0
+  s.v.chi_p = s.v.psi_pp;
+  csincos_(w, s.w.psi_p, s.w.psi_pp);
+  s.w.chi_pp = -s.w.psi_p;
+  s.w.chi_p = s.w.psi_pp;
+  double sn, cs;
+  sincos(y, &sn, &cs);
+  s.y = RbPair<double>{sn, cs, cs, -sn};
+  return s;
+}
+// Rows n0 .. n1 from the state before n0; the slot's row 0 is n0.  ab1: a, b
+// of the first row (the pair across a segment boundary), or null.
 template <bool DD, bool STORE>
-__device__ __forceinline__ void coated_up(const CoatedPt& c, __amdgpu_buffer_rsrc_t rs,
-                                          uint32_t plane, int lane, int64_t off,
-                                          double* __restrict__ an, double* __restrict__ bn,
-                                          Props& pr) {
+__device__ __forceinline__ void coated_rows(const CoatedPt& c, const CoatedState& st, int n0,
+                                            int n1, __amdgpu_buffer_rsrc_t rs, uint32_t plane,
+                                            int lane, int64_t off, double* __restrict__ an,
+                                            double* __restrict__ bn, Props& pr, cd* ab1) {
   const cdd vinv = crcp_dd(c.v), winv = crcp_dd(c.w), minv = crcp_dd(c.m);
   const ddr yinv = rcp_dd(c.y);
   const cd m = c.m, m2 = c.m2;
-  const int nmax = c.nmax, nsw_v = c.nsw_v, nsw_w = c.nsw_w, nsw_y = c.nsw_y;
-  cd pv_p, pv_pp;   // psi_0(v) = sin v, psi_{-1}(v) = cos v
-  csincos_(c.v, pv_p, pv_pp);
-  cd cv_pp = -pv_p, cv_p = pv_pp;             // chi_{-1}(v), chi_0(v)
-  cd pw_p, pw_pp;
-  csincos_(c.w, pw_p, pw_pp);
-  cd cw_pp = -pw_p, cw_p = pw_pp;
-  double sn, cs;
-  sincos(c.y, &sn, &cs);
-  double py_pp = cs, py_p = sn, cy_pp = -sn, cy_p = cs;
-  // byte offsets of row 1 of each plane for this lane; a row adds 64 entries
+  const int nsw_v = c.nsw_v, nsw_w = c.nsw_w, nsw_y = c.nsw_y;
+  cd pv_p = st.v.psi_p, pv_pp = st.v.psi_pp, cv_p = st.v.chi_p, cv_pp = st.v.chi_pp;
+  cd pw_p = st.w.psi_p, pw_pp = st.w.psi_pp, cw_p = st.w.chi_p, cw_pp = st.w.chi_pp;
+  double py_p = st.y.psi_p, py_pp = st.y.psi_pp, cy_p = st.y.chi_p, cy_pp = st.y.chi_pp;
+  // byte offsets of row n0 of each plane for this lane; a row adds 64 entries
   const uint32_t b_du = 16u * (uint32_t)lane, b_rv = 16u * (plane + (uint32_t)lane),
                  b_rw = 16u * (2u * plane + (uint32_t)lane),
                  b_ddv = 16u * (3u * plane + (uint32_t)lane),
                  b_ddw = 16u * (4u * plane + (uint32_t)lane),
                  b_ry = 8u * (10u * plane + (uint32_t)lane);
   // the stored rows of step n + 1 are loaded during step n
-  cd du_nx = ld_cd(rs, b_du, true), rv_nx = ld_cd(rs, b_rv, nsw_v < 1),
-     rw_nx = ld_cd(rs, b_rw, nsw_w < 1);
-  double ry_nx = ld_d(rs, b_ry, nsw_y < 1);
+  cd du_nx = ld_cd(rs, b_du, true), rv_nx = ld_cd(rs, b_rv, nsw_v < n0),
+     rw_nx = ld_cd(rs, b_rw, nsw_w < n0);
+  double ry_nx = ld_d(rs, b_ry, nsw_y < n0);
 #pragma unroll 2
-  for (int n = 1; n <= nmax; ++n) {
-    const uint32_t r = (uint32_t)(n - 1) * 64u;
+  for (int n = n0; n <= n1; ++n) {
+    const uint32_t r = (uint32_t)(n - n0) * 64u;
     const cd du = du_nx, rv = rv_nx, rw = rw_nx;
     const double ry = ry_nx;
-    const bool more = n < nmax;
+    const bool more = n < n1;
     du_nx = ld_cd(rs, b_du + 16u * (r + 64u), more);
     rv_nx = ld_cd(rs, b_rv + 16u * (r + 64u), more && n >= nsw_v);
     rw_nx = ld_cd(rs, b_rw + 16u * (r + 64u), more && n >= nsw_w);
@@ -1164,6 +1185,10 @@ __device__ __forceinline__ void coated_up(const CoatedPt& c, __amdgpu_buffer_rsr
     cd a, b;
     cdiv2(Pa * py - Ma * py_p, Pa * xi - Ma * xi1, Pb * py - Dg * py_p, Pb * xi - Dg * xi1, a, b);
     pr.add_seq(n, a, b);
+    if (ab1 && n == n0) {
+      ab1[0] = a;
+      ab1[1] = b;
+    }
     if constexpr (STORE) {
       an[2 * (off + n - 1)] = a.re;
       an[2 * (off + n - 1) + 1] = a.im;
@@ -1271,21 +1296,351 @@ __global__ __launch_bounds__(64, MINW) void k_mie_coated_stable(
       dn_chain(wi, nmx + 16 + 8 * (int)ceil(cbrt(aw)), nmax, DDW, lane, true);
     }
     // ---- pass 2: upward Riccati-Bessel recurrences and the combination,
-    // without divergent branches (coated_up); the start-index corrections
+    // without divergent branches (coated_rows); the start-index corrections
     // are compiled in only when a lane of the wavefront needs them
     Props pr;
     pr.init_seq();
     const int64_t off = coef_off ? coef_off[p] : 0;
     const CoatedPt cp{v, w, yy, m, m2, nmax, nsw_v, nsw_w, nsw_y, ddv_on, ddw_on};
     const __amdgpu_buffer_rsrc_t rs = slot_rsrc(slot, (uint32_t)(plane * 11 * sizeof(double)));
+    const CoatedState st = coated_state1(v, w, yy);
+    const uint32_t pl = (uint32_t)plane;
     if (__any(ddv_on || ddw_on)) {
-      if (coef_off) coated_up<true, true>(cp, rs, (uint32_t)plane, lane, off, an, bn, pr);
-      else coated_up<true, false>(cp, rs, (uint32_t)plane, lane, off, an, bn, pr);
+      if (coef_off) coated_rows<true, true>(cp, st, 1, nmax, rs, pl, lane, off, an, bn, pr, nullptr);
+      else coated_rows<true, false>(cp, st, 1, nmax, rs, pl, lane, off, an, bn, pr, nullptr);
     } else {
-      if (coef_off) coated_up<false, true>(cp, rs, (uint32_t)plane, lane, off, an, bn, pr);
-      else coated_up<false, false>(cp, rs, (uint32_t)plane, lane, off, an, bn, pr);
+      if (coef_off)
+        coated_rows<false, true>(cp, st, 1, nmax, rs, pl, lane, off, an, bn, pr, nullptr);
+      else coated_rows<false, false>(cp, st, 1, nmax, rs, pl, lane, off, an, bn, pr, nullptr);
     }
     if (props) pr.finish(yy, p, n_all, props);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Coated sphere, real or weakly absorbing shell, P lanes per point (small batches)
+// ---------------------------------------------------------------------------
+// k_mie_coated_stable's arithmetic on k_mie_homog_coop's split: lane j of a
+// group takes rows jL+1 .. (j+1)L, and the serial chains (D_n(u) and the psi
+// ratios of v, w, y downward; psi and chi of v, w, y upward) are joined across
+// the lanes by scans of their transfer matrices.  A batch of a few thousand
+// points is otherwise a few dozen wavefronts, each as long as its longest
+// point: 1266 points to y = 209 took 305 us a call on 20 of 1024 SIMDs, 56 with 32
+// lanes a point.  What bounds it then is the scans' fixed cost, about 20 us a
+// wavefront, and their full matrix products: two to three times the serial
+// instructions for a series of 200 rows, so a batch that fills the chip runs one
+// point per lane.  Largest |a_n| errors against extended precision (2048 points,
+// y to 400): 1.8e-11 here, 2.8e-9 one point per lane (the start-index correction
+// next to poles of D_n(m2 y), coop_dd).
+//
+// One step of a downward chain, t -> [[r, r^2 - 1], [1, r]] t, and of an
+// upward one, t -> [[f, -1], [1, 0]] t.
+template <class M, class T>
+__device__ __forceinline__ void step_down(M& t, T r) {
+  const T c = t.a + r * t.c, d = t.b + r * t.d;
+  t.a = r * c - t.c;
+  t.b = r * d - t.d;
+  t.c = c;
+  t.d = d;
+}
+template <class M, class T>
+__device__ __forceinline__ void step_up(M& t, T f) {
+  const T a = f * t.a - t.c, b = f * t.b - t.d;
+  t.c = t.a;
+  t.d = t.b;
+  t.a = a;
+  t.b = b;
+}
+template <class T>
+struct ChainOf;
+template <>
+struct ChainOf<cd> {
+  using M = cm2;
+  using Z = cdd;
+  static __device__ __forceinline__ M eye() { return cm2_eye(); }
+  static __device__ __forceinline__ cd one() { return cd{1.0, 0.0}; }
+  static __device__ __forceinline__ cd rcp(cd z) { return crcp_fast(z); }
+  static __device__ __forceinline__ cd div(cd a, cd b) { return cdiv(a, b); }
+  static __device__ __forceinline__ cd scale(cd a, int e) {
+    return cd{ldexp(a.re, e), ldexp(a.im, e)};
+  }
+};
+template <>
+struct ChainOf<double> {
+  using M = rm2;
+  using Z = ddr;
+  static __device__ __forceinline__ M eye() { return rm2_eye(); }
+  static __device__ __forceinline__ double one() { return 1.0; }
+  static __device__ __forceinline__ double rcp(double z) { return rcp_nr(z); }
+  static __device__ __forceinline__ double div(double a, double b) { return a / b; }
+  static __device__ __forceinline__ double scale(double a, int e) { return ldexp(a, e); }
+};
+template <int P>
+__device__ __forceinline__ cd grp_up(cd v, int d) {
+  return cd{grp_up<P>(v.re, d), grp_up<P>(v.im, d)};
+}
+template <int P>
+__device__ __forceinline__ cd grp_get(cd v, int src) {
+  return cd{grp_get<P>(v.re, src), grp_get<P>(v.im, src)};
+}
+template <int P>
+__device__ __forceinline__ cm2 grp_up(const cm2& m, int d) {
+  return cm2{grp_up<P>(m.a, d), grp_up<P>(m.b, d), grp_up<P>(m.c, d), grp_up<P>(m.d, d)};
+}
+// Transfer matrix (times 2^e) of a downward chain from above row `start` to below
+// row n1 + 1 of this lane's rows lo .. n1: rows start .. nmax+1, split over the
+// lanes as well, and the higher lanes' rows.  The chain's r at row k is
+// (k + add) / z.  Four steps between rescalings stay in range below |r| = 1e10.
+template <int P, class T>
+__device__ __forceinline__ typename ChainOf<T>::M coop_down(typename ChainOf<T>::Z zi, int add,
+                                                            int start, int nmax, int lo, int n1,
+                                                            double zabs, int j, int& e) {
+  using C = ChainOf<T>;
+  const int mask = (double)(start + add) < 1e10 * zabs ? 3 : 0;
+  const int HL = (start - nmax + P - 1) / P;
+  auto run = [&](int k1, int k0, int& ex) {
+    auto t = C::eye();
+    int cnt = 0;
+    ex = 0;
+    for (int k = k1; k >= k0; --k) {
+      step_down(t, mul_dd((double)(k + add), zi));
+      if ((++cnt & mask) == 0) ex += renorm(t);
+    }
+    ex += renorm(t);
+    // inclusive suffix product: T_j T_{j+1} ... T_{P-1}
+#pragma unroll
+    for (int d = 1; d < P; d <<= 1) {
+      const auto o = grp_down<P>(t, d);
+      const int oe = __shfl_down(ex, d, P);
+      if (j + d < P) {
+        t = t * o;
+        ex += oe + renorm(t);
+      }
+    }
+    return t;
+  };
+  int eh, es;
+  const auto head = grp_get<P>(
+      run(min(nmax + (j + 1) * HL, start), nmax + 1 + j * HL, eh), 0);
+  eh = __shfl(eh, 0, P);
+  auto sfx = grp_down<P>(run(n1, lo, es), 1);   // T_{j+1} ... T_{P-1}
+  es = __shfl_down(es, 1, P);
+  if (j == P - 1) {
+    sfx = C::eye();
+    es = 0;
+  }
+  auto t = sfx * head;
+  e = es + eh + renorm(t);
+  return t;
+}
+// Value entering this lane's rows from above, of a chain that is zero above row
+// `start`.
+template <int P, class T>
+__device__ __forceinline__ T coop_enter(typename ChainOf<T>::Z zi, int add, int start, int nmax,
+                                        int lo, int n1, double zabs, int j) {
+  int e;
+  const auto t = coop_down<P, T>(zi, add, start, nmax, lo, n1, zabs, j, e);
+  return ChainOf<T>::div(t.b, t.d);
+}
+// D_n of z from D_nmx = 0 on this lane's rows.
+template <int P>
+__device__ __forceinline__ void coop_dn(cdd zi, int nmx, int nmax, int n0, int n1, double zabs,
+                                        int j, cd* __restrict__ plane) {
+  cd dd = coop_enter<P, cd>(zi, 1, nmx - 1, nmax, n0, n1, zabs, j);
+  for (int k = n1; k >= n0; --k) {
+    const cd r = mul_dd((double)(k + 1), zi);
+    dd = r - crcp_fast(dd + r);
+    plane[(size_t)(k - n0) * 64] = dd;
+  }
+}
+// Start-index correction dD = D (from D_nmx = 0) - D (from D_far = 0) on this
+// lane's rows.  Joined over lanes, two separate chains would not fall onto the
+// same bits once converged, as serial ones do, and a row near a pole of D would
+// magnify what they differ by; so the difference itself is carried:
+// dD_k = dD_{k+1} / ((D_{k+1} + r) (D'_{k+1} + r)), and across the rows above
+// through the determinant, which is 1 a step.
+template <int P>
+__device__ __forceinline__ void coop_dd(cdd zi, int nmx, int far, int nmax, int n0, int n1,
+                                        double zabs, int j, cd* __restrict__ plane) {
+  cd f = cd{0.0, 0.0};                               // D' at nmx, where D is 0
+  for (int k = far - 1; k >= nmx; --k) {
+    const cd r = mul_dd((double)(k + 1), zi);
+    f = r - crcp_fast(f + r);
+  }
+  int e;
+  const cm2 t = coop_down<P, cd>(zi, 1, nmx - 1, nmax, n0, n1, zabs, j, e);
+  const cd den = t.c * f + t.d;
+  cd d0 = cdiv(t.b, t.d), d1 = cdiv(t.a * f + t.b, den);
+  cd dd = ChainOf<cd>::scale(cdiv(cd{-f.re, -f.im}, t.d * den), -2 * e);
+  for (int k = n1; k >= n0; --k) {
+    const cd r = mul_dd((double)(k + 1), zi);
+    const cd i0 = crcp_fast(d0 + r), i1 = crcp_fast(d1 + r);
+    dd = dd * (i0 * i1);
+    plane[(size_t)(k - n0) * 64] = dd;
+    d0 = r - i0;
+    d1 = r - i1;
+  }
+}
+// One Riccati-Bessel argument: the psi ratios of this lane's rows above nsw
+// into `plane`, and the psi, chi pairs before row n0.  chi's transfer products
+// carry their exponent apart, so chi leaves the range exactly where the serial
+// recurrence does.
+template <int P, class T>
+__device__ __forceinline__ RbPair<T> coop_rb(typename ChainOf<T>::Z zi, double zabs, T sn, T cs,
+                                             int nsw, int nmax, int L, int n0, int n1, int j,
+                                             T* __restrict__ plane) {
+  using C = ChainOf<T>;
+  RbPair<T> s;
+  {
+    const int mask = (double)(2 * nmax) < 1e30 * zabs ? 7 : 0;
+    auto u = C::eye();
+    int e = 0, cnt = 0;
+    for (int n = n0; n <= n1; ++n) {
+      step_up(u, mul_dd((double)(2 * n - 1), zi));
+      if ((++cnt & mask) == 0) e += renorm(u);
+    }
+    e += renorm(u);
+#pragma unroll
+    for (int d = 1; d < P; d <<= 1) {
+      const auto o = grp_up<P>(u, d);
+      const int oe = __shfl_up(e, d, P);
+      if (j >= d) {
+        u = u * o;
+        e += oe + renorm(u);
+      }
+    }
+    auto ex = grp_up<P>(u, 1);                       // U_{j-1} ... U_0
+    int ee = __shfl_up(e, 1, P);
+    if (j == 0) {
+      ex = C::eye();
+      ee = 0;
+    }
+    s.psi_p = C::scale(ex.a * sn + ex.b * cs, ee);   // psi_{n0-1}
+    s.psi_pp = C::scale(ex.c * sn + ex.d * cs, ee);
+    s.chi_p = C::scale(ex.a * cs - ex.b * sn, ee);
+    s.chi_pp = C::scale(ex.c * cs - ex.d * sn, ee);
+  }
+  if (nsw < nmax) {
+    const int lo = max(n0, nsw + 1);
+    T dr = coop_enter<P, T>(zi, 0, ratio_start(nmax, zabs), nmax, lo, n1, zabs, j);
+    T prod = C::one();
+    for (int k = n1; k >= lo; --k) {
+      const T r = mul_dd((double)k, zi);
+      const T it = C::rcp(dr + r);
+      plane[(size_t)(k - n0) * 64] = it;
+      prod = prod * it;
+      dr = r - it;
+    }
+    // psi at nsw, upward from the pair of the lane whose rows hold it
+    T pn = sn;
+    const int js = nsw >= 1 ? (nsw - 1) / L : 0;
+    if (nsw >= 1 && j == js) {
+      T b = s.psi_pp;
+      pn = s.psi_p;
+      for (int n = n0; n <= nsw; ++n) {
+        const T c = mul_dd((double)(2 * n - 1), zi) * pn - b;
+        b = pn;
+        pn = c;
+      }
+    }
+    pn = grp_get<P>(pn, js);
+    // product of the ratios below this lane's rows
+#pragma unroll
+    for (int d = 1; d < P; d <<= 1) {
+      const T o = grp_up<P>(prod, d);
+      if (j >= d) prod = prod * o;
+    }
+    T pre = grp_up<P>(prod, 1);
+    if (j == 0) pre = C::one();
+    if (n0 - 1 >= nsw) s.psi_p = pn * pre;
+  }
+  return s;
+}
+
+template <int P>
+__global__ __launch_bounds__(64) void k_mie_coated_coop(
+    const int64_t* __restrict__ order, const int64_t* __restrict__ range, int64_t n_all,
+    const double* __restrict__ x, const double* __restrict__ y, const double* __restrict__ eps,
+    const double* __restrict__ mu, const double* __restrict__ eps2,
+    const int64_t* __restrict__ coef_off, double* __restrict__ an, double* __restrict__ bn,
+    double* __restrict__ props, int32_t* __restrict__ status, double* __restrict__ scratch,
+    int lcap, int dn_extra) {
+  constexpr int W = 64 / P;
+  const int lane = threadIdx.x;
+  const int j = lane % P, grp = lane / P;
+  const int64_t begin = range[2], end = range[3];
+  const size_t plane = (size_t)lcap * 64;
+  double* slot = scratch + (size_t)blockIdx.x * plane * 11;
+  cd* DU = reinterpret_cast<cd*>(slot) + lane;           // [row in segment][lane]
+  cd* RV = reinterpret_cast<cd*>(slot + 2 * plane) + lane;
+  cd* RW = reinterpret_cast<cd*>(slot + 4 * plane) + lane;
+  cd* DDV = reinterpret_cast<cd*>(slot + 6 * plane) + lane;
+  cd* DDW = reinterpret_cast<cd*>(slot + 8 * plane) + lane;
+  double* RY = slot + 10 * plane + lane;
+  const __amdgpu_buffer_rsrc_t rs = slot_rsrc(slot, (uint32_t)(plane * 11 * sizeof(double)));
+
+  for (int64_t base = begin + (int64_t)blockIdx.x * W; base < end;
+       base += (int64_t)gridDim.x * W) {
+    const int64_t idx = base + grp;
+    if (idx >= end) continue;                    // the whole group: no shuffle partners lost
+    const int64_t p = order[idx];
+    PointDesc d = describe(p, x, y, eps, mu, eps2);
+    if (d.cls != 1) continue;
+    const double yy = d.size, xx = d.xcore;
+    const int nmax = nmax_rule(yy);
+    const int L = (nmax + P - 1) / P;
+    if (L > lcap) {
+      if (j == 0) atomicOr(status, 1);
+      continue;
+    }
+    const cd m1 = csqrt_(d.eps), m2 = csqrt_(d.eps2);
+    const cd m = cdiv(m2, m1);
+    const cd u = m1 * xx, v = m2 * xx, w = m2 * yy;
+    const double mxv = fmax(cabs_(m1 * yy), cabs_(w));
+    const int nmx =
+        nmx_rule(nmax, mxv) + (dn_extra < 0 ? 16 + 10 * (int)ceil(cbrt(mxv)) : dn_extra);
+    const double av = cabs_(v), aw = cabs_(w);
+    const int nsw_v = min((int)av, nmax), nsw_w = min((int)aw, nmax), nsw_y = min((int)yy, nmax);
+    const int n0 = j * L + 1, n1 = min((j + 1) * L, nmax);   // this lane's rows (may be empty)
+    const cdd vi = crcp_dd(v), wi = crcp_dd(w);
+
+    coop_dn<P>(crcp_dd(u), nmx, nmax, n0, n1, cabs_(u), j, DU);
+    CoatedState st = coated_state1(v, w, yy);
+    st.v = coop_rb<P, cd>(vi, av, st.v.psi_p, st.v.psi_pp, nsw_v, nmax, L, n0, n1, j, RV);
+    st.w = coop_rb<P, cd>(wi, aw, st.w.psi_p, st.w.psi_pp, nsw_w, nmax, L, n0, n1, j, RW);
+    st.y = coop_rb<P, double>(rcp_dd(yy), yy, st.y.psi_p, st.y.psi_pp, nsw_y, nmax, L, n0, n1, j,
+                              RY);
+    const bool ddv_on = !converged_start(nmx, av), ddw_on = !converged_start(nmx, aw);
+    if (ddv_on)
+      coop_dd<P>(vi, nmx, nmx + 16 + 8 * (int)ceil(cbrt(av)), nmax, n0, n1, av, j, DDV);
+    if (ddw_on)
+      coop_dd<P>(wi, nmx, nmx + 16 + 8 * (int)ceil(cbrt(aw)), nmax, n0, n1, aw, j, DDW);
+    Props pr;
+    pr.init_seq();
+    pr.rn = rcp_nr((double)n0);
+    const int64_t off = coef_off ? coef_off[p] : 0;
+    const CoatedPt cp{v, w, yy, m, m2, nmax, nsw_v, nsw_w, nsw_y, ddv_on, ddw_on};
+    const uint32_t pl = (uint32_t)plane;
+    cd ab1[2] = {cd{0.0, 0.0}, cd{0.0, 0.0}};
+    if (__any(ddv_on || ddw_on)) {
+      if (coef_off) coated_rows<true, true>(cp, st, n0, n1, rs, pl, lane, off, an, bn, pr, ab1);
+      else coated_rows<true, false>(cp, st, n0, n1, rs, pl, lane, off, an, bn, pr, ab1);
+    } else {
+      if (coef_off) coated_rows<false, true>(cp, st, n0, n1, rs, pl, lane, off, an, bn, pr, ab1);
+      else coated_rows<false, false>(cp, st, n0, n1, rs, pl, lane, off, an, bn, pr, ab1);
+    }
+    // the pair (n0 - 1, n0) across the segment boundary
+    const cd pa = grp_up<P>(pr.ap, 1), pb = grp_up<P>(pr.bp, 1);
+    if (j > 0 && n0 <= nmax)
+      pr.asy1 = fma((double)n0 - rcp_nr((double)n0),
+                    pa.re * ab1[0].re + pa.im * ab1[0].im + pb.re * ab1[1].re + pb.im * ab1[1].im,
+                    pr.asy1);
+    pr.sext = grp_sum<P>(pr.sext);
+    pr.ssca = grp_sum<P>(pr.ssca);
+    pr.asy1 = grp_sum<P>(pr.asy1);
+    pr.asy2 = grp_sum<P>(pr.asy2);
+    pr.qb = cd{grp_sum<P>(pr.qb.re), grp_sum<P>(pr.qb.im)};
+    if (j == 0 && props) pr.finish(yy, p, n_all, props);
   }
 }
 
@@ -1296,7 +1651,7 @@ __global__ __launch_bounds__(64, MINW) void k_mie_coated_stable(
 // (block 0 as pass 1 left them; block b > 0 regenerated from checkpoint b,
 // the next one in flight, with exactly pass 1's operations), then the K
 // upward steps, unrolled by two.  The upward steps are branch-free as in
-// coated_up (both psi forms formed, one selected; the LDS rows of an
+// coated_rows (both psi forms formed, one selected; the LDS rows of an
 // inactive chain are read and ignored), the start-index corrections come
 // through range-checked loads and are compiled in only when a lane of the
 // wavefront needs them (DD); STORE writes a_n, b_n.
@@ -1838,6 +2193,9 @@ template __global__ void k_mie_homog_coop<4>(GM_MIE_ARGS);
 template __global__ void k_mie_homog_coop<16>(GM_MIE_ARGS);
 template __global__ void k_mie_homog_coop<32>(GM_MIE_ARGS);
 template __global__ void k_mie_homog_coop<64>(GM_MIE_ARGS);
+template __global__ void k_mie_coated_coop<16>(GM_MIE_ARGS);
+template __global__ void k_mie_coated_coop<32>(GM_MIE_ARGS);
+template __global__ void k_mie_coated_coop<64>(GM_MIE_ARGS);
 #undef GM_MIE_ARGS
 
 __global__ void k_nmax_of(int64_t n, const double* __restrict__ size, int64_t* __restrict__ cnt) {

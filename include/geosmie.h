@@ -100,7 +100,9 @@ enum gm_tune_param {
   GM_TUNE_MIE_CKPT = 7          /* coated kernel (real / weakly absorbing shells): the downward
                                    chains' states kept every 4, 5 or 8 rows and each block of rows
                                    regenerated in LDS before use (4, the default), or 0 = every
-                                   row kept in scratch; results agree to rounding.  Non-zero also
+                                   row kept in scratch; results agree to rounding.  Once set, every
+                                   batch runs one coated point per lane; unset, small batches split
+                                   each point's rows over 16, 32 or 64 lanes.  Non-zero also
                                    selects the checkpointed one-point-per-lane homogeneous kernel
                                    (every 4 rows, unless GM_TUNE_MIE_WAVES forces a register
                                    budget; bit-identical results) */,
