@@ -136,6 +136,8 @@ struct MieGrids {
   int lcap = 0;       // rows per lane segment (lanes > 1)
   int coated_lanes = 1;     // coated class (real / weakly absorbing shells): lanes per point
   int coated_lcap = 0;      // rows per lane segment (coated_lanes > 1)
+  int coated_long = 0;      // coated_lanes = 1: lanes per point of the long series (0: none)
+  int64_t coated_long_grid = 0;
   int64_t small_grid = 0;   // grid of the 4-lane kernel for the short series (lanes > 1)
   int long_lcap = 0;        // lanes = 1: rows per lane of the long series' kernel (0: none)
   int64_t long_grid = 0;
@@ -154,6 +156,14 @@ struct MieGrids {
 constexpr int kLongLanes = 64;
 constexpr int kLongCost = 1024;
 constexpr int kLongRows = 512;
+
+// Long coated series: a batch that runs one coated point per lane has its longest
+// points split over 16 or 64 lanes each where that shortens it (coated_split in
+// gm_mie.hip).  100k points, shells log-distributed to y = 209: 317 us with every
+// point serial, 180 split; 350k points 338 and 249.  From about 700k such points on the
+// longest chain is below an even share of the batch: above this size only batches
+// with long series look for a split, the others save the launch (5 us).
+constexpr int64_t kCoatedLongMax = 512 * 1024;
 
 // Lanes per point of the homogeneous kernel: the tuned value, or by batch:
 // one point per lane once the batch fills the GPU (64 points per wavefront,
@@ -244,10 +254,12 @@ MieGrids mie_grids(const gm_ctx* ctx, int64_t n, int rows_cap, size_t budget) {
   g.literal = grid_for(ctx->occ_literal, gm::kCoatedRowDoubles);
   const int ck = ctx->tune_mie_ckpt;
   g.coated_lanes = coated_lanes(ctx, n, rows_cap);
+  auto coop_slot = [&](int lanes) {
+    return (size_t)((rows_cap + lanes - 1) / lanes) * 64 * gm::kCoatedRowDoubles * sizeof(double);
+  };
   if (g.coated_lanes > 1) {
     g.coated_lcap = (rows_cap + g.coated_lanes - 1) / g.coated_lanes;
-    const size_t slot_bytes =
-        (size_t)g.coated_lcap * 64 * gm::kCoatedRowDoubles * sizeof(double);
+    const size_t slot_bytes = coop_slot(g.coated_lanes);
     const int64_t per_wave = 64 / g.coated_lanes;
     int64_t gg = std::min<int64_t>((n + per_wave - 1) / per_wave,
                                    (int64_t)ctx->n_cu * std::max(ctx->occ_coated_coop, 1));
@@ -267,6 +279,19 @@ MieGrids mie_grids(const gm_ctx* ctx, int64_t n, int rows_cap, size_t budget) {
         waves, (int64_t)ctx->n_cu * std::max(occ, 1) * std::max(ctx->tune_mie_grid_mult, 1));
     gg = std::min<int64_t>(gg, std::max<int64_t>(1, (int64_t)(budget / slot_bytes)));
     g.stable = std::make_pair(gg, (size_t)gg * slot_bytes);
+  }
+  if (g.coated_lanes == 1 && !ctx->mie_ckpt_set && ctx->tune_mie_waves == 0 &&
+      (n <= kCoatedLongMax || rows_cap >= kLongRows)) {
+    // the long series run first, on the same slots
+    g.coated_long = rows_cap <= 1200 ? 16 : 64;
+    const int64_t per_wave = 64 / g.coated_long;
+    int64_t gg = std::min<int64_t>((n + per_wave - 1) / per_wave,
+                                   (int64_t)ctx->n_cu * std::max(ctx->occ_coated_coop, 1));
+    g.coated_long_grid = std::min<int64_t>(gg, (int64_t)(budget / coop_slot(g.coated_long)));
+    if (g.coated_long_grid < 1) g.coated_long = 0;
+    else
+      g.stable.second =
+          std::max(g.stable.second, (size_t)g.coated_long_grid * coop_slot(g.coated_long));
   }
   return g;
 }
@@ -315,7 +340,8 @@ int mie_batch_run(gm_ctx* ctx, int64_t n, const double* x, const double* y, cons
                        ws.key, nmax_out, hist, ws.status, per);
     hipLaunchKernelGGL(gm::k_plan_scan, dim3(1), dim3(256), 0, s, hist, cursor, range,
                        (g.long_lcap ? kLongCost : gm::kSmallCost) >> gm::kBucketShift,
-                       g.long_lcap ? g.homog.first : (int64_t)0, ab);
+                       g.long_lcap ? g.homog.first : (int64_t)0, y ? g.coated_long : 0,
+                       ctx->n_cu * 4, ab);
     hipLaunchKernelGGL(gm::k_plan_scatter, dim3(pblk), dim3(256), 0, s, n,
                        (const int32_t*)ws.key, cursor, ws.order, per);
   } else {
@@ -375,6 +401,13 @@ int mie_batch_run(gm_ctx* ctx, int64_t n, const double* x, const double* y, cons
                : g.coated_lanes == 32 ? gm::k_mie_coated_coop<32>
                                       : gm::k_mie_coated_coop<64>;
       coated_cap = g.coated_lcap;
+    }
+    if (g.coated_long && (flags & GM_MIE_SORT)) {
+      auto lng = g.coated_long == 16 ? gm::k_mie_coated_coop<16> : gm::k_mie_coated_coop<64>;
+      hipLaunchKernelGGL(lng, dim3((unsigned)g.coated_long_grid), dim3(64), 0, s, order,
+                         range + gm::kCoatedLong, n, x, y, eps, mu, eps2, coef_off, an, bn, props,
+                         ws.status, ws.slots, (rows_cap + g.coated_long - 1) / g.coated_long,
+                         dn_extra);
     }
     hipLaunchKernelGGL(stable, dim3((unsigned)g.stable.first), dim3(64), 0, s, order, range, n, x,
                        y, eps, mu, eps2, coef_off, an, bn, props, ws.status, ws.slots, coated_cap,
@@ -633,7 +666,7 @@ int gm_mie_batch(gm_ctx* ctx, int64_t n, const double* x, const double* y, const
   const int nb = gm::kClasses * gm::kBuckets;
   if ((rc = ctx->reserve(ctx->order, sizeof(int64_t) * n))) return rc;
   if ((rc = ctx->reserve(ctx->key, sizeof(int32_t) * n))) return rc;
-  if ((rc = ctx->reserve(ctx->hist, sizeof(int64_t) * (2 * nb + gm::kQueueSlot + 1)))) return rc;
+  if ((rc = ctx->reserve(ctx->hist, sizeof(int64_t) * (2 * nb + gm::kPlanWords)))) return rc;
   MieWs ws;
   ws.order = (int64_t*)ctx->order.ptr;
   ws.key = (int32_t*)ctx->key.ptr;
@@ -671,7 +704,7 @@ int gm_mie_batch_noalloc(gm_ctx* ctx, int64_t n, const double* x, const double* 
   // layout of the static array: plan histogram/cursors/ranges, sort keys,
   // sorted order, then the recurrence slots in what is left
   const int nb = gm::kClasses * gm::kBuckets;
-  const size_t hist_bytes = sizeof(int64_t) * (2 * nb + gm::kQueueSlot + 1);
+  const size_t hist_bytes = sizeof(int64_t) * (2 * nb + gm::kPlanWords);
   auto up = [](size_t v) { return (v + 255) / 256 * 256; };
   const size_t plan_bytes = up(hist_bytes) + up(sizeof(int32_t) * (size_t)n) +
                             up(sizeof(int64_t) * (size_t)n);

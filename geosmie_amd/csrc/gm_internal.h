@@ -20,7 +20,7 @@ __global__ void k_plan_keys(int64_t n, const double* x, const double* y, const d
                             const double* mu, const double* eps2, int32_t* key,
                             int32_t* nmax_out, int64_t* hist, int32_t* status, int per);
 __global__ void k_plan_scan(const int64_t* hist, int64_t* cursor, int64_t* range, int small_b,
-                            int64_t slots, int64_t* ab);
+                            int64_t slots, int coated_lanes, int simds, int64_t* ab);
 __global__ void k_plan_scatter(int64_t n, const int32_t* key, int64_t* cursor, int64_t* order,
                                int per);
 __global__ void k_plan_identity(int64_t n, int64_t* order, int64_t* range, int64_t* ab);
@@ -31,6 +31,10 @@ constexpr int kSmallCost = 160;
 // homogeneous split ab[4], then one work-queue counter; kQueueSlot is the
 // counter's offset from range.
 constexpr int kQueueSlot = 2 * kClasses + 4;
+// The coated class's long series [begin, end) follow the counter;
+// range + kCoatedLong is the view of them as a coated class range (words 2, 3).
+constexpr int kCoatedLong = kQueueSlot - 1;
+constexpr int kPlanWords = kQueueSlot + 3;
 constexpr int kSmallLcap = 12;
 template <int MINW>
 __global__ void k_mie_homog(const int64_t* order, const int64_t* range, int64_t n_all,

@@ -177,11 +177,34 @@ __global__ __launch_bounds__(256) void k_plan_keys(
 // (the wavefronts of the lane-per-point kernel) raises the bound to the cost that
 // an even share of the batch puts on a lane of one of them: only points that would
 // keep a wavefront running after the others have finished are split over lanes.
+// coated_lanes > 0: the coated class is split too, at the bucket where the modelled
+// time is least (coated_split below); the long part goes to ab[5], ab[6] and the
+// class range keeps the rest.
+//
+// Time of the coated class, in steps of one lane's chain (about 0.19 us), when
+// the n_long points of summed cost w_long run with `lanes` lanes per point and the
+// rest, of largest cost c_rest, one per lane.  Each round of wavefronts of the
+// former takes 105 (its scans) and the chip works off 1.43 steps per cost
+// (measured: 20 us + 13 us at cost 1400 with 16 lanes, 20 us + 96 us at 5700; two
+// rounds 67 us); the latter takes its longest chain or 1.2 even shares of all
+// SIMDs' lanes, whichever is longer (84 us at c_rest = 284; 268 us at a share of
+// 1071, 2700 us at 12850).
+__device__ __forceinline__ float coated_split(float n_long, float w_long, float c_max, float c_rest,
+                                              float w_rest, int lanes, int simds) {
+  const float slots = 64.0f * (float)simds;
+  const float rest = w_rest > 0.0f ? 110.0f + fmaxf(c_rest, 1.2f * w_rest / slots) : 0.0f;
+  if (n_long == 0.0f) return rest;
+  return rest + 25.0f + 105.0f * ceilf(n_long * (float)lanes / slots) +
+         1.43f * fmaxf(c_max / (float)lanes, w_long / slots);
+}
 __global__ __launch_bounds__(256) void k_plan_scan(const int64_t* __restrict__ hist,
                                                    int64_t* __restrict__ cursor,
                                                    int64_t* __restrict__ range, int small_b,
-                                                   int64_t slots, int64_t* __restrict__ ab) {
+                                                   int64_t slots, int coated_lanes, int simds,
+                                                   int64_t* __restrict__ ab) {
   __shared__ int64_t part[256];
+  __shared__ int64_t part_n[256];
+  __shared__ unsigned long long best;
   constexpr int per = (kClasses * kBuckets) / 256;
   static_assert(per * 256 == kClasses * kBuckets, "histogram must split into 256 runs");
   const int t = threadIdx.x;
@@ -231,6 +254,66 @@ __global__ __launch_bounds__(256) void k_plan_scan(const int64_t* __restrict__ h
     const int64_t share = part[0] / (64 * slots);
     if (share > small_b) small_b = (int)min(share, (int64_t)kBuckets);
   }
+  if (coated_lanes > 0) {
+    // prefix sums of the coated class's counts and costs, longest first; every
+    // thread prices its buckets as the first of the rest
+    auto bucket = [&](int i) { return 2 * kBuckets - 1 - (t * per + i); };   // cost >> shift
+    int64_t cn = 0, cw = 0;
+    int c_max = 0;
+    if (t == 0) best = ~0ull;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < per; ++i) {
+      const int b = bucket(i);
+      if (b >= 0 && b < kBuckets && h[i] > 0) {
+        cn += h[i];
+        cw += h[i] * (int64_t)b;
+        c_max = max(c_max, b);
+      }
+    }
+    part[t] = cw;
+    part_n[t] = cn;
+    __syncthreads();
+    for (int off = 1; off < 256; off <<= 1) {
+      const int64_t v = t >= off ? part[t - off] : 0, w = t >= off ? part_n[t - off] : 0;
+      __syncthreads();
+      part[t] += v;
+      part_n[t] += w;
+      __syncthreads();
+    }
+    const int64_t w_all = part[255], n_all = part_n[255];
+    // the highest bucket in use, of any thread
+    __shared__ int wave_max[4];
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) c_max = max(c_max, __shfl_xor(c_max, d));
+    if (t % 64 == 0) wave_max[t / 64] = c_max;
+    __syncthreads();
+    c_max = max(max(wave_max[0], wave_max[1]), max(wave_max[2], wave_max[3]));
+    unsigned long long mine = ~0ull;
+    constexpr float unit = (float)(1 << kBucketShift);
+    if (t == 0 && n_all > 0)   // every point split
+      mine = ((unsigned long long)__float_as_uint(
+                  coated_split((float)n_all, unit * (float)w_all, unit * (float)c_max, 0.0f, 0.0f,
+                               coated_lanes, simds)) << 32) | (unsigned)n_all;
+    cw = part[t] - cw;
+    cn = part_n[t] - cn;
+#pragma unroll
+    for (int i = 0; i < per; ++i) {
+      const int b = bucket(i);
+      if (b >= 0 && b < kBuckets && h[i] > 0) {
+        const float time = coated_split((float)cn, unit * (float)cw, unit * (float)c_max,
+                                        unit * (float)b, unit * (float)(w_all - cw), coated_lanes,
+                                        simds);
+        // the smallest time, then the fewest long points (counts fit 32 bits)
+        mine = min(mine, ((unsigned long long)__float_as_uint(time) << 32) | (unsigned)cn);
+        cn += h[i];
+        cw += h[i] * (int64_t)b;
+      }
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) mine = min(mine, (unsigned long long)__shfl_xor(mine, d));
+    if (t % 64 == 0) atomicMin(&best, mine);
+  }
   __syncthreads();
   if (t == 0 && ab) {
     const int key = kBuckets - min(max(small_b, 0), kBuckets);   // class 0's first small key
@@ -240,6 +323,11 @@ __global__ __launch_bounds__(256) void k_plan_scan(const int64_t* __restrict__ h
     ab[2] = split;
     ab[3] = range[1];
     ab[4] = 0;   // the coated class's work queue (kQueueSlot)
+    ab[5] = ab[6] = range[2];
+    if (coated_lanes > 0 && best != ~0ull) {
+      ab[6] += (int64_t)(best & 0xffffffffull);
+      range[2] = ab[6];
+    }
   }
 }
 

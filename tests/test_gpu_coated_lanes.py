@@ -134,3 +134,29 @@ def test_lanes_per_point(gpu, n, y_hi, q_lo, sort):
                                            + b * np.append(b[1:], 0).conj()).real).sum())
         assert abs(props[0, i] - ext) <= 2e-9 * ext and abs(props[1, i] - sca) <= 2e-9 * sca, i
         assert abs(props[4, i] - 4 * asy / (sca * y[i] ** 2)) <= 2e-9, i
+
+
+# above 24576 points one per lane: the split of the longest (skewed sizes), of every
+# point (uniform long series) and of none (uniform short ones)
+@pytest.mark.parametrize("y_lo, y_hi, skew", [(0.02, 209.0, True), (600.0, 700.0, False),
+                                              (1.0, 20.0, False)])
+def test_long_points_of_a_batch(gpu, y_lo, y_hi, skew):
+    import torch
+    from geosmie_amd import _lib
+    from geosmie_amd.autotune import set_knob
+    n = 24576 + 1
+    rng = np.random.default_rng(int(y_hi))
+    y = (np.exp(rng.uniform(np.log(y_lo), np.log(y_hi), n)) if skew
+         else rng.uniform(y_lo, y_hi, n))
+    x = y * rng.uniform(0.3, 0.9, n)
+    m1, m2 = np.full(n, 1.95 + 0.79j), np.full(n, 1.4 + 0j)
+    x[5::500] = y[5::500]
+    h, ref = _lib.private_ctx(), _lib.private_ctx()
+    set_knob(ref, "mie_ckpt", 4)
+    got, want = _run(h, x, y, m1, m2, True), _run(ref, x, y, m1, m2, True)
+    # an absorbing core needs no start correction: both forms hold 1e-9
+    for a, b in zip(got[:2], want[:2]):
+        assert torch.equal(torch.isnan(a), torch.isnan(b))
+        assert float(torch.nan_to_num(a - b).abs().max()) <= 2e-9
+    for q in (0, 1, 4):
+        assert float(((got[2][q] - want[2][q]) / want[2][q]).abs().max()) <= 2e-9, q
