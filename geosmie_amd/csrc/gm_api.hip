@@ -148,8 +148,9 @@ struct MieGrids {
 // nmx + 2 n_max, about 300 rows) and more than a lane's even share of the batch
 // (k_plan_scan) take a wavefront each.  One point per lane walks its rows serially, so a
 // point of x = 3400 held its wavefront for the whole 3.0 ms of a 1.2M-point LUT
-// batch whose CUs were 46% busy.  That batch: 2.97 ms serial; 2.35 with 16 lanes
-// for the long points, 2.25 with 32, 2.15 with 64, bounds of 1024 and 2048 alike.
+// batch whose CUs were 46% busy.  Those recurrences: 2.97 ms serial, 2.35 split; the
+// whole call of 400 slabs 10.41 ms with 16 lanes for the long points, 10.2 with
+// 32, 10.07 with 64, bounds of 1024 and 2048 alike.
 // Splitting points over lanes costs about twice the instructions: 300k points of x
 // uniform in 1..1500, where it saves no tail, took 2.9 ms serial and 3.6 with a
 // bound of half the share.

@@ -885,11 +885,10 @@ __device__ __forceinline__ void rows_lp_epilogue(const float4_ (&accp)[MT][4],
   }
 }
 
-// S1/S2 of 8 MT points x 64 angles per wavefront on the FP32 or split-BF16
-// matrix cores (operands as in k_s12_f32 / k_s12_bf16x3, coefficients from
-// k_s12_split_coef), then the Mueller elements and their weighted row sums
-// in FP64 as k_s12_rows_f64 forms them; same partial buffer and reduction
-// (k_s12_rows_reduce).  A chunk is one group of MT 8-point tiles: each
+// S1/S2 of 8 MT points x 64 angles per wavefront on the split-BF16 matrix
+// cores (operands as in k_s12_bf16x3, coefficients from k_s12_split_coef),
+// then the Mueller elements and their weighted row sums in FP64; same partial
+// buffer and reduction as k_s12_rows (k_s12_rows_reduce).  A chunk is one group of MT 8-point tiles: each
 // angle-table word fetched feeds the products of all MT tiles, and the row
 // sums are formed once, after the K loop, so they hold no registers while
 // it runs.
