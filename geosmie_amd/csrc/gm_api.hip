@@ -138,7 +138,8 @@ struct MieGrids {
   int coated_lcap = 0;      // rows per lane segment (coated_lanes > 1)
   int coated_long = 0;      // coated_lanes = 1: lanes per point of the long series (0: none)
   int64_t coated_long_grid = 0;
-  int64_t small_grid = 0;   // grid of the 4-lane kernel for the short series (lanes > 1)
+  int64_t mid_grid = 0;     // blocks of the 16-lane part for the middle series (lanes > 16)
+  int64_t small_grid = 0;   // blocks of the 4-lane part for the short series (lanes > 1)
   int long_lcap = 0;        // lanes = 1: rows per lane of the long series' kernel (0: none)
   int64_t long_grid = 0;
 };
@@ -244,13 +245,31 @@ MieGrids mie_grids(const gm_ctx* ctx, int64_t n, int rows_cap, size_t budget) {
     int64_t gg = std::min<int64_t>((n + per_wave - 1) / per_wave,
                                    (int64_t)ctx->n_cu * std::max(ctx->occ_coop, 1) *
                                        std::max(ctx->tune_mie_grid_mult, 1));
-    gg = std::min<int64_t>(gg, std::max<int64_t>(1, (int64_t)(budget / slot_bytes)));
-    // the 4-lane kernel of the short series runs after it on the same slots
+    // three parts in one launch, each on slots of its own
+    auto fit = [&](int64_t blocks, size_t bytes) {
+      return std::min<int64_t>(blocks, std::max<int64_t>(1, (int64_t)(budget / 3 / bytes)));
+    };
+    const int64_t resident = (int64_t)ctx->n_cu * std::max(ctx->occ_coop, 1);
+    gg = fit(gg, slot_bytes);
+    const size_t mid_slot = (size_t)gm::kMidLcap * 64 * gm::kHomogRowDoubles * sizeof(double);
+    // Middle series apart: where 64 lanes hold less than four of their rows each and the
+    // batch is several rounds of wavefronts (40k points to x = 2094: Mie 319 us with
+    // two launches, 291 two parts in one, 249 with the middle part at cost 640, 258 at
+    // 320, 255 at 1024; 20k points to x = 417 run 32 lanes and gain nothing, 136 us
+    // a step against 141).
+    if (g.lanes == 64 && !ctx->tune_mie_lanes && n >= 4 * resident) {
+      const int64_t per = 64 / gm::kMidLanes;
+      g.mid_grid = fit(std::min<int64_t>((n + per - 1) / per, resident), mid_slot);
+    }
     const size_t small_slot = (size_t)gm::kSmallLcap * 64 * gm::kHomogRowDoubles * sizeof(double);
-    int64_t gsm = std::min<int64_t>((n + 15) / 16, (int64_t)ctx->n_cu * std::max(ctx->occ_coop, 1));
-    gsm = std::max<int64_t>(1, std::min<int64_t>(gsm, (int64_t)(budget / small_slot)));
-    g.small_grid = gsm;
-    g.homog = std::make_pair(gg, std::max((size_t)gg * slot_bytes, (size_t)gsm * small_slot));
+    g.small_grid = fit(std::min<int64_t>((n + 15) / 16, resident), small_slot);
+    size_t bytes = (size_t)gg * slot_bytes + (size_t)g.mid_grid * mid_slot +
+                   (size_t)g.small_grid * small_slot;
+    if (bytes > budget) {   // no room for a slot of each: all points with many lanes
+      g.mid_grid = g.small_grid = 0;
+      bytes = (size_t)gg * slot_bytes;
+    }
+    g.homog = std::make_pair(gg, bytes);
   }
   g.literal = grid_for(ctx->occ_literal, gm::kCoatedRowDoubles);
   const int ck = ctx->tune_mie_ckpt;
@@ -341,6 +360,7 @@ int mie_batch_run(gm_ctx* ctx, int64_t n, const double* x, const double* y, cons
                        ws.key, nmax_out, hist, ws.status, per);
     hipLaunchKernelGGL(gm::k_plan_scan, dim3(1), dim3(256), 0, s, hist, cursor, range,
                        (g.long_lcap ? kLongCost : gm::kSmallCost) >> gm::kBucketShift,
+                       g.mid_grid ? gm::kMidCost >> gm::kBucketShift : 0,
                        g.long_lcap ? g.homog.first : (int64_t)0, y ? g.coated_long : 0,
                        ctx->n_cu * 4, ab);
     hipLaunchKernelGGL(gm::k_plan_scatter, dim3(pblk), dim3(256), 0, s, n,
@@ -365,8 +385,7 @@ int mie_batch_run(gm_ctx* ctx, int64_t n, const double* x, const double* y, cons
   if (g.lanes > 1) {
     homog = g.lanes == 16 ? gm::k_mie_homog_coop<16>
             : g.lanes == 32 ? gm::k_mie_homog_coop<32> : gm::k_mie_homog_coop<64>;
-    cap_arg = g.lcap;
-    hrange = ab;
+    cap_arg = g.lcap;   // all points, unless the parts below take them
   }
   if (g.long_lcap && (flags & GM_MIE_SORT)) {
     hipLaunchKernelGGL(gm::k_mie_homog_coop<kLongLanes>, dim3((unsigned)g.long_grid), dim3(64), 0,
@@ -374,14 +393,16 @@ int mie_batch_run(gm_ctx* ctx, int64_t n, const double* x, const double* y, cons
                        ws.slots, g.long_lcap, dn_extra);
     hrange = ab + 2;
   }
-  hipLaunchKernelGGL(homog, dim3((unsigned)g.homog.first), dim3(64), 0, s, order, hrange, n, x, y,
-                     eps, mu, eps2, coef_off, an, bn, props, ws.status, ws.slots, cap_arg,
-                     dn_extra);
-  if (g.lanes > 1 && (flags & GM_MIE_SORT)) {
-    // the short series (sorted last): 4 lanes per point, 16 points per wavefront
-    hipLaunchKernelGGL(gm::k_mie_homog_coop<4>, dim3((unsigned)g.small_grid), dim3(64), 0, s,
-                       order, ab + 2, n, x, y, eps, mu, eps2, coef_off, an, bn, props, ws.status,
-                       ws.slots, gm::kSmallLcap, dn_extra);
+  if (g.small_grid && (flags & GM_MIE_SORT)) {
+    auto tiers = g.lanes == 16   ? gm::k_mie_homog_tiers<16>
+                 : g.lanes == 32 ? gm::k_mie_homog_tiers<32> : gm::k_mie_homog_tiers<64>;
+    hipLaunchKernelGGL(tiers, dim3((unsigned)(g.homog.first + g.mid_grid + g.small_grid)), dim3(64),
+                       0, s, order, ab, n, x, y, eps, mu, eps2, coef_off, an, bn, props, ws.status,
+                       ws.slots, cap_arg, dn_extra, (int)g.homog.first, (int)g.mid_grid);
+  } else {
+    hipLaunchKernelGGL(homog, dim3((unsigned)g.homog.first), dim3(64), 0, s, order, hrange, n, x,
+                       y, eps, mu, eps2, coef_off, an, bn, props, ws.status, ws.slots, cap_arg,
+                       dn_extra);
   }
   ctx->mark_end(slot, s);
   HIP_OK(hipGetLastError());

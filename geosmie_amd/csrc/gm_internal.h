@@ -19,7 +19,7 @@ __global__ void k_zero_i32(int32_t* p, int n);
 __global__ void k_plan_keys(int64_t n, const double* x, const double* y, const double* eps,
                             const double* mu, const double* eps2, int32_t* key,
                             int32_t* nmax_out, int64_t* hist, int32_t* status, int per);
-__global__ void k_plan_scan(const int64_t* hist, int64_t* cursor, int64_t* range, int small_b,
+__global__ void k_plan_scan(const int64_t* hist, int64_t* cursor, int64_t* range, int small_b, int mid_b,
                             int64_t slots, int coated_lanes, int simds, int64_t* ab);
 __global__ void k_plan_scatter(int64_t n, const int32_t* key, int64_t* cursor, int64_t* order,
                                int per);
@@ -36,6 +36,16 @@ constexpr int kQueueSlot = 2 * kClasses + 4;
 constexpr int kCoatedLong = kQueueSlot - 1;
 constexpr int kPlanWords = kQueueSlot + 3;
 constexpr int kSmallLcap = 12;
+// those of cost below this 16 lanes per point (3 n_max + 16 <= cost)
+constexpr int kMidCost = 640;
+constexpr int kMidLanes = 16;
+constexpr int kMidLcap = (kMidCost / 3 + kMidLanes - 1) / kMidLanes;
+template <int P>
+__global__ void k_mie_homog_tiers(const int64_t* order, const int64_t* ab, int64_t n_all,
+                                  const double* x, const double* y, const double* eps,
+                                  const double* mu, const double* eps2, const int64_t* coef_off,
+                                  double* an, double* bn, double* props, int32_t* status,
+                                  double* scratch, int lcap, int dn_extra, int g_big, int g_mid);
 template <int MINW>
 __global__ void k_mie_homog(const int64_t* order, const int64_t* range, int64_t n_all,
                             const double* x, const double* y, const double* eps, const double* mu,

@@ -171,9 +171,10 @@ __global__ __launch_bounds__(256) void k_plan_keys(
 // Each thread sums its run of buckets, the 256 run sums are scanned in LDS
 // (Hillis-Steele, 8 steps), then each thread writes its run's cursors and the
 // class boundaries that fall in it.
-// Also splits the homogeneous class at the first bucket of cost below
-// small_b (buckets descend along the order): ab = {begin, split, split, end},
-// the points run with many lanes per point and those run with few.  slots > 0
+// Also splits the homogeneous class at the first buckets of cost below mid_b and
+// small_b (buckets descend along the order): ab = {begin, mid, small, end}, the
+// points run with many lanes per point, those run with kMidLanes (none if mid_b <=
+// small_b) and those run with few.  slots > 0
 // (the wavefronts of the lane-per-point kernel) raises the bound to the cost that
 // an even share of the batch puts on a lane of one of them: only points that would
 // keep a wavefront running after the others have finished are split over lanes.
@@ -200,6 +201,7 @@ __device__ __forceinline__ float coated_split(float n_long, float w_long, float 
 __global__ __launch_bounds__(256) void k_plan_scan(const int64_t* __restrict__ hist,
                                                    int64_t* __restrict__ cursor,
                                                    int64_t* __restrict__ range, int small_b,
+                                                   int mid_b,
                                                    int64_t slots, int coated_lanes, int simds,
                                                    int64_t* __restrict__ ab) {
   __shared__ int64_t part[256];
@@ -318,8 +320,9 @@ __global__ __launch_bounds__(256) void k_plan_scan(const int64_t* __restrict__ h
   if (t == 0 && ab) {
     const int key = kBuckets - min(max(small_b, 0), kBuckets);   // class 0's first small key
     const int64_t split = key < kBuckets ? cursor[key] : range[1];
+    const int mid = kBuckets - min(max(mid_b, 0), kBuckets);   // class 0's first middle key
     ab[0] = range[0];
-    ab[1] = split;
+    ab[1] = mid_b <= small_b ? split : mid < kBuckets ? cursor[mid] : range[1];
     ab[2] = split;
     ab[3] = range[1];
     ab[4] = 0;   // the coated class's work queue (kQueueSlot)
@@ -877,24 +880,23 @@ __device__ __forceinline__ double grp_sum(double v) {
   return v;
 }
 
+// The points order[begin .. end) on `blocks` blocks, this one `block`, its rows in `slot`.
 template <int P>
-__global__ __launch_bounds__(64) void k_mie_homog_coop(
-    const int64_t* __restrict__ order, const int64_t* __restrict__ range, int64_t n_all,
-    const double* __restrict__ x, const double* __restrict__ y, const double* __restrict__ eps,
-    const double* __restrict__ mu, const double* __restrict__ eps2,
-    const int64_t* __restrict__ coef_off, double* __restrict__ an, double* __restrict__ bn,
-    double* __restrict__ props, int32_t* __restrict__ status, double* __restrict__ scratch,
-    int lcap, int dn_extra) {
+__device__ __forceinline__ void homog_coop(
+    const int64_t* __restrict__ order, int64_t begin, int64_t end, int64_t block, int64_t blocks,
+    int64_t n_all, const double* __restrict__ x, const double* __restrict__ y,
+    const double* __restrict__ eps, const double* __restrict__ mu,
+    const double* __restrict__ eps2, const int64_t* __restrict__ coef_off,
+    double* __restrict__ an, double* __restrict__ bn, double* __restrict__ props,
+    int32_t* __restrict__ status, double* __restrict__ slot, int lcap, int dn_extra) {
   constexpr int W = 64 / P;
   const int lane = threadIdx.x;
   const int j = lane % P, grp = lane / P;
-  const int64_t begin = range[0], end = range[1];
-  double* slot = scratch + (size_t)blockIdx.x * (size_t)lcap * 64 * 3;
   cd* Ds = reinterpret_cast<cd*>(slot);            // [row in segment][lane]
   double* Rs = slot + (size_t)lcap * 64 * 2;       // [row in segment][lane]
 
-  for (int64_t base = begin + (int64_t)blockIdx.x * W; base < end;
-       base += (int64_t)gridDim.x * W) {
+  for (int64_t base = begin + block * W; base < end;
+       base += blocks * W) {
     const int64_t idx = base + grp;
     if (idx >= end) continue;                      // the whole group: no shuffle partners lost
     const int64_t p = order[idx];
@@ -1105,6 +1107,54 @@ __global__ __launch_bounds__(64) void k_mie_homog_coop(
       props[5 * n_all + p] = qbv / qsca;
     }
   }
+}
+
+template <int P>
+__global__ __launch_bounds__(64) void k_mie_homog_coop(
+    const int64_t* __restrict__ order, const int64_t* __restrict__ range, int64_t n_all,
+    const double* __restrict__ x, const double* __restrict__ y, const double* __restrict__ eps,
+    const double* __restrict__ mu, const double* __restrict__ eps2,
+    const int64_t* __restrict__ coef_off, double* __restrict__ an, double* __restrict__ bn,
+    double* __restrict__ props, int32_t* __restrict__ status, double* __restrict__ scratch,
+    int lcap, int dn_extra) {
+  homog_coop<P>(order, range[0], range[1], blockIdx.x, gridDim.x, n_all, x, y, eps, mu, eps2,
+                coef_off, an, bn, props, status,
+                scratch + (size_t)blockIdx.x * (size_t)lcap * 64 * 3, lcap, dn_extra);
+}
+
+// A sorted batch's series in one launch: the longest with P lanes per point on the
+// first g_big blocks, the middle ones with kMidLanes on the next g_mid, the short
+// ones with 4 on the rest.  Each part is bound by its longest wavefronts, 20 to 30
+// us for a few thousand points however short, so launched one after the other they
+// add up: 20k points to x = 417 took 30 + 24 us, a captured step of them 158 us
+// against 136 in one launch.
+template <int P>
+__global__ __launch_bounds__(64) void k_mie_homog_tiers(
+    const int64_t* __restrict__ order, const int64_t* __restrict__ ab, int64_t n_all,
+    const double* __restrict__ x, const double* __restrict__ y, const double* __restrict__ eps,
+    const double* __restrict__ mu, const double* __restrict__ eps2,
+    const int64_t* __restrict__ coef_off, double* __restrict__ an, double* __restrict__ bn,
+    double* __restrict__ props, int32_t* __restrict__ status, double* __restrict__ scratch,
+    int lcap, int dn_extra, int g_big, int g_mid) {
+  const int b = blockIdx.x;
+  if (b < g_big) {
+    homog_coop<P>(order, ab[0], ab[1], b, g_big, n_all, x, y, eps, mu, eps2, coef_off, an, bn,
+                  props, status, scratch + (size_t)b * (size_t)lcap * 64 * 3, lcap, dn_extra);
+    return;
+  }
+  scratch += (size_t)g_big * (size_t)lcap * 64 * 3;
+  if (b < g_big + g_mid) {
+    homog_coop<kMidLanes>(order, ab[1], ab[2], b - g_big, g_mid, n_all, x, y, eps, mu, eps2,
+                          coef_off, an, bn, props, status,
+                          scratch + (size_t)(b - g_big) * (size_t)kMidLcap * 64 * 3, kMidLcap,
+                          dn_extra);
+    return;
+  }
+  scratch += (size_t)g_mid * (size_t)kMidLcap * 64 * 3;
+  const int c = b - g_big - g_mid;
+  homog_coop<4>(order, ab[2], ab[3], c, (int)gridDim.x - g_big - g_mid, n_all, x, y, eps, mu, eps2,
+                coef_off, an, bn, props, status, scratch + (size_t)c * (size_t)kSmallLcap * 64 * 3,
+                kSmallLcap, dn_extra);
 }
 
 // ---------------------------------------------------------------------------
@@ -2277,7 +2327,9 @@ template __global__ void k_mie_coated_ckpt<1, 4>(GM_MIE_ARGS);
 template __global__ void k_mie_coated_ckpt<3, 4>(GM_MIE_ARGS);
 template __global__ void k_mie_coated_ckpt<1, 5>(GM_MIE_ARGS);
 template __global__ void k_mie_coated_ckpt<1, 8>(GM_MIE_ARGS);
-template __global__ void k_mie_homog_coop<4>(GM_MIE_ARGS);
+template __global__ void k_mie_homog_tiers<16>(GM_MIE_ARGS, int, int);
+template __global__ void k_mie_homog_tiers<32>(GM_MIE_ARGS, int, int);
+template __global__ void k_mie_homog_tiers<64>(GM_MIE_ARGS, int, int);
 template __global__ void k_mie_homog_coop<16>(GM_MIE_ARGS);
 template __global__ void k_mie_homog_coop<32>(GM_MIE_ARGS);
 template __global__ void k_mie_homog_coop<64>(GM_MIE_ARGS);
