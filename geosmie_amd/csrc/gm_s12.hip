@@ -311,8 +311,8 @@ __global__ __launch_bounds__(256) void k_s12_unit_order(int64_t units,
 // Element r of lane (i, g) is point p0 + 4 g + r.  LP: the coefficients come from
 // gm_s12_split_coef, 16 bytes {U.re, V.re, U.im, V.im} a term.  Tiles of 8 points and
 // 64 angles spent 8 8-byte or 4-byte loads and two coefficient loads on 8 MFMAs of
-// half the FP64 length: 40k points x 1801 angles with row sums 1.51 -> 1.02 ms, P11
-// of 1.5M points x 371 angles 6.2 -> 4.6 ms.
+// half the FP64 length: 40k points x 1801 angles with row sums 1.61 -> 1.09 ms; a LUT
+// call of 512 queries, half of it this kernel, 12.0 -> 10.5 ms.
 template <int TT, bool LP, int kCd>
 __device__ __forceinline__ void s12_tile32(const S12Tables& T, int64_t p0, int64_t pend, int j0,
                                            int lane, const int64_t* __restrict__ off,
@@ -1172,7 +1172,8 @@ namespace {
 // (20k points x 181 angles: 158 us a step with 16 angles each, 183 at 32, 213 at
 // 64; 40k x 1801 the same time from 2k to 16k), tiles from which the pairing pass
 // pays (8 to 13 us; 40k points x 1801 angles 3.25 against 3.61 ms, 1.2M x 371
-// 13.7 against 14.5; below 256 tiles the launch costs more than it saves), and the
+// 13.7 against 14.5; 20k points x 181 angles, 1250 tiles, 183 against 186: the line
+// lies where that gain no longer pays the launch), and the
 // table rows from which units are sorted by length (1.2M points, n_max to 3400:
 // 11.60 against 11.86 ms; 20k points, n_max to 449: 178 us against 168 unsorted).
 constexpr int64_t kS12Want = 8192;
