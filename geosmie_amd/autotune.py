@@ -14,10 +14,11 @@ Knobs (include/geosmie.h, enum gm_tune_param):
   mie_waves      register budget of the Mie recurrence kernels (0 unconstrained,
                  3 or 4 resident wavefronts per SIMD)
   s12_layout     kept for saved settings; no effect
-  mie_ckpt       coated kernel: downward-chain states kept every 4, 5 or 8 rows and
+  mie_ckpt       coated kernel, one point per lane: downward-chain states kept every 4, 5 or 8 rows and
                  regenerated per block in LDS, or every row kept in scratch (0);
                  non-zero also selects the checkpointed lane-per-point
                  homogeneous kernel (every 4 rows)
+  coated_lanes   coated kernel: lanes per point, as mie_lanes
   mie_lanes      homogeneous kernel: lanes per point (1, or 16/32/64 with the serial
                  recurrences joined by parallel scans; 0 = chosen by batch)
   s12_row_tiles  fused S1/S2 row sums: tiles per work unit (0 = by batch)
@@ -44,6 +45,7 @@ KNOBS = {"mie_grid_mult": (0, (1, 2, 4)),
          "mie_lanes": (8, (0, 1, 16, 32, 64)),
          "s12_row_tiles": (10, (0, 1, 2, 4)),
          "s12_share": (11, (1, 0)),
+         "coated_lanes": (12, (0, 1, 16, 32, 64)),
          # a precision setting rather than a shape; set explicitly, never tuned for speed
          "mlp_weight_terms": (3, (1, 2)),
          # a behaviour setting: the integratePSD quirks reproduced (bit 0: the aliased

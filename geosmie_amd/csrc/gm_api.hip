@@ -186,10 +186,11 @@ int mie_lanes(const gm_ctx* ctx, int64_t n, int rows_cap) {
 // 281 / 59 / 51 / 48, 2048 points 282 / 64 / 55 / 76, 8192 points 278 / 106, 24576
 // points 289 / 245, 32768 points 295 / 318; y in 800..1000: 24576 points 1217 / 745.
 // Short series gain less (y in 1..20: 2048 points 68 / 46, 8192 points 68 / 72),
-// so the bound falls with the series length.  A caller who sets the checkpoint
-// knob or a register budget chooses among the lane-per-point forms.
+// so the bound falls with the series length.  A register budget chooses among the
+// lane-per-point forms.
 int coated_lanes(const gm_ctx* ctx, int64_t n, int rows_cap) {
-  if (ctx->mie_ckpt_set || ctx->tune_mie_waves != 0) return 1;
+  if (ctx->tune_coated_lanes) return ctx->tune_coated_lanes;
+  if (ctx->tune_mie_waves != 0) return 1;
   if (n > (int64_t)ctx->n_cu * std::min(96, std::max(24, rows_cap / 2))) return 1;
   return n <= (int64_t)ctx->n_cu * 4 ? 64 : n <= (int64_t)ctx->n_cu * 8 ? 32 : 16;
 }
@@ -300,7 +301,7 @@ MieGrids mie_grids(const gm_ctx* ctx, int64_t n, int rows_cap, size_t budget) {
     gg = std::min<int64_t>(gg, std::max<int64_t>(1, (int64_t)(budget / slot_bytes)));
     g.stable = std::make_pair(gg, (size_t)gg * slot_bytes);
   }
-  if (g.coated_lanes == 1 && !ctx->mie_ckpt_set && ctx->tune_mie_waves == 0 &&
+  if (g.coated_lanes == 1 && !ctx->tune_coated_lanes && ctx->tune_mie_waves == 0 &&
       (n <= kCoatedLongMax || rows_cap >= kLongRows)) {
     // the long series run first, on the same slots
     g.coated_long = rows_cap <= 1200 ? 16 : 64;
@@ -578,12 +579,16 @@ int gm_ctx_tune(gm_ctx* ctx, int param, int value) {
       if (value != 0 && value != 4 && value != 5 && value != 8)
         return gm_fail(GM_EINVAL, "gm_ctx_tune: rows per checkpoint must be 0, 4, 5 or 8");
       ctx->tune_mie_ckpt = value;
-      ctx->mie_ckpt_set = true;
       return GM_OK;
     case GM_TUNE_MIE_LANES:
       if (value != 0 && value != 1 && value != 16 && value != 32 && value != 64)
         return gm_fail(GM_EINVAL, "gm_ctx_tune: lanes per point must be 0, 1, 16, 32 or 64");
       ctx->tune_mie_lanes = value;
+      return GM_OK;
+    case GM_TUNE_COATED_LANES:
+      if (value != 0 && value != 1 && value != 16 && value != 32 && value != 64)
+        return gm_fail(GM_EINVAL, "gm_ctx_tune: lanes per coated point must be 0, 1, 16, 32 or 64");
+      ctx->tune_coated_lanes = value;
       return GM_OK;
     case GM_TUNE_S12_ROW_TILES:
       if (value != 0 && value != 1 && value != 2 && value != 4)
@@ -622,6 +627,7 @@ int gm_ctx_get_tune(gm_ctx* ctx, int param, int* value) {
     case GM_TUNE_S12_LAYOUT: *value = ctx->tune_s12_layout; return GM_OK;
     case GM_TUNE_MIE_CKPT: *value = ctx->tune_mie_ckpt; return GM_OK;
     case GM_TUNE_MIE_LANES: *value = ctx->tune_mie_lanes; return GM_OK;
+    case GM_TUNE_COATED_LANES: *value = ctx->tune_coated_lanes; return GM_OK;
     case GM_TUNE_PSD_QUIRKS: *value = ctx->psd_quirks; return GM_OK;
     case GM_TUNE_S12_ROW_TILES: *value = ctx->tune_s12_row_tiles; return GM_OK;
     case GM_TUNE_S12_SHARE: *value = ctx->tune_s12_share; return GM_OK;

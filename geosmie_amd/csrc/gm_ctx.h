@@ -38,9 +38,9 @@ struct gm_ctx {
   int tune_mlp_wterms = 1;      // BF16 terms per MLP weight (1 = BF16 weights, 2 = hi + lo)
   int tune_mie_waves = 0;       // Mie register variant: 0 unconstrained, 3 or 4 waves per SIMD
   int tune_s12_layout = 0;      // accepted, no effect
-  int tune_mie_ckpt = 4;        // coated kernel: rows per checkpoint (4, 8) or 0 = every row stored
-  bool mie_ckpt_set = false;    // tune_mie_ckpt chosen by the caller: one coated point per lane
+  int tune_mie_ckpt = 4;        // coated kernel: rows per checkpoint (4, 5, 8) or 0 = every row stored
   int tune_mie_lanes = 0;       // homogeneous kernel: lanes per point (1, 16, 32, 64; 0 = by batch)
+  int tune_coated_lanes = 0;    // coated kernel: lanes per point (1, 16, 32, 64; 0 = by batch)
   int psd_quirks = 1;           // integratePSD quirks reproduced (GM_PSD_QUIRK_* bits)
   int tune_s12_share = 1;        // split-BF16 fused S1/S2: angle-table tiles shared through LDS
   int tune_s12_row_tiles = 0;    // reduced-precision fused S1/S2: 8-point tiles per wave (0 = auto)

@@ -100,10 +100,9 @@ enum gm_tune_param {
   GM_TUNE_MIE_CKPT = 7          /* coated kernel (real / weakly absorbing shells): the downward
                                    chains' states kept every 4, 5 or 8 rows and each block of rows
                                    regenerated in LDS before use (4, the default), or 0 = every
-                                   row kept in scratch; results agree to rounding.  Once set, every
-                                   batch runs one coated point per lane; unset, small batches split
-                                   each point's rows over 16, 32 or 64 lanes.  Non-zero also
-                                   selects the checkpointed one-point-per-lane homogeneous kernel
+                                   row kept in scratch; results agree to rounding.  It acts where
+                                   one coated point runs per lane (GM_TUNE_COATED_LANES).  Non-zero
+                                   also selects the checkpointed one-point-per-lane homogeneous kernel
                                    (every 4 rows, unless GM_TUNE_MIE_WAVES forces a register
                                    budget; bit-identical results) */,
   GM_TUNE_MIE_LANES = 8         /* homogeneous kernel: lanes per point.  1 = one point per lane
@@ -122,7 +121,13 @@ enum gm_tune_param {
   GM_TUNE_S12_SHARE = 11        /* gm_s12_contract_rows at split-BF16 with one tile per work
                                    unit: 1 (default) = four work units per block share each
                                    K-step's angle-table tile through LDS; 0 = each wavefront
-                                   fetches its own.  Identical results */
+                                   fetches its own.  Identical results */,
+  GM_TUNE_COATED_LANES = 12     /* coated kernel: lanes per point.  1 = one point per lane; 16, 32,
+                                   64 = each point's rows split over that many lanes; 0 (default) =
+                                   chosen from the batch size and series length, the longest
+                                   points of a batch that runs one per lane split where that is
+                                   faster (with a GM_TUNE_MIE_WAVES budget: 1).  Results agree to
+                                   rounding */
 };
 int gm_ctx_tune(gm_ctx* ctx, int param, int value);
 int gm_ctx_get_tune(gm_ctx* ctx, int param, int* value);

@@ -53,6 +53,7 @@ def test_mie_register_variants_agree(gpu):
     x = y * r.uniform(0.3, 0.9, y.size)
     xs = np.logspace(-2, 3, 2000)
     ref = None
+    autotune.set_knob(h, "coated_lanes", 1)
     for waves in (0, 3, 4):
         autotune.set_knob(h, "mie_waves", waves)
         c = mie_batch(x, m=1.95 + 0.79j, y=y, m2=1.45 + 0j, coeffs=True)
@@ -70,6 +71,7 @@ def test_mie_register_variants_agree(gpu):
                 else:
                     assert np.all(np.abs(a - b) <= 1e-9 * np.abs(a)), waves
     autotune.set_knob(h, "mie_waves", 0)
+    autotune.set_knob(h, "coated_lanes", 0)
 
 
 def test_tune_picks_a_candidate(gpu):
@@ -105,11 +107,13 @@ def test_coated_checkpoint_variants_agree(gpu):
     m2 = np.where(m1.real > 1.5, 1.45 + 0j, 1.5 + 1e-3j)
     res = {}
     try:
+        autotune.set_knob(h, "coated_lanes", 1)
         for ck in (0, 4, 5, 8):
             autotune.set_knob(h, "mie_ckpt", ck)
             res[ck] = mie_batch(x, m=m1, y=y, m2=m2, coeffs=True)
     finally:
         autotune.set_knob(h, "mie_ckpt", 4)
+        autotune.set_knob(h, "coated_lanes", 0)
     for ck in (4, 5, 8):
         same = True
         for k in ("qext", "qsca", "asy", "qb"):
@@ -120,6 +124,39 @@ def test_coated_checkpoint_variants_agree(gpu):
             same &= bool(np.array_equal(a, b))
             assert np.all(np.abs(a - b) <= 1e-12 * np.abs(a).max()), ck
         print("checkpoint every %d rows: bitwise identical to the full-row kernel: %s" % (ck, same))
+
+
+def test_checkpoint_knob_leaves_the_coated_lanes(gpu):
+    """Setting the checkpoint interval, to its own value or another, leaves a small
+    batch on the kernel that splits each point over lanes (the same bits), and
+    GM_TUNE_COATED_LANES alone takes it off (other bits: another order of the same
+    operations)."""
+    import torch
+    from geosmie_amd import _lib, autotune
+    from geosmie_amd._lib import check, ptr
+    h = _lib.private_ctx()
+    y = np.exp(np.linspace(np.log(0.05), np.log(209.0), 1266))
+    d = [_lib.to_dev(0.7 * y), _lib.to_dev(y), _lib.cplx_dev(np.full(y.size, (1.95 + 0.79j) ** 2)),
+         _lib.cplx_dev(np.full(y.size, 1.45 ** 2 + 0j))]
+
+    def run():
+        props = torch.empty(6 * y.size, dtype=torch.float64, device="cuda")
+        check(_lib.lib().gm_mie_batch(h, y.size, ptr(d[0]), ptr(d[1]), ptr(d[2]), None, ptr(d[3]),
+                                      209.0, None, None, None, ptr(props), None, _lib.GM_MIE_SORT,
+                                      _lib.stream()))
+        return props
+    first = run()
+    autotune.set_knob(h, "mie_ckpt", autotune.get(h, "mie_ckpt"))
+    assert torch.equal(run(), first)
+    for ck in (0, 5, 8, 4):
+        autotune.set_knob(h, "mie_ckpt", ck)
+        assert torch.equal(run(), first), ck
+    autotune.set_knob(h, "coated_lanes", 1)
+    assert not torch.equal(run(), first)
+    autotune.set_knob(h, "coated_lanes", 0)
+    assert torch.equal(run(), first)
+    with pytest.raises(ValueError):
+        autotune.set_knob(h, "coated_lanes", 8)
 
 
 def test_homog_checkpoint_agrees(gpu):

@@ -3,8 +3,7 @@ combination in extended precision (64-bit mantissa) on a sample of the points.
 
 The tolerance is the 1e-9 of every comparison with the oracle, doubled for the
 sampled points' own conditioning (rounded m x, m y next to a resonance): |a_n|, |b_n| <= 1
-absolute, efficiencies relative, g absolute.  Against the same points one per lane (a
-context whose checkpoint knob is set): the same points are NaN (series that
+absolute, efficiencies relative, g absolute.  Against the same points one per lane: the same points are NaN (series that
 overflow, tiny cores in large shells), and the other classes are unchanged.
 """
 import numpy as np
@@ -108,7 +107,7 @@ def test_lanes_per_point(gpu, n, y_hi, q_lo, sort):
         x[5::50] = y[5::50]
         m2[7::50] = 1.6 + 0.4j
     h, ref = _lib.private_ctx(), _lib.private_ctx()
-    set_knob(ref, "mie_ckpt", 4)
+    set_knob(ref, "coated_lanes", 1)
     got, want = _run(h, x, y, m1, m2, sort), _run(ref, x, y, m1, m2, sort)
     assert all(torch.equal(torch.isnan(a), torch.isnan(b)) for a, b in zip(got, want))
     coated = (x != y) & (m2.imag * y <= 1.0)
@@ -152,7 +151,7 @@ def test_long_points_of_a_batch(gpu, y_lo, y_hi, skew):
     m1, m2 = np.full(n, 1.95 + 0.79j), np.full(n, 1.4 + 0j)
     x[5::500] = y[5::500]
     h, ref = _lib.private_ctx(), _lib.private_ctx()
-    set_knob(ref, "mie_ckpt", 4)
+    set_knob(ref, "coated_lanes", 1)
     got, want = _run(h, x, y, m1, m2, True), _run(ref, x, y, m1, m2, True)
     # an absorbing core needs no start correction: both forms hold 1e-9
     for a, b in zip(got[:2], want[:2]):

@@ -118,12 +118,12 @@ def test_very_large_size_parameter(gpu, lanes):
         assert np.abs(s2[i] - o2).max() <= 1e-11 * scale, i
 
 
-@pytest.mark.parametrize("ckpt", [4, 0])
-def test_coated_large_shells(gpu, ckpt):
+@pytest.mark.parametrize("ckpt, lanes", [(4, 1), (0, 1), (4, 0)])
+def test_coated_large_shells(gpu, ckpt, lanes):
     """Coated spheres out to y = 1000 (5x the coated workload's largest
     shell), real and weakly absorbing shells, strongly and weakly absorbing
-    cores, with the checkpointed kernel (4) and the one that keeps every row
-    (0), against the C restatement's cancellation-free form (its literal form
+    cores, one point per lane with the checkpointed kernel (4) and the one that
+    keeps every row (0) and with each point split over lanes (lanes 0), against the C restatement's cancellation-free form (its literal form
     agrees with it to 5e-11 on these points): Qext, Qsca 1e-9 relative, g
     1e-9 absolute."""
     from oracle import cmie
@@ -137,9 +137,11 @@ def test_coated_large_shells(gpu, ckpt):
     m2 = np.where(r.uniform(size=y.size) < 0.5, 1.33 + 0j, 1.45 + 1e-4j)
     try:
         autotune.set_knob(h, "mie_ckpt", ckpt)
+        autotune.set_knob(h, "coated_lanes", lanes)
         got = mie_batch(x, m=m1, y=y, m2=m2)
     finally:
         autotune.set_knob(h, "mie_ckpt", 4)
+        autotune.set_knob(h, "coated_lanes", 0)
     c = cmie.batch(x, m1, y, m2, threads=8, stable=True)
     for j, k in enumerate(("qext", "qsca")):
         rel = np.abs(got[k] - c[j]) / np.abs(c[j])

@@ -51,10 +51,11 @@ def test_graph_replay_matches_eager(gpu, precision):
         _same(eager, ch.results())
 
 
-def test_coated_batch_graph_replays(gpu):
-    """A coated gm_mie_batch (plan kernels, then the checkpointed kernel,
-    whose work-queue counter the plan's scan kernel resets) captured as a HIP
-    graph, as bench.py times it: three replays, each after unrelated coated
+@pytest.mark.parametrize("lanes", [1, 0])
+def test_coated_batch_graph_replays(gpu, lanes):
+    """A coated gm_mie_batch (plan kernels, then, one point per lane, the
+    checkpointed kernel, whose work-queue counter the plan's scan kernel resets, or
+    the kernel that splits each point over lanes) captured as a HIP graph, as bench.py times it: three replays, each after unrelated coated
     work on the default context and with the output clobbered, reproduce the
     eager step bit for bit."""
     t = __import__("torch")
@@ -71,6 +72,8 @@ def test_coated_batch_graph_replays(gpu):
     d_props = t.empty(6 * n, dtype=t.float64, device="cuda")
     L = _lib.lib()
     h = _lib.private_ctx()
+    from geosmie_amd.autotune import set_knob
+    set_knob(h, "coated_lanes", lanes)
 
     def step():
         check(L.gm_mie_batch(h, n, ptr(d_x), ptr(d_y), ptr(d_eps), None, ptr(d_eps2),
