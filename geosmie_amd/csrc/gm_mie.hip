@@ -26,6 +26,8 @@
 // psi_n = psi_{n-1} / (D_n(s) + n/s) with D_n(s) from a separate downward
 // recurrence started 16 + 8 ceil(|s|^(1/3)) above nmax (converged), which is
 // stable where psi_n decays.
+#include <type_traits>
+
 #include "gm_complex.h"
 #include "gm_internal.h"
 
@@ -1441,15 +1443,20 @@ __global__ __launch_bounds__(64, MINW) void k_mie_coated_stable(
     const int64_t off = coef_off ? coef_off[p] : 0;
     const CoatedPt cp{v, w, yy, m, m2, nmax, nsw_v, nsw_w, nsw_y, ddv_on, ddw_on};
     const __amdgpu_buffer_rsrc_t rs = slot_rsrc(slot, (uint32_t)(plane * 11 * sizeof(double)));
-    const CoatedState st = coated_state1(v, w, yy);
     const uint32_t pl = (uint32_t)plane;
+    // the state before row 1 is formed in each branch, not kept over them: 40 registers
+    // that would leave one wavefront per SIMD (265 registers against 245, 1057 us a
+    // batch of 300k shells to y = 209 against 860)
+    auto up = [&](auto dd, auto store) {
+      coated_rows<dd(), store()>(cp, coated_state1(v, w, yy), 1, nmax, rs, pl, lane, off, an, bn,
+                                 pr, nullptr);
+    };
     if (__any(ddv_on || ddw_on)) {
-      if (coef_off) coated_rows<true, true>(cp, st, 1, nmax, rs, pl, lane, off, an, bn, pr, nullptr);
-      else coated_rows<true, false>(cp, st, 1, nmax, rs, pl, lane, off, an, bn, pr, nullptr);
+      if (coef_off) up(std::true_type{}, std::true_type{});
+      else up(std::true_type{}, std::false_type{});
     } else {
-      if (coef_off)
-        coated_rows<false, true>(cp, st, 1, nmax, rs, pl, lane, off, an, bn, pr, nullptr);
-      else coated_rows<false, false>(cp, st, 1, nmax, rs, pl, lane, off, an, bn, pr, nullptr);
+      if (coef_off) up(std::false_type{}, std::true_type{});
+      else up(std::false_type{}, std::false_type{});
     }
     if (props) pr.finish(yy, p, n_all, props);
   }

@@ -122,3 +122,43 @@ def test_autotune_cache_file(tmp_path):
     with open(path, "w") as f:
         f.write("{not json")
     assert autotune.load_cache(path) == {}
+
+
+def _kernel_notes():
+    """{kernel symbol: (registers, bytes of scratch a lane)} of the built library's gfx950
+    code, from the metadata the compiler leaves in it."""
+    import struct
+    import subprocess
+    import tempfile
+    from geosmie_amd import _lib
+    data, out = open(_lib.LIB_PATH, "rb").read(), {}
+    for m in re.finditer(b"__CLANG_OFFLOAD_BUNDLE__", data):
+        n, = struct.unpack_from("<Q", data, m.start() + 24)
+        at = m.start() + 32
+        for _ in range(n):
+            off, size, tl = struct.unpack_from("<QQQ", data, at)
+            triple = data[at + 24:at + 24 + tl]
+            at += 24 + tl
+            if b"gfx950" not in triple:
+                continue
+            with tempfile.NamedTemporaryFile(suffix=".co") as f:
+                f.write(data[m.start() + off:m.start() + off + size])
+                f.flush()
+                notes = subprocess.run(["/opt/rocm/llvm/bin/llvm-readelf", "--notes", f.name],
+                                       capture_output=True, text=True, check=True).stdout
+            for blk in notes.split(".agpr_count:")[1:]:
+                name = re.search(r"\.name:\s+(_Z\S+)", blk).group(1)
+                out[name] = tuple(int(re.search(r"\.%s:\s+(\d+)" % k, blk).group(1))
+                                  for k in ("vgpr_count", "private_segment_fixed_size"))
+    return out
+
+
+def test_coated_kernels_leave_two_wavefronts_per_simd():
+    """The one-point-per-lane coated kernels without a register budget are built to
+    have two wavefronts per SIMD resident: at most 256 of its 512 registers a lane,
+    nothing in scratch."""
+    notes = _kernel_notes()
+    for k in ("k_mie_coated_stableILi1E", "k_mie_coated_ckptILi1ELi4E",
+              "k_mie_coated_ckptILi1ELi5E", "k_mie_coated_ckptILi1ELi8E"):
+        (name,) = [n for n in notes if k in n]
+        assert notes[name][0] <= 256 and notes[name][1] == 0, (name, notes[name])
