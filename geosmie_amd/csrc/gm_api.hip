@@ -12,6 +12,7 @@
 #include "geosmie.h"
 #include "gm_ctx.h"
 #include "gm_internal.h"
+#include "gm_parts.h"
 
 static thread_local char g_err[512] = "";
 
@@ -243,16 +244,11 @@ MieGrids mie_grids(const gm_ctx* ctx, int64_t n, int rows_cap, size_t budget) {
     g.lcap = (rows_cap + g.lanes - 1) / g.lanes;
     const size_t slot_bytes = (size_t)g.lcap * 64 * gm::kHomogRowDoubles * sizeof(double);
     const int64_t per_wave = 64 / g.lanes;
-    int64_t gg = std::min<int64_t>((n + per_wave - 1) / per_wave,
-                                   (int64_t)ctx->n_cu * std::max(ctx->occ_coop, 1) *
-                                       std::max(ctx->tune_mie_grid_mult, 1));
-    // three parts in one launch, each on slots of its own
-    auto fit = [&](int64_t blocks, size_t bytes) {
-      return std::min<int64_t>(blocks, std::max<int64_t>(1, (int64_t)(budget / 3 / bytes)));
-    };
     const int64_t resident = (int64_t)ctx->n_cu * std::max(ctx->occ_coop, 1);
-    gg = fit(gg, slot_bytes);
-    const size_t mid_slot = (size_t)gm::kMidLcap * 64 * gm::kHomogRowDoubles * sizeof(double);
+    // three parts in one launch, each on slots of its own
+    gm::HomogParts want{};
+    want.big = std::min<int64_t>((n + per_wave - 1) / per_wave,
+                                 resident * std::max(ctx->tune_mie_grid_mult, 1));
     // Middle series apart: where 64 lanes hold less than four of their rows each and the
     // batch is several rounds of wavefronts (40k points to x = 2094: Mie 319 us with
     // two launches, 291 two parts in one, 249 with the middle part at cost 640, 258 at
@@ -260,17 +256,15 @@ MieGrids mie_grids(const gm_ctx* ctx, int64_t n, int rows_cap, size_t budget) {
     // a step against 141).
     if (g.lanes == 64 && !ctx->tune_mie_lanes && n >= 4 * resident) {
       const int64_t per = 64 / gm::kMidLanes;
-      g.mid_grid = fit(std::min<int64_t>((n + per - 1) / per, resident), mid_slot);
+      want.mid = std::min<int64_t>((n + per - 1) / per, resident);
     }
-    const size_t small_slot = (size_t)gm::kSmallLcap * 64 * gm::kHomogRowDoubles * sizeof(double);
-    g.small_grid = fit(std::min<int64_t>((n + 15) / 16, resident), small_slot);
-    size_t bytes = (size_t)gg * slot_bytes + (size_t)g.mid_grid * mid_slot +
-                   (size_t)g.small_grid * small_slot;
-    if (bytes > budget) {   // no room for a slot of each: all points with many lanes
-      g.mid_grid = g.small_grid = 0;
-      bytes = (size_t)gg * slot_bytes;
-    }
-    g.homog = std::make_pair(gg, bytes);
+    want.small = std::min<int64_t>((n + 15) / 16, resident);
+    const gm::HomogParts parts = gm::homog_parts(
+        budget, want, slot_bytes, (size_t)gm::kMidLcap * 64 * gm::kHomogRowDoubles * sizeof(double),
+        (size_t)gm::kSmallLcap * 64 * gm::kHomogRowDoubles * sizeof(double));
+    g.mid_grid = parts.mid;
+    g.small_grid = parts.small;
+    g.homog = std::make_pair(parts.big, parts.bytes);
   }
   g.literal = grid_for(ctx->occ_literal, gm::kCoatedRowDoubles);
   const int ck = ctx->tune_mie_ckpt;

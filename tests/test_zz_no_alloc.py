@@ -80,6 +80,16 @@ def test_noalloc_matches_batch_twice_homogeneous(gpu):
         assert np.all(got["props"][:x.size] > 0)
 
 
+# the static scratch holds about 640 of the long part's 2048 slots at x = 8000, all at 2094
+@pytest.mark.parametrize("hi", [8000.0, 2094.0])
+def test_noalloc_matches_batch_long_series(gpu, hi):
+    x = np.exp(np.linspace(np.log(0.02), np.log(hi), 9001))
+    np.random.default_rng(1).shuffle(x)
+    ref = _run("batch", x, None, 1.53 + 0.005j, None, True)
+    got = _run("noalloc", x, None, 1.53 + 0.005j, None, True)
+    _same(ref, got)
+
+
 def test_noalloc_matches_batch_twice_coated(gpu):
     for n in (60000, 5000):
         x, y, m1, m2 = _coated(n)
