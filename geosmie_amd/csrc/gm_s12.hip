@@ -1221,12 +1221,23 @@ dim3 s12_grid(int64_t blocks) {
               (unsigned)((blocks + gm::kGridRow - 1) / gm::kGridRow));
 }
 
+// Whether `stream` is being captured, where a workspace cannot grow.
+bool capturing(hipStream_t stream) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;   // the legacy stream beside a capture
+}
+
 // The (P, M) pairs, and the launch order of `units` units of unit_pts points
 // (*order, NULL where the series are too short or the units too few for a long
-// unit at the end to matter: sorting costs two launches, about 10 us).
-int s12_pairs(gm_ctx* ctx, int precision, const S12Shape& h, int n_ang, const double* pi_t,
-              const double* tau_t, int nmax_cap, gm::S12Tables& T, const gm::RowGroups& g, int unit_pts, int64_t units,
-              int64_t n, const int32_t* nmax, const int** order, hipStream_t s) {
+// unit at the end to matter: sorting costs two launches, about 10 us).  In a capture
+// whose workspace is too small the order is left out and then, at FP64, the pairs
+// (h.raw set): the same results, slower.
+int s12_pairs(gm_ctx* ctx, int precision, S12Shape& h, int n_ang, const double* pi_t,
+              const double* tau_t, int nmax_cap, gm::S12Tables& T, const gm::RowGroups& g,
+              int unit_pts, int64_t units, int64_t n, const int32_t* nmax, const int** order,
+              hipStream_t s) {
   *order = nullptr;
   T.pi_t = pi_t;
   T.tau_t = tau_t;
@@ -1237,12 +1248,19 @@ int s12_pairs(gm_ctx* ctx, int precision, const S12Shape& h, int n_ang, const do
   T.nmax_cap = nmax_cap;
   if (h.raw) return GM_OK;
   const int64_t total = (int64_t)((nmax_cap + 3) / 4 * 4) * T.apad;
-  const bool sorted = nmax_cap >= kS12SortRows && units >= 1024 && units <= 0x7fffffffLL;
+  bool sorted = nmax_cap >= kS12SortRows && units >= 1024 && units <= 0x7fffffffLL;
   // pairs, then (sorted) the histogram and its cursors, the order and the bins
   const bool f64 = precision == GM_PREC_FP64;
   const size_t o_hist = (size_t)total * (f64 ? sizeof(double2) : sizeof(float2));
   const size_t o_ord = o_hist + 2 * gm::kUnitBins * sizeof(int);
   const size_t o_bin = o_ord + (size_t)units * sizeof(int);
+  if ((sorted ? o_bin + (size_t)units : o_hist) > ctx->tab_lp.bytes && capturing(s)) {
+    sorted = false;
+    if (f64 && o_hist > ctx->tab_lp.bytes) {
+      h.raw = true;
+      return GM_OK;
+    }
+  }
   int rc = ctx->reserve(ctx->tab_lp, sorted ? o_bin + (size_t)units : o_hist);
   if (rc) return rc;
   char* ws = (char*)ctx->tab_lp.ptr;
@@ -1283,8 +1301,8 @@ int launch_s12(gm_ctx* ctx, const char* who, int64_t n, const int64_t* off, cons
   if (precision != GM_PREC_BF16X3) {
     ctx->mark_begin(gm::kKS12, s, &slot);
     const int64_t units = (n + 15) / 16;
-    const S12Shape h = precision == GM_PREC_FP64 ? s12_shape(units, n_ang, kS12Want)
-                                                 : s12_shape32(units, n_ang, 8);
+    S12Shape h = precision == GM_PREC_FP64 ? s12_shape(units, n_ang, kS12Want)
+                                           : s12_shape32(units, n_ang, 8);
     gm::S12Tables T;
     const int* order;
     gm::RowGroups none{};
@@ -1477,7 +1495,8 @@ int gm_s12_contract_rows(gm_ctx* ctx, int64_t n, const int64_t* coef_off, const 
   hipLaunchKernelGGL((gm::k_s12_rows<P_, R_, T_, W_, M_>), g64, dim3(64 * h64.wpb), 0, s, g,     \
                      chunk_pts, T, coef_off, nmax, an, bn, cf, w, n, part, h64.ablocks, order)
 #define GM_ROWS_F64(R_)                                                                        \
-  if (per > 1) GM_ROWS(GM_PREC_FP64, R_, (R_ == 1 ? 4 : 2), false, true);                       \
+  if (per > 1 && h64.raw) GM_ROWS(GM_PREC_FP64, R_, (R_ == 1 ? 4 : 2), true, true);             \
+  else if (per > 1) GM_ROWS(GM_PREC_FP64, R_, (R_ == 1 ? 4 : 2), false, true);                  \
   else if (h64.tt == 4 && h64.raw) GM_ROWS(GM_PREC_FP64, R_, 4, true, false);                   \
   else if (h64.tt == 4) GM_ROWS(GM_PREC_FP64, R_, 4, false, false);                             \
   else if (h64.tt == 2 && h64.raw) GM_ROWS(GM_PREC_FP64, R_, 2, true, false);                   \

@@ -221,7 +221,9 @@ int gm_angle_tables(gm_ctx* ctx, int n_ang, const double* cos_theta, int nmax_ca
 /* S1, S2 (complex, [n][n_ang]) of n coefficient sets against an angle table.
  * Replaces mie_S12_backend_pt / numba_dot (mie_props.py:133-149) as looped by
  * runS12Loop (mie_coated.py:31-39).  nmax[n] int32 per set; the table must
- * have nmax_cap >= max(nmax) rows.  precision: gm_precision. */
+ * have nmax_cap >= max(nmax) rows.  precision: gm_precision.  The tables are
+ * regrouped in a workspace of ctx (at FP64 from 4096 sets on; a stream capture that
+ * finds it too small reads them as they are at FP64, and fails at the others). */
 int gm_mie_s12(gm_ctx* ctx, int64_t n, const int64_t* coef_off, const int32_t* nmax,
                const double* an, const double* bn, int n_ang, const double* pi_t,
                const double* tau_t, int nmax_cap, double* s1, double* s2, int precision,

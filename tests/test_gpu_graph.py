@@ -96,3 +96,63 @@ def test_coated_batch_graph_replays(gpu, lanes):
         graph.replay()
         t.cuda.synchronize()
         assert np.array_equal(d_props.cpu().numpy(), eager)
+
+
+# 4113 points: from 4096 points on FP64 S1/S2 builds its angle-table pairs in the
+# context's workspace; cap 600: and sorts the tiles by length (17000 points); row sums
+# of one tile per work unit and of two
+@pytest.mark.parametrize("n, cap, tiles", [(4113, 0, 0), (17000, 600, 0), (4113, 0, 2)])
+def test_fp64_s12_captured_on_a_new_context(gpu, n, cap, tiles):
+    """gm_s12_mueller at FP64 captured as the first call of its context (nothing can
+    be allocated), then after an eager call, then, its workspace sized by a call with
+    a shorter table, gm_s12_contract_rows with a longer one: every replay gives the
+    eager bits."""
+    import ctypes
+    t = __import__("torch")
+    from geosmie_amd import _lib
+    from geosmie_amd._lib import check, ptr
+    from geosmie_amd.autotune import set_knob
+    from geosmie_amd.lut import _DevMie
+    from geosmie_amd.s12 import angle_tables_dev
+    rng = np.random.default_rng(n)
+    dm = _DevMie(10 ** rng.uniform(-1.5, 1.0, n), complex(1.5, 0.01))
+    n_ang = 33
+    pi_t, tau_t = angle_tables_dev(np.cos(np.radians(np.linspace(0.0, 180.0, n_ang))),
+                                   max(cap, dm.nmax_max + 40))
+    L, full = _lib.lib(), int(pi_t.shape[0])
+    out = t.empty((n, 4, n_ang), dtype=t.float64, device="cuda")
+    w = t.rand(n, dtype=t.float64, device="cuda")
+    rows = t.empty((1, 4, n_ang), dtype=t.float64, device="cuda")
+    st, ct = (ctypes.c_int64 * 1)(0), (ctypes.c_int64 * 1)(n)
+
+    def mueller(h):
+        check(L.gm_s12_mueller(h, n, ptr(dm.d_off), ptr(dm.d_nmax), ptr(dm.d_an), ptr(dm.d_bn),
+                               n_ang, ptr(pi_t), ptr(tau_t), full, ptr(out), 0, _lib.stream()))
+
+    def contract(h, cap):
+        check(L.gm_s12_contract_rows(h, n, ptr(dm.d_off), ptr(dm.d_nmax), ptr(dm.d_an),
+                                     ptr(dm.d_bn), n_ang, ptr(pi_t), ptr(tau_t), cap, 1, st, ct,
+                                     ptr(w), ptr(rows), 0, None, _lib.stream()))
+
+    def replays(step, dst):
+        eager = dst.clone()
+        graph = t.cuda.CUDAGraph()
+        with t.cuda.graph(graph):
+            step()
+        for _ in range(3):
+            dst.fill_(-1.0)
+            mueller(_lib.ctx()) if dst is rows else contract(_lib.ctx(), full)
+            graph.replay()
+            t.cuda.synchronize()
+            assert t.equal(dst, eager)
+    mueller(_lib.ctx())
+    new = _lib.private_ctx()
+    replays(lambda: mueller(new), out)
+    mueller(new)
+    replays(lambda: mueller(new), out)
+    other, ref = _lib.private_ctx(), _lib.private_ctx()
+    set_knob(other, "s12_row_tiles", tiles)
+    set_knob(ref, "s12_row_tiles", tiles)
+    contract(other, dm.nmax_max)          # sizes the partial sums, pairs of a shorter table
+    contract(ref, full)
+    replays(lambda: contract(other, full), rows)
