@@ -104,7 +104,8 @@ __global__ __launch_bounds__(256) void k_s12_prep_pairs(int n_ang, int nmax_cap,
   tab[id] = v;
 }
 
-// The same as FP32 pairs; total counts pairs.
+// The same as FP32 pairs; total counts pairs.  Columns 2 i and 2 i + 1 of every 32 are
+// its angles i and 16 + i: the two that a lane loads as 16 bytes.
 __global__ __launch_bounds__(256) void k_s12_prep_pairs32(int n_ang, int nmax_cap, int apad,
                                                           int64_t total,
                                                           const double* __restrict__ pi_t,
@@ -115,7 +116,8 @@ __global__ __launch_bounds__(256) void k_s12_prep_pairs32(int n_ang, int nmax_ca
   if (hist && blockIdx.x == 0)
     for (int b = threadIdx.x; b < 2 * kUnitBins; b += 256) hist[b] = 0;
   if (id >= total) return;
-  const int k = (int)(id / apad), j = (int)(id - (int64_t)k * apad);
+  const int k = (int)(id / apad), c = (int)(id - (int64_t)k * apad);
+  const int j = (c & ~31) + 16 * (c & 1) + ((c & 31) >> 1);
   double P = 0.0, M = 0.0;
   if (k < nmax_cap && j < n_ang) {
     const double p = pi_t[(size_t)k * n_ang + j], t = tau_t[(size_t)k * n_ang + j];
@@ -305,9 +307,11 @@ __global__ __launch_bounds__(256) void k_s12_unit_order(int64_t units,
 }
 
 // The same sums at FP32 (v_mfma_f32_16x16x4_f32, results in FP32): U, V rounded from
-// FP64 sums, tables FP32 pairs.  A lane loads the pairs of two neighbouring angles
-// as 16 bytes: sub-tiles t and t + 1 (t even) are the even and odd columns of 32
-// angles, column i of sub-tile t being angle j0 + 16 (t & ~1) + 2 i + (t & 1).
+// FP64 sums, tables FP32 pairs.  A lane loads the pairs of two angles as 16 bytes:
+// column i of sub-tiles t and t + 1 (t even), angles j0 + 16 t + i and 16 further on
+// (k_s12_prep_pairs32 puts them side by side).  With neighbouring angles side by side
+// in the table a sub-tile was every other angle and its stores half of every line:
+// Mueller elements of 4090 points x 1801 angles 88 us, 65 as here.
 // Element r of lane (i, g) is point p0 + 4 g + r.  LP: the coefficients come from
 // gm_s12_split_coef, 16 bytes {U.re, V.re, U.im, V.im} a term.  Tiles of 8 points and
 // 64 angles spent 8 8-byte or 4-byte loads and two coefficient loads on 8 MFMAs of
@@ -437,14 +441,17 @@ __global__ __launch_bounds__(256, 2) void k_s12_tiles(S12Tables T, int64_t n,
   if (j0 >= T.n_ang) return;
   double4_ spr[TT], spi[TT], smr[TT], smi[TT];
   s12_tile64<TT, RAW, 4, 1>(T, p0, n, j0, lane, off, nmax, an, bn, spr, spi, smr, smi);
+  // a point's sub-tiles one after the other: rows start anywhere in a line (n_ang may be
+  // odd), and consecutive stores fill the lines that a sub-tile ends in (Mueller
+  // elements of 5000 short series x 1801 angles 104 us by sub-tile, 91 by point)
 #pragma unroll
-  for (int t = 0; t < TT; ++t) {
-    const int j = j0 + 16 * t + (lane & 15);
-    if (j >= T.n_ang) continue;
+  for (int r = 0; r < 4; ++r) {
+    const int64_t p = p0 + (lane >> 4) + 4 * r;
+    if (p >= n) continue;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int64_t p = p0 + (lane >> 4) + 4 * r;
-      if (p < n)
+    for (int t = 0; t < TT; ++t) {
+      const int j = j0 + 16 * t + (lane & 15);
+      if (j < T.n_ang)
         s12_store(mode, p, j, T.n_ang, cd{spr[t][r], spi[t][r]}, cd{smr[t][r], smi[t][r]}, out0,
                   out1);
     }
@@ -469,13 +476,13 @@ __global__ __launch_bounds__(256, 2) void k_s12_tiles32(S12Tables T, int64_t n,
   float4_ spr[TT], spi[TT], smr[TT], smi[TT];
   s12_tile32<TT, false, 4>(T, p0, n, j0, lane, off, nmax, an, bn, nullptr, spr, spi, smr, smi);
 #pragma unroll
-  for (int t = 0; t < TT; ++t) {
-    const int j = j0 + 16 * (t & ~1) + 2 * (lane & 15) + (t & 1);
-    if (j >= T.n_ang) continue;
+  for (int r = 0; r < 4; ++r) {
+    const int64_t p = p0 + 4 * (lane >> 4) + r;
+    if (p >= n) continue;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int64_t p = p0 + 4 * (lane >> 4) + r;
-      if (p < n)
+    for (int t = 0; t < TT; ++t) {
+      const int j = j0 + 16 * t + (lane & 15);
+      if (j < T.n_ang)
         s12_store(mode, p, j, T.n_ang, cd{(double)spr[t][r], (double)spi[t][r]},
                   cd{(double)smr[t][r], (double)smi[t][r]}, out0, out1);
     }
@@ -558,7 +565,7 @@ __global__ __launch_bounds__(64 * kRowsWaves, 2) void k_s12_rows(
                         : kq == 1 ? -0.5 * v[2]
                         : kq == 2 ? 0.25 * (v[0] - v[1])
                                   : -0.5 * v[3];
-    const int j = F64 ? j0 + 16 * t + i : j0 + 16 * (t & ~1) + 2 * i + (t & 1);
+    const int j = j0 + 16 * t + i;
     if (r < nr && j < T.n_ang) dst[((size_t)r * 4 + kq) * T.n_ang + j] = mine;
   };
   if (MANY) {
@@ -1180,7 +1187,10 @@ constexpr int64_t kS12Want = 8192;
 // FP32: up to 128 angles per wavefront where a and b are read as FP64 (1.5M points x
 // 371 angles 10.49 against 11.03 ms at 64; 60k points, 11k wavefronts, 1.97 against
 // 1.87), 64 where they come converted (40k x 1801 1.73 against 1.75 ms at 128).
+// 64 angles from 10k wavefronts on (60k points x 181 angles, 11k: amplitudes 127 against
+// 148 us at 32, to x = 1000 691 against 806; 5k points x 1801 angles, 9k: 186 against 168).
 constexpr int64_t kS12Want32 = 16384;
+constexpr int64_t kS12Want32Half = 10240;
 constexpr int64_t kS12PairTiles = 256;
 constexpr int kS12SortRows = 512;
 
@@ -1206,9 +1216,10 @@ S12Shape s12_shape(int64_t tiles, int n_ang, int64_t want, int max_tt = 4) {
 // FP32: 32, 64 or 128 angles per wavefront, always on the paired tables.
 S12Shape s12_shape32(int64_t tiles, int n_ang, int max_tt) {
   S12Shape h = s12_shape(tiles, n_ang, kS12Want32, max_tt);
-  if (h.tt < 2) {
-    h.tt = 2;
-    const int waves = (n_ang + 31) / 32;
+  if (h.tt < 4) {
+    const int tt = tiles * ((n_ang + 63) / 64) >= kS12Want32Half ? 4 : 2;
+    const int waves = (n_ang + 16 * tt - 1) / (16 * tt);
+    h.tt = tt;
     h.ablocks = (waves + 3) / 4;
     h.wpb = (waves + h.ablocks - 1) / h.ablocks;
   }
