@@ -167,6 +167,10 @@ constexpr int kLongRows = 512;
 // longest chain is below an even share of the batch: above this size only batches
 // with long series look for a split, the others save the launch (5 us).
 constexpr int64_t kCoatedLongMax = 512 * 1024;
+// Nor do short series: up to this many rows a wavefront of split points costs what the
+// longest chain takes (shells y in 1..20, 33 rows, 8192 / 60k points: 76 / 93 us with
+// the search, 67 / 87 without).
+constexpr int kCoatedShortRows = 64;
 
 // Lanes per point of the homogeneous kernel: the tuned value, or by batch:
 // one point per lane once the batch fills the GPU (64 points per wavefront,
@@ -296,7 +300,7 @@ MieGrids mie_grids(const gm_ctx* ctx, int64_t n, int rows_cap, size_t budget) {
     g.stable = std::make_pair(gg, (size_t)gg * slot_bytes);
   }
   if (g.coated_lanes == 1 && !ctx->tune_coated_lanes && ctx->tune_mie_waves == 0 &&
-      (n <= kCoatedLongMax || rows_cap >= kLongRows)) {
+      rows_cap > kCoatedShortRows && (n <= kCoatedLongMax || rows_cap >= kLongRows)) {
     // the long series run first, on the same slots
     g.coated_long = rows_cap <= 1200 ? 16 : 64;
     const int64_t per_wave = 64 / g.coated_long;

@@ -191,7 +191,10 @@ __global__ __launch_bounds__(256) void k_plan_keys(
 // (measured: 20 us + 13 us at cost 1400 with 16 lanes, 20 us + 96 us at 5700; two
 // rounds 67 us); the latter takes its longest chain or 1.2 even shares of all
 // SIMDs' lanes, whichever is longer (84 us at c_rest = 284; 268 us at a share of
-// 1071, 2700 us at 12850).
+// 1071, 2700 us at 12850).  Splits are taken where they save kCoatedGain of the
+// unsplit time: 250k points log-distributed to y = 400 took 618 us with the split that
+// the model put just below it, 550 whole; 200k 534 and 541, 100k 349 and 528.
+constexpr float kCoatedGain = 0.07f;
 __device__ __forceinline__ float coated_split(float n_long, float w_long, float c_max, float c_rest,
                                               float w_rest, int lanes, int simds) {
   const float slots = 64.0f * (float)simds;
@@ -207,8 +210,10 @@ __global__ __launch_bounds__(256) void k_plan_scan(const int64_t* __restrict__ h
                                                    int64_t slots, int coated_lanes, int simds,
                                                    int64_t* __restrict__ ab) {
   __shared__ int64_t part[256];
-  __shared__ int64_t part_n[256];
+  __shared__ int64_t wave_w[4], wave_n[4];
+  __shared__ int wave_max[4];
   __shared__ unsigned long long best;
+  float whole = 0.0f;   // the coated class's modelled time without a split
   constexpr int per = (kClasses * kBuckets) / 256;
   static_assert(per * 256 == kClasses * kBuckets, "histogram must split into 256 runs");
   const int t = threadIdx.x;
@@ -275,32 +280,44 @@ __global__ __launch_bounds__(256) void k_plan_scan(const int64_t* __restrict__ h
         c_max = max(c_max, b);
       }
     }
-    part[t] = cw;
-    part_n[t] = cn;
-    __syncthreads();
-    for (int off = 1; off < 256; off <<= 1) {
-      const int64_t v = t >= off ? part[t - off] : 0, w = t >= off ? part_n[t - off] : 0;
-      __syncthreads();
-      part[t] += v;
-      part_n[t] += w;
-      __syncthreads();
-    }
-    const int64_t w_all = part[255], n_all = part_n[255];
-    // the highest bucket in use, of any thread
-    __shared__ int wave_max[4];
+    int64_t iw = cw, in = cn;   // inclusive sums: of the wavefront, then of those before it
+    const int lane = t & 63, wv = t >> 6;
 #pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) c_max = max(c_max, __shfl_xor(c_max, d));
-    if (t % 64 == 0) wave_max[t / 64] = c_max;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int64_t a = __shfl_up(iw, d), b = __shfl_up(in, d);
+      if (lane >= d) {
+        iw += a;
+        in += b;
+      }
+      c_max = max(c_max, __shfl_xor(c_max, d));
+    }
+    if (lane == 63) {
+      wave_w[wv] = iw;
+      wave_n[wv] = in;
+      wave_max[wv] = c_max;
+    }
     __syncthreads();
-    c_max = max(max(wave_max[0], wave_max[1]), max(wave_max[2], wave_max[3]));
+    int64_t w_all = 0, n_all = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (q < wv) {
+        iw += wave_w[q];
+        in += wave_n[q];
+      }
+      w_all += wave_w[q];
+      n_all += wave_n[q];
+      c_max = max(c_max, wave_max[q]);   // the highest bucket in use
+    }
     unsigned long long mine = ~0ull;
     constexpr float unit = (float)(1 << kBucketShift);
+    whole = coated_split(0.0f, 0.0f, 0.0f, unit * (float)c_max, unit * (float)w_all, coated_lanes,
+                         simds);
     if (t == 0 && n_all > 0)   // every point split
       mine = ((unsigned long long)__float_as_uint(
                   coated_split((float)n_all, unit * (float)w_all, unit * (float)c_max, 0.0f, 0.0f,
                                coated_lanes, simds)) << 32) | (unsigned)n_all;
-    cw = part[t] - cw;
-    cn = part_n[t] - cn;
+    cw = iw - cw;
+    cn = in - cn;
 #pragma unroll
     for (int i = 0; i < per; ++i) {
       const int b = bucket(i);
@@ -329,7 +346,8 @@ __global__ __launch_bounds__(256) void k_plan_scan(const int64_t* __restrict__ h
     ab[3] = range[1];
     ab[4] = 0;   // the coated class's work queue (kQueueSlot)
     ab[5] = ab[6] = range[2];
-    if (coated_lanes > 0 && best != ~0ull) {
+    if (coated_lanes > 0 && best != ~0ull &&
+        __uint_as_float((unsigned)(best >> 32)) < (1.0f - kCoatedGain) * whole) {
       ab[6] += (int64_t)(best & 0xffffffffull);
       range[2] = ab[6];
     }

@@ -135,27 +135,50 @@ def test_lanes_per_point(gpu, n, y_hi, q_lo, sort):
         assert abs(props[4, i] - 4 * asy / (sca * y[i] ** 2)) <= 2e-9, i
 
 
-# above 24576 points one per lane: the split of the longest (skewed sizes), of every
-# point (uniform long series) and of none (uniform short ones)
+# above 24576 points one per lane: the split of the longest (skewed sizes; 16 and, from
+# 1200 rows on, 64 lanes) and of every point (uniform long series)
 @pytest.mark.parametrize("y_lo, y_hi, skew", [(0.02, 209.0, True), (600.0, 700.0, False),
-                                              (1.0, 20.0, False)])
+                                              (1.0, 2000.0, None)])
 def test_long_points_of_a_batch(gpu, y_lo, y_hi, skew):
+    got, want = _both(24576 + 1, y_lo, y_hi, skew)
+    # an absorbing core needs no start correction: both forms hold 1e-9
+    for a, b in zip(got, want):
+        assert _torch().equal(_torch().isnan(a), _torch().isnan(b))
+    for a, b in zip(got[:2], want[:2]):
+        assert float(_torch().nan_to_num(a - b).abs().max()) <= 2e-9
+    for q in (0, 1, 4):
+        rel = _torch().nan_to_num((got[2][q] - want[2][q]) / want[2][q])
+        assert float(rel.abs().max()) <= 2e-9, q
+
+
+# no split where it would not pay: short series, and sizes whose longest chain costs
+# about what splitting it would (then every point is serial: the same bits)
+@pytest.mark.parametrize("n, y_lo, y_hi, skew", [(24577, 1.0, 20.0, False),
+                                                 (250000, 0.02, 400.0, True)])
+def test_batches_that_stay_whole(gpu, n, y_lo, y_hi, skew):
+    got, want = _both(n, y_lo, y_hi, skew)
+    assert all(_torch().equal(_torch().nan_to_num(a), _torch().nan_to_num(b))
+               for a, b in zip(got, want))
+
+
+def _torch():
     import torch
+    return torch
+
+
+def _both(n, y_lo, y_hi, skew):
+    """The batch with its lanes chosen by size and with one point per lane; skew: sizes
+    log-distributed, None: a few of the longest among short ones."""
     from geosmie_amd import _lib
     from geosmie_amd.autotune import set_knob
-    n = 24576 + 1
     rng = np.random.default_rng(int(y_hi))
     y = (np.exp(rng.uniform(np.log(y_lo), np.log(y_hi), n)) if skew
-         else rng.uniform(y_lo, y_hi, n))
+         else rng.uniform(y_lo, y_hi if skew is False else 20.0, n))
+    if skew is None:
+        y[::400] = np.linspace(0.65 * y_hi, y_hi, y[::400].size)
     x = y * rng.uniform(0.3, 0.9, n)
     m1, m2 = np.full(n, 1.95 + 0.79j), np.full(n, 1.4 + 0j)
     x[5::500] = y[5::500]
     h, ref = _lib.private_ctx(), _lib.private_ctx()
     set_knob(ref, "coated_lanes", 1)
-    got, want = _run(h, x, y, m1, m2, True), _run(ref, x, y, m1, m2, True)
-    # an absorbing core needs no start correction: both forms hold 1e-9
-    for a, b in zip(got[:2], want[:2]):
-        assert torch.equal(torch.isnan(a), torch.isnan(b))
-        assert float(torch.nan_to_num(a - b).abs().max()) <= 2e-9
-    for q in (0, 1, 4):
-        assert float(((got[2][q] - want[2][q]) / want[2][q]).abs().max()) <= 2e-9, q
+    return _run(h, x, y, m1, m2, True), _run(ref, x, y, m1, m2, True)
