@@ -948,6 +948,16 @@ int fuse_launch(const gm::FuseNet& f, int terms, int64_t n, const float* params,
   return GM_OK;
 }
 
+// Whether the forward pass runs fused: not for one layer, and not for two with at most
+// 64 features between them, where the activations kept out of memory do not pay for
+// splitting the weights and padding the rows.  us fused / layer by layer, 16k and
+// 400k queries: 256-256 41 / 18 and 682 / 480; 64-64-64 16 / 15 and 159 / 117; 6-32-3
+// 15.5 / 14.1 and 74 / 72; 6-64-3 15.5 / 14.0, but 78 / 87; 6-128-3 15.6 / 16.3 and 94 /
+// 152; 6-32-32-3 15.5 / 19.3 and 93 / 107.
+bool fuse_forward_pays(const Net& net) {
+  return net.L > 2 || (net.L == 2 && net.dims[1] > 64);
+}
+
 // y = net(x), or (post.on) the surrogate's table rows from it.
 int forward_any(gm_ctx* ctx, const Net& net, int64_t n, const float* params, const float* x,
                 float* y, const gm::FusePost& post, bool* posted, hipStream_t s) {
@@ -956,7 +966,7 @@ int forward_any(gm_ctx* ctx, const Net& net, int64_t n, const float* params, con
   gm::FuseNet f;
   size_t slot;
   *posted = false;
-  if (fuse_net(net, terms, f)) {
+  if (fuse_forward_pays(net) && fuse_net(net, terms, f)) {
     if ((rc = ctx->reserve(ctx->mlp_ws, (size_t)f.n_frag * 64 * terms * sizeof(uint4)))) return rc;
     uint4* frag = (uint4*)ctx->mlp_ws.ptr;
     ctx->mark_begin(gm::kKMlp, s, &slot);
@@ -1103,7 +1113,7 @@ int gm_surrogate_rows(gm_ctx* ctx, int n_layers, const int* dims, int64_t n, con
   post.on = 1;
   bool posted;
   if ((rc = forward_any(ctx, net, n, params, x, rows, post, &posted, (hipStream_t)stream))) return rc;
-  // a net too wide for the fused kernel wrote y: transform it in place
+  // a net that ran layer by layer wrote y: transform it in place
   return posted ? GM_OK
                 : gm_surrogate_post(ctx, n, net.dims[net.L], q, m_water_re, rows, tgt_mean, tgt_std,
                                     rows, stream);

@@ -24,10 +24,13 @@ def _setup(dims, n):
 
 
 # rows around one and two 64-row blocks; widths at and past the 16-, 32-, 64- and
-# 128-feature splits of the wavefronts, one layer, and 257 (the layer-by-layer path)
+# 128-feature splits of the wavefronts; 257 (layer by layer), and one layer and two
+# with 33 or 64 features between them (forward layer by layer, gradients fused)
 @pytest.mark.parametrize("dims,n", [((6, 256, 35), 63), ((6, 256, 35), 64), ((32, 33, 16), 65),
                                     ((33, 128, 129, 3), 128), ((256, 65, 256), 129),
-                                    ((5, 7), 200), ((6, 257, 4), 65)])
+                                    ((5, 7), 200), ((256, 256), 70), ((6, 64, 35), 65),
+                                    ((32, 33, 20, 16), 65), ((5, 7, 7, 7), 200),
+                                    ((6, 257, 4), 65)])
 def test_tile_edges_vs_oracle(gpu, dims, n):
     from geosmie_amd import _lib
     from geosmie_amd.surrogate import MLP
@@ -46,13 +49,14 @@ def test_tile_edges_vs_oracle(gpu, dims, n):
             assert np.linalg.norm(g[lo:hi] - gref[lo:hi]) <= 2e-3 * np.linalg.norm(gref[lo:hi])
 
 
-@pytest.mark.parametrize("width,n,baseline", [(256, 65, True), (40, 130, False), (300, 65, True)])
-def test_rows_match_forward_and_post(gpu, width, n, baseline):
+@pytest.mark.parametrize("hidden,n,baseline", [((256,), 65, True), ((40,), 130, False),
+                                               ((40, 40), 130, False), ((300,), 65, True)])
+def test_rows_match_forward_and_post(gpu, hidden, n, baseline):
     import torch
     from geosmie_amd import _lib
     from geosmie_amd._lib import ptr
     from geosmie_amd.surrogate import MLP, make_queries
-    dims = (6, width, 35)
+    dims = (6, *hidden, 35)
     p, x, _, _ = _setup(dims, n)
     rng = np.random.default_rng(n)
     q = make_queries(rng.uniform(0.01, 5, n), rng.uniform(1.4, 2.6, n), rng.uniform(1.3, 1.8, n),
