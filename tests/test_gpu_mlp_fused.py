@@ -74,3 +74,48 @@ def test_rows_match_forward_and_post(gpu, hidden, n, baseline):
                                    ptr(mean), ptr(std), ptr(got), s))
     # exp(t + ln B) with |t + ln B| < 30: 2 ulp of its argument
     np.testing.assert_allclose(got.cpu().numpy(), want.cpu().numpy(), rtol=4e-6, atol=1e-7)
+
+
+def _bf16(v):
+    u = np.ascontiguousarray(v, np.float32).view(np.uint32)
+    return (((u + 0x7fff + ((u >> 16) & 1)) >> 16) << 16).astype(np.uint32).view(np.float32)
+
+
+def _pair(a):
+    """hi + lo, the two BF16 terms that an activation is kept in."""
+    a = np.float32(a)
+    h = _bf16(a)
+    return h.astype(np.float64) + _bf16(a - h)
+
+
+def test_silu_error(gpu):
+    """SiLU of the fused kernel, read back through a last layer that is the identity:
+    weights 0 and bias z in the first.  The pair of BF16 terms hides an error unless
+    it moves a value over a rounding boundary, so the values that differ from the
+    exact ones' pairs are counted: at most as many as the stated bound (4.1e-7 at
+    z = -87, relative) moves when every value is off by it.  Large arguments keep
+    their limits."""
+    from geosmie_amd import _lib
+    from geosmie_amd.surrogate import MLP
+    dims, w = (1, 256, 256), 256
+    p = np.zeros(O.layout(dims)[1], np.float32)
+    (_, b0, _, _), (w1, _, _, _) = O.layout(dims)[0]
+    p[w1:w1 + w * w] = np.eye(w, dtype=np.float32).ravel()
+    x = _lib.to_dev(np.ones((1, 1)), np.float32)
+
+    def run(z):
+        p[b0:b0 + w] = z
+        return MLP(dims, params=p).forward(x).cpu().numpy()[0].astype(np.float64)
+    z = np.linspace(-87.0, -30.0, 32 * w).astype(np.float32)
+    got = np.concatenate([run(c) for c in z.reshape(-1, w)])
+    exact = z / (1.0 + np.exp(-z.astype(np.float64)))
+    moved = (_pair(exact * (1.0 + 4.1e-7)) != _pair(exact)).mean()
+    assert (got != _pair(exact)).mean() <= moved
+    z = np.linspace(-30.0, 30.0, w).astype(np.float32)
+    exact = z / (1.0 + np.exp(-z.astype(np.float64)))
+    assert np.all(np.abs(run(z) - exact) <= (2.0 ** -17 + 3e-7) * np.abs(exact))
+    z = np.resize(np.float32([-3e38, -1e4, -104.0, -88.0, 0.0, 104.0, 1e4, 3e38]), w)
+    got = run(z)
+    assert np.all(np.abs(got - np.maximum(z, 0)) <= 2.0 ** -17 * np.maximum(z, 0) + 1e-35)
+    z[3] = np.nan
+    assert np.isnan(run(z)).all()
