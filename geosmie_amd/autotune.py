@@ -8,14 +8,16 @@ cache per (device, workload name) and reused without timing.
 
 Knobs (include/geosmie.h, enum gm_tune_param):
   mie_grid_mult  persistent Mie grid as a multiple of the resident wavefronts
-  s12_waves      wavefronts (64 angles each) per FP32 / split-BF16 S1/S2 block
-  psd_chunk      points per split-K chunk of the few-PSD contraction
+  s12_waves      wavefronts (64 angles each) per split-BF16 S1/S2 block
+  psd_chunk      points per split-K chunk of the contraction of few PSDs with more than
+                 16 columns
   s12_points     kept for saved settings; no effect
   mie_waves      register budget of the Mie recurrence kernels (0 unconstrained,
                  3 or 4 resident wavefronts per SIMD)
   s12_layout     kept for saved settings; no effect
-  mie_ckpt       coated kernel, one point per lane: downward-chain states kept every 4, 5 or 8 rows and
-                 regenerated per block in LDS, or every row kept in scratch (0);
+  mie_ckpt       coated kernel, one point per lane: downward-chain states kept every 4,
+                 5 or 8 rows and regenerated per block in LDS, or every row kept in
+                 scratch (0);
                  non-zero also selects the checkpointed lane-per-point
                  homogeneous kernel (every 4 rows)
   coated_lanes   coated kernel: lanes per point, as mie_lanes
@@ -97,7 +99,7 @@ def store_cache(path, entry_key, choices):
     os.replace(tmp, path)
 
 
-def tune(ctx, workload, knobs=("mie_grid_mult", "s12_points", "s12_waves", "psd_chunk"), reps=3,
+def tune(ctx, workload, knobs=("mie_grid_mult", "psd_chunk"), reps=3,
          warmup=1, candidates=None, cache_key=None, cache=None, tie=0.0):
     """Returns {knob: {"best": value, "ms": {value: ms per pass}}}; the context
     keeps the best values.  With cache_key (a name for the workload), choices

@@ -1,6 +1,6 @@
 """Launch-shape knobs change timing only: results are bitwise identical for
-every persistent-grid multiple and S1/S2 block width, and the autotuner
-leaves a valid setting on the context."""
+every persistent-grid multiple and split-BF16 S1/S2 block width, and the
+autotuner leaves a valid setting on the context."""
 import numpy as np
 import pytest
 
@@ -8,24 +8,22 @@ pytestmark = pytest.mark.gpu
 
 
 def test_knobs_do_not_change_results(gpu):
+    """The persistent Mie grid's multiple, and at split BF16 the wavefronts per S1/S2
+    block: the same bits."""
     from geosmie_amd import _lib, autotune
     from geosmie_amd.mie import mie_batch
     from geosmie_amd.s12 import s12_batch
     h = _lib.ctx()
     x = np.logspace(-2, 2.5, 700)
     ref = None
-    for mult, waves, pts, lay in [(1, 4, 8, 0), (2, 4, 8, 0), (4, 4, 8, 0), (1, 1, 8, 0),
-                                  (1, 2, 16, 0), (2, 4, 16, 0), (1, 1, 16, 0), (1, 4, 8, 1),
-                                  (1, 2, 8, 1), (1, 4, 16, 1), (1, 1, 16, 1), (1, 4, 8, 2),
-                                  (2, 1, 16, 2)]:
+    cost = np.cos(np.radians(np.linspace(0, 180, 300)))
+    for mult, waves in [(1, 4), (2, 2), (4, 1), (1, 1)]:
         autotune.set_knob(h, "mie_grid_mult", mult)
         autotune.set_knob(h, "s12_waves", waves)
-        autotune.set_knob(h, "s12_points", pts)
-        autotune.set_knob(h, "s12_layout", lay)
         r = mie_batch(x, m=1.5 + 0.02j, coeffs=True)
-        s1, s2 = s12_batch(r["an"][::37], r["bn"][::37],
-                           cost=np.cos(np.radians(np.linspace(0, 180, 300))))
-        got = (np.stack([r[k] for k in ("qext", "qsca", "asy")]), s1, s2)
+        got = [np.stack([r[k] for k in ("qext", "qsca", "asy")])]
+        for precision in (0, 2):
+            got += s12_batch(r["an"][::37], r["bn"][::37], cost=cost, precision=precision)
         if ref is None:
             ref = got
         else:
@@ -33,8 +31,6 @@ def test_knobs_do_not_change_results(gpu):
                 assert np.array_equal(a, b)
     autotune.set_knob(h, "mie_grid_mult", 1)
     autotune.set_knob(h, "s12_waves", 4)
-    autotune.set_knob(h, "s12_points", 8)
-    autotune.set_knob(h, "s12_layout", 0)
 
 
 def test_mie_register_variants_agree(gpu):
@@ -83,6 +79,7 @@ def test_tune_picks_a_candidate(gpu):
     ch = RunopticsChain(x, 1.5 + 0.01j, np.linspace(0, 180, 181), w / w.sum(), [0.55],
                         [(0, x.size)])
     res = autotune.tune(ch.ctx, ch.step, reps=2)
+    assert not set(res) & {"s12_points", "s12_layout", "s12_waves"}   # nothing to time at FP64
     for name, r_ in res.items():
         assert r_["best"] in autotune.KNOBS[name][1]
         assert autotune.get(ch.ctx, name) == r_["best"]
