@@ -1,10 +1,11 @@
 """Small coated batches with 16, 32 or 64 lanes per point, against the shell
 combination in extended precision (64-bit mantissa) on a sample of the points.
 
-The tolerance is the 1e-9 of every comparison with the oracle, doubled for the
-sampled points' own conditioning (rounded m x, m y next to a resonance): |a_n|, |b_n| <= 1
-absolute, efficiencies relative, g absolute.  Against the same points one per lane: the same points are NaN (series that
-overflow, tiny cores in large shells), and the other classes are unchanged.
+The kernel's largest errors on these points are 1.8e-11 in a_n, b_n (rounded m x, m y
+next to a resonance) and 4.7e-13 in the efficiencies and g; asserted are 1e-10 and
+5e-12: |a_n|, |b_n| <= 1 absolute, efficiencies relative, g absolute.  Against the same
+points one per lane: the same points are NaN (series that overflow, tiny cores in
+large shells), and the other classes are unchanged.
 """
 import numpy as np
 import pytest
@@ -122,7 +123,7 @@ def test_lanes_per_point(gpu, n, y_hi, q_lo, sort):
         a, b = _exact(x[i], y[i], (m1 ** 2)[i], (m2 ** 2)[i])
         for z, r in ((an, a), (bn, b)):
             d = np.abs(z[off[i]:off[i + 1]] - r)
-            assert np.all(np.isnan(d) | (d <= 2e-9)), i
+            assert np.all(np.isnan(d) | (d <= 1e-10)), i
         if np.isnan(props[0, i]):
             continue
         k = np.arange(1, a.size + 1)
@@ -131,16 +132,18 @@ def test_lanes_per_point(gpu, n, y_hi, q_lo, sort):
         asy = (((2 * k + 1) / (k * (k + 1)) * (a * b.conj()).real).sum()
                + (k * (k + 2) / (k + 1) * (a * np.append(a[1:], 0).conj()
                                            + b * np.append(b[1:], 0).conj()).real).sum())
-        assert abs(props[0, i] - ext) <= 2e-9 * ext and abs(props[1, i] - sca) <= 2e-9 * sca, i
-        assert abs(props[4, i] - 4 * asy / (sca * y[i] ** 2)) <= 2e-9, i
+        assert abs(props[0, i] - ext) <= 5e-12 * ext and abs(props[1, i] - sca) <= 5e-12 * sca, i
+        assert abs(props[4, i] - 4 * asy / (sca * y[i] ** 2)) <= 5e-12, i
 
 
 # above 24576 points one per lane: the split of the longest (skewed sizes; 16 and, from
-# 1200 rows on, 64 lanes) and of every point (uniform long series)
-@pytest.mark.parametrize("y_lo, y_hi, skew", [(0.02, 209.0, True), (600.0, 700.0, False),
-                                              (1.0, 2000.0, None)])
-def test_long_points_of_a_batch(gpu, y_lo, y_hi, skew):
-    got, want = _both(24576 + 1, y_lo, y_hi, skew)
+# 1200 rows on, 64 lanes) and of every point (uniform long series); more than 512k
+# points, which only look for a split where series reach 512 rows
+@pytest.mark.parametrize("n, y_lo, y_hi, skew", [
+    (24577, 0.02, 209.0, True), (24577, 600.0, 700.0, False), (24577, 1.0, 2000.0, None),
+    (512 * 1024 + 1, 1.0, 600.0, None)])
+def test_long_points_of_a_batch(gpu, n, y_lo, y_hi, skew):
+    got, want = _both(n, y_lo, y_hi, skew)
     # an absorbing core needs no start correction: both forms hold 1e-9
     for a, b in zip(got, want):
         assert _torch().equal(_torch().isnan(a), _torch().isnan(b))

@@ -3,8 +3,8 @@
 1. FP64 S1/S2 at series lengths up to 2147 (size parameters 250-2094, the
    large-x workload's refractive-index range) against sums carried out in
    mpmath on 12 angles from exact forward to exact back scattering
-   (tests/golden/mp_largex_vectors.npz), for every launch shape the
-   autotuner can choose, and against the numpy oracle on 1801 angles.
+   (tests/golden/mp_largex_vectors.npz), for every shape that the batch
+   size and the angles can select, and against the numpy oracle on 1801 angles.
    The fused S1/S2 -> Mueller -> row-sum kernel is checked on the same
    coefficients.
 2. Coated spheres whose shell is denser than the core (|m2| >= |m1|), where
@@ -33,19 +33,6 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 MPL = np.load(os.path.join(HERE, "golden", "mp_largex_vectors.npz"))
 
 
-def _with_knobs(knobs, fn):
-    from geosmie_amd import _lib, autotune
-    h = _lib.ctx()
-    old = {k: autotune.get(h, k) for k in knobs}
-    try:
-        for k, v in knobs.items():
-            autotune.set_knob(h, k, v)
-        return fn()
-    finally:
-        for k, v in old.items():
-            autotune.set_knob(h, k, v)
-
-
 def _homog_coeffs():
     from geosmie_amd.mie import mie_batch
     return mie_batch(MPL["hx_x"], m=MPL["hx_m"], coeffs=True)
@@ -61,28 +48,43 @@ def test_large_x_efficiencies_vs_mp(gpu):
     assert np.abs(r["asy"] - ref[:, 4]).max() < 1e-9
 
 
-SHAPES = [{"s12_layout": lay, "s12_points": pts, "s12_waves": wv}
-          for lay in (0, 1, 2) for pts in (8, 16) for wv in ((1, 4) if lay < 2 else (4,))]
+# (copies of the 20 points, of the 12 angles): the angle tables read as they are up to
+# 4080 points, as pairs from 4096 on, the tiles sorted by length from 16384 on; 16, 32 or
+# 64 angles per wavefront (as many as leave 8192 wavefronts)
+SHAPES = {"raw16": (1, 1), "raw32": (204, 90), "raw64": (204, 172), "pairs16": (210, 1),
+          "pairs32": (210, 90), "pairs64": (210, 180), "sorted16": (820, 3), "sorted64": (820, 40)}
 
 
-@pytest.mark.parametrize("shape", SHAPES, ids=["layout%d-pts%d-waves%d" % (s["s12_layout"],
-                                                                          s["s12_points"],
-                                                                          s["s12_waves"])
-                                               for s in SHAPES])
+@pytest.mark.parametrize("shape", SHAPES)
 def test_s12_fp64_large_x_vs_mp(gpu, shape):
     """S1/S2 within 1e-11 of max|S| of the mpmath sums (float64 rounding of
     ~2000-term sums is ~5e-13 there)."""
-    from geosmie_amd.s12 import s12_batch
+    import torch
+    from geosmie_amd import _lib
+    from geosmie_amd._lib import ptr
+    from geosmie_amd.s12 import _coef_dev, angle_tables_dev
+    copies, angles = SHAPES[shape]
     r = _homog_coeffs()
-    cost = np.cos(np.radians(MPL["theta"]))
-    s1, s2 = _with_knobs(shape, lambda: s12_batch(r["an"], r["bn"], cost=cost))
+    off, nmax, an, bn = _coef_dev(r["an"], r["bn"])
+    n, total = copies * nmax.numel(), int(off[-1])
+    an, bn, nmax = an.repeat(copies), bn.repeat(copies), nmax.repeat(copies)
+    off = torch.cat([(torch.arange(copies, device="cuda")[:, None] * total + off[None, :-1]).ravel(),
+                     torch.tensor([copies * total], device="cuda")])
+    cost = np.tile(np.cos(np.radians(MPL["theta"])), angles)
+    pi_t, tau_t = angle_tables_dev(cost, int(r["nmax"].max()))
+    s1 = torch.empty((n, cost.size), dtype=torch.complex128, device="cuda")
+    s2 = torch.empty_like(s1)
+    _lib.check(_lib.lib().gm_mie_s12(_lib.ctx(), n, ptr(off), ptr(nmax), ptr(an), ptr(bn), cost.size,
+                                     ptr(pi_t), ptr(tau_t), int(pi_t.shape[0]),
+                                     ptr(torch.view_as_real(s1)), ptr(torch.view_as_real(s2)), 0,
+                                     _lib.stream()), "gm_mie_s12")
+    ref = [torch.from_numpy(MPL[k]).to("cuda") for k in ("hx_s1", "hx_s2")]
+    scale = torch.maximum(ref[0].abs().amax(1), ref[1].abs().amax(1))[None, :, None, None]
     worst = 0.0
-    for i in range(s1.shape[0]):
-        scale = max(np.abs(MPL["hx_s1"][i]).max(), np.abs(MPL["hx_s2"][i]).max())
-        e1 = np.abs(s1[i] - MPL["hx_s1"][i]).max() / scale
-        e2 = np.abs(s2[i] - MPL["hx_s2"][i]).max() / scale
-        assert max(e1, e2) < 1e-11, (i, MPL["hx_x"][i], MPL["hx_m"][i], e1, e2)
-        worst = max(worst, e1, e2)
+    for s, e in zip((s1, s2), ref):
+        err = (s.view(copies, -1, angles, 12) - e[None, :, None, :]).abs() / scale
+        worst = max(worst, float(err.max()))
+    assert worst < 1e-11
     print("%s: max error / max|S| vs mpmath = %.2e" % (shape, worst))
 
 
