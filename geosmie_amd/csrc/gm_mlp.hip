@@ -291,8 +291,8 @@ __global__ void k_mlp_adam(int64_t n, float* __restrict__ p, const float* __rest
 // queries, so a weight fragment it loads (16 bytes a lane, laid out for that
 // by k_mlp_split_weights) feeds four products per term.  64 rows: 67 KB of
 // planes, two blocks per CU, so one block's SiLU can run under the other's
-// products.  1M queries (6-256-256-256-256-35, two-term weights): 5284 -> 1640
-// us, MFMA 36% busy, the SiLU and splits about as many VALU cycles as the
+// products.  1M queries (6-256-256-256-256-35, two-term weights): 5284 -> 1556
+// us, MFMA 34% busy, the SiLU and splits more VALU cycles than the
 // products take; the products alone are 0.59 ms of matrix-core time.
 //
 // Training runs the same block forward and back: dZ_l takes the activations'
@@ -340,23 +340,21 @@ __device__ __forceinline__ void bf_split(float v, __bf16& h, __bf16& l) {
 }
 
 // SiLU(z) = z / (1 + exp(-z)), and in training its derivative, on the hardware exp2 and
-// reciprocal (1 ulp each), both corrected: the exponential by what rounding
-// z log2 e left out, the quotient by its residual.  Largest error of SiLU against 64 bits,
-// relative, for z in -87..-30 / -10..-4 / 0..1: 4.1e-7 / 2.1e-7 / 1.2e-7, where expf and a
-// division as compiled here have 2.8e-6 / 4.6e-7 / 1.3e-7 and the bare instructions
-// 3.9e-6 / 5.9e-7 / 1.8e-7.  Zero below -87 (1e-36).  12 instructions a value, the bare ones
-// 5, and the epilogue is as long as the products: 1M queries 1640 us with these, 1500
-// bare, 1731 with expf and a Newton step.
+// reciprocal (1 ulp each): log2 e in two terms, the quotient corrected by its residual.
+// Largest relative error of SiLU against 64 bits for z in -87..-30 / -10..-4 / 0..10: 2.75e-6
+// / 4.52e-7 / 1.25e-7, where expf and a division as compiled here have 2.76e-6 / 4.59e-7
+// / 1.26e-7 and the bare instructions 3.89e-6 / 5.91e-7 / 1.82e-7.  The bound on exp
+// leaves z * 0 for z below -87 (1e-36) with a finite residual.  The epilogue is as long as
+// the products: 1M queries 1556 us, 1486 with the bare instructions, 1731 with expf and
+// a Newton step.
 template <bool GRAD>
 __device__ __forceinline__ void silu_hw(float z, float& a, float& d) {
-  const float zc = __builtin_amdgcn_fmed3f(z, -87.0f, 104.0f), t = zc * -1.44269504088896341f;
-  float e = __builtin_amdgcn_exp2f(t);
-  e = fmaf(e, fmaf(t, -0.693147180559945309f, -zc), e);
-  const float den = 1.0f + e, i = __builtin_amdgcn_rcpf(den);
-  const float n = z < -87.0f ? 0.0f : z, q = n * i;
-  a = fmaf(fmaf(-den, q, n), i, q);
+  const float t = fmaf(z, -1.44269502162933349609375f, z * -1.92596299112661746887e-8f);
+  const float e = fminf(__builtin_amdgcn_exp2f(t), 3.402823466e38f);
+  const float den = 1.0f + e, i = __builtin_amdgcn_rcpf(den), q = z * i;
+  a = fmaf(fmaf(-den, q, z), i, q);
   if (GRAD) {
-    const float s = z < -87.0f ? 0.0f : fmaf(fmaf(-den, i, 1.0f), i, i);
+    const float s = fmaf(fmaf(-den, i, 1.0f), i, i);
     d = s * (1.0f + z * (1.0f - s));
   }
 }
@@ -1023,8 +1021,9 @@ int grad_fused(gm_ctx* ctx, const Net& net, const gm::FuseNet& f, int terms, int
     fg.units += ((f.nt[l] * 16 + 63) / 64) * ((f.kt[l] * 32 + 63) / 64);
   }
   fg.first[f.L] = fg.units;
-  // about four wavefronts per CU over the weight tiles, at least four K steps each;
-  // whole rounds of the eight XCDs
+  // about four wavefronts per CU over the weight tiles, four K steps or more each
+  // before the splits are rounded up to whole rounds of the eight XCDs (a small batch's
+  // get fewer, or none and write zeros)
   fg.groups = nb * (kFuseMtTrain / 2);
   const int64_t want = std::max<int64_t>(1, std::min<int64_t>((4 * ctx->n_cu + fg.units - 1) / fg.units,
                                                               fg.groups / 4));
