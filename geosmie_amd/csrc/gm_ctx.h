@@ -32,9 +32,9 @@ struct gm_ctx {
   size_t scratch_budget = (size_t)3 << 30;       // bytes of recurrence scratch
   // launch shapes chosen by gm_ctx_tune (an autotuner's knobs)
   int tune_mie_grid_mult = 1;   // persistent Mie grid = multiple of resident wavefronts
-  int tune_s12_waves = 4;       // wavefronts (64 angles each) per FP32 / split-BF16 S1/S2 block
+  int tune_s12_waves = 4;       // wavefronts (64 angles each) per split-BF16 S1/S2 block
   int tune_s12_points = 8;      // accepted, no effect
-  int tune_psd_chunk = 128;     // points per split-K chunk of the few-PSD contraction
+  int tune_psd_chunk = 128;     // points per split-K chunk, few PSDs and > 16 columns
   int tune_mlp_wterms = 1;      // BF16 terms per MLP weight (1 = BF16 weights, 2 = hi + lo)
   int tune_mie_waves = 0;       // Mie register variant: 0 unconstrained, 3 or 4 waves per SIMD
   int tune_s12_layout = 0;      // accepted, no effect
@@ -43,7 +43,7 @@ struct gm_ctx {
   int tune_coated_lanes = 0;    // coated kernel: lanes per point (1, 16, 32, 64; 0 = by batch)
   int psd_quirks = 1;           // integratePSD quirks reproduced (GM_PSD_QUIRK_* bits)
   int tune_s12_share = 1;        // split-BF16 fused S1/S2: angle-table tiles shared through LDS
-  int tune_s12_row_tiles = 0;    // reduced-precision fused S1/S2: 8-point tiles per wave (0 = auto)
+  int tune_s12_row_tiles = 0;    // fused S1/S2 row sums: tiles per work unit (0 = auto)
   Buf status;                                    // int32 flags + scan scratch
   Buf order, key, hist, scratch, scan_tmp;
   Buf tab_pi, tab_tau, gemm_tmp, feat_tmp, gsf_tab, tab_lp, lut_tmp, mlp_ws;

@@ -1488,9 +1488,9 @@ __global__ __launch_bounds__(64, MINW) void k_mie_coated_stable(
 // ratios of v, w, y downward; psi and chi of v, w, y upward) are joined across
 // the lanes by scans of their transfer matrices.  A batch of a few thousand
 // points is otherwise a few dozen wavefronts, each as long as its longest
-// point: 1266 points to y = 209 took 305 us a call on 20 of 1024 SIMDs, 56 with 32
-// lanes a point.  What bounds it then is the scans' fixed cost, about 20 us a
-// wavefront, and their full matrix products: two to three times the serial
+// point: 1266 points to y = 209 took 305 us a call on 20 of 1024 SIMDs, 49 with 32
+// lanes a point.  What bounds it then is the scans' and the set-up's fixed cost (64 points
+// of y = 2 take 28 us, of y = 200 29) and the scans' full matrix products: two to three times the serial
 // instructions for a series of 200 rows, so a batch that fills the chip runs one
 // point per lane.  Largest |a_n| errors against extended precision (2048 points,
 // y to 400): 1.8e-11 here, 2.8e-9 one point per lane (the start-index correction

@@ -7,9 +7,9 @@
 // real GEMMs  [Re U; Im U](2P x K) x P(K x N_ang)  and the same for V, M, with
 // K = n (ragged per point, zero-padded to the tile maximum).
 //
-// FP64 path: v_mfma_f64_16x16x4_f64.  A wavefront owns 16 points (one row tile of
-// real and one of imaginary parts) x 16 TT angles and walks K in steps of 4.
-// Operand layouts of v_mfma_f64_16x16x4_f64 (measured on gfx950):
+// FP64 and FP32 paths: v_mfma_f64_16x16x4_f64 and v_mfma_f32_16x16x4_f32.  A wavefront
+// owns 16 points (one row tile of real and one of imaginary parts) x 16 TT angles
+// and walks K in steps of 4.  Operand layouts (measured on gfx950):
 // A[i][k] from lane i + 16k, B[k][j] from lane j + 16k, D[g + 4r][j] in lane
 // j + 16g, element r  (the f32/bf16 16x16 variants use D[4g + r][j] instead).
 // Epilogue modes: write S1, S2 (complex), or the four independent Mueller
@@ -20,12 +20,11 @@
 //   BF16X3  v_mfma_f32_16x16x32_bf16 on split operands x = x_hi + x_lo (both
 //           BF16, x_lo = bf16(x - x_hi)); U P ~ U_hi P_hi + U_hi P_lo + U_lo P_hi
 //           (the lo*lo term, ~2^-18 relative, is dropped), FP32 accumulation.
-// Both read P, M from a per-call table (k_s12_prep_tables) padded to whole
-// K-steps and 64-angle tiles, so the inner loops carry no bounds tests on it.
-// f32 / bf16 16x16 results land as D[4g + r][j] in lane j + 16g, element r;
-// A row i is then point p0 + (i >> 1), component i & 1, which gives the same
-// per-lane element order as the FP64 kernel: (0,1) = point p0 + 2g (re, im),
-// (2,3) = point p0 + 2g + 1.
+// They read P, M from a per-call table padded to whole K-steps and angle tiles
+// (FP32 k_s12_prep_pairs32, BF16X3 k_s12_prep_tables), so the inner loops carry no
+// bounds tests on it.  BF16X3 tiles are 8 points, real and imaginary parts in
+// turn: A row i is point p0 + (i >> 1), component i & 1, and a lane's four results
+// are (re, im) of points p0 + 2g and p0 + 2g + 1.
 #include <algorithm>
 #include <type_traits>
 
@@ -224,7 +223,7 @@ __device__ __forceinline__ void s12_tile64(const S12Tables& T, int64_t p0, int64
 }
 
 constexpr int kRowsPerCall = 64;   // rows per call (range arrays passed by value)
-constexpr int kRowsWaves = 4;      // wavefronts (64 angles each) per block
+constexpr int kRowsWaves = 4;      // most wavefronts per block
 
 struct RowGroups {
   int n_groups;

@@ -85,9 +85,10 @@ int gm_ctx_check(gm_ctx* ctx, gm_stream stream, int32_t* flags_host);
  * budgets let the compiler fuse a different set of multiply-adds. */
 enum gm_tune_param {
   GM_TUNE_MIE_GRID_MULT = 0,  /* persistent Mie grid = this x resident wavefronts (1..16; 1) */
-  GM_TUNE_S12_WAVES = 1,      /* wavefronts of 64 angles per S1/S2 block at FP32 and split-BF16
-                                   (1, 2, 4; 4); FP64 chooses from the sizes */
-  GM_TUNE_PSD_CHUNK = 2,      /* points per split-K chunk, few-PSD contraction (16..2^20; 128) */
+  GM_TUNE_S12_WAVES = 1,      /* wavefronts of 64 angles per S1/S2 block at split-BF16 (1, 2, 4;
+                                   4); FP64 and FP32 choose from the sizes */
+  GM_TUNE_PSD_CHUNK = 2,      /* points per split-K chunk of the contraction of few PSDs with more
+                                   than 16 columns and of gm_psd_contract_rows (16..2^20; 128) */
   GM_TUNE_MLP_WEIGHT_TERMS = 3, /* precision, not shape: BF16 terms per MLP weight on the matrix
                                    cores, 1 = BF16 weights (default), 2 = hi + lo BF16 pair */
   GM_TUNE_S12_POINTS = 4,       /* accepted (8, 16; 8), no effect: the FP64 S1/S2 kernel takes 16
@@ -115,7 +116,7 @@ enum gm_tune_param {
                                    quirks gm_integrate_psd[_rows] reproduce (GM_PSD_QUIRK_* bits;
                                    default GM_PSD_QUIRK_ALIAS) */
   GM_TUNE_S12_ROW_TILES = 10,   /* gm_s12_contract_rows: tiles per work unit (1, 2, 4): at FP64
-                                   16-point tiles one after the other, at FP32 / split-BF16
+                                   and FP32 16-point tiles one after the other, at split-BF16
                                    8-point tiles multiplied together, sharing each angle-table
                                    fetch; 0 (default) = by batch size.  Results agree to rounding */
   GM_TUNE_S12_SHARE = 11        /* gm_s12_contract_rows at split-BF16 with one tile per work
