@@ -1186,8 +1186,10 @@ constexpr int64_t kS12Want = 8192;
 // FP32: up to 128 angles per wavefront where a and b are read as FP64 (1.5M points x
 // 371 angles 10.49 against 11.03 ms at 64; 60k points, 11k wavefronts, 1.97 against
 // 1.87), 64 where they come converted (40k x 1801 1.73 against 1.75 ms at 128).
-// 64 angles from 10k wavefronts on (60k points x 181 angles, 11k: amplitudes 127 against
-// 148 us at 32, to x = 1000 691 against 806; 5k points x 1801 angles, 9k: 186 against 168).
+// Where they are read as FP64, 64 angles from 10k wavefronts on (60k points x 181 angles,
+// 11k: amplitudes 127 against 148 us at 32, to x = 1000 691 against 806; 5k points x
+// 1801 angles, 9k: 186 against 168); the row sums of 4k points x 1801 angles, whose rows'
+// tiles count 15k, take 53.5 us at 64 and 49.9 at 32.
 constexpr int64_t kS12Want32 = 16384;
 constexpr int64_t kS12Want32Half = 10240;
 constexpr int64_t kS12PairTiles = 256;
@@ -1213,10 +1215,10 @@ S12Shape s12_shape(int64_t tiles, int n_ang, int64_t want, int max_tt = 4) {
 }
 
 // FP32: 32, 64 or 128 angles per wavefront, always on the paired tables.
-S12Shape s12_shape32(int64_t tiles, int n_ang, int max_tt) {
+S12Shape s12_shape32(int64_t tiles, int n_ang, int max_tt, int64_t want4) {
   S12Shape h = s12_shape(tiles, n_ang, kS12Want32, max_tt);
   if (h.tt < 4) {
-    const int tt = tiles * ((n_ang + 63) / 64) >= kS12Want32Half ? 4 : 2;
+    const int tt = tiles * ((n_ang + 63) / 64) >= want4 ? 4 : 2;
     const int waves = (n_ang + 16 * tt - 1) / (16 * tt);
     h.tt = tt;
     h.ablocks = (waves + 3) / 4;
@@ -1312,7 +1314,7 @@ int launch_s12(gm_ctx* ctx, const char* who, int64_t n, const int64_t* off, cons
     ctx->mark_begin(gm::kKS12, s, &slot);
     const int64_t units = (n + 15) / 16;
     S12Shape h = precision == GM_PREC_FP64 ? s12_shape(units, n_ang, kS12Want)
-                                           : s12_shape32(units, n_ang, 8);
+                                           : s12_shape32(units, n_ang, 8, kS12Want32Half);
     gm::S12Tables T;
     const int* order;
     gm::RowGroups none{};
@@ -1442,7 +1444,7 @@ int gm_s12_contract_rows(gm_ctx* ctx, int64_t n, const int64_t* coef_off, const 
   for (int r = 1; r < n_rows; ++r)
     many |= start_host[r] == start_host[r - 1] && count_host[r] == count_host[r - 1];
   S12Shape h64 = precision == GM_PREC_FP64 ? s12_shape((tiles + 1) / 2, n_ang, kS12Want)
-                                           : s12_shape32((tiles + 1) / 2, n_ang, 4);
+                                           : s12_shape32((tiles + 1) / 2, n_ang, 4, kS12Want32);
   int64_t per = 1;
   while (per < 8 && nmax_cap <= 256 &&
          (tiles / 2) / (2 * per) * h64.ablocks * h64.wpb >= 2 * kS12Want)
