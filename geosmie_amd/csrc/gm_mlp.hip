@@ -960,12 +960,16 @@ int fuse_launch(const gm::FuseNet& f, int terms, int64_t n, const float* params,
 
 // Whether the forward pass runs fused: not for one layer, and not for two with at most
 // 64 features between them, where the activations kept out of memory do not pay for
-// splitting the weights and padding the rows.  us fused / layer by layer, 16k and
-// 400k queries: 256-256 41 / 18 and 682 / 480; 64-64-64 16 / 15 and 159 / 117; 6-32-3
-// 15.5 / 14.1 and 74 / 72; 6-64-3 15.5 / 14.0, but 78 / 87; 6-128-3 15.6 / 16.3 and 94 /
-// 152; 6-32-32-3 15.5 / 19.3 and 93 / 107.
-bool fuse_forward_pays(const Net& net) {
-  return net.L > 2 || (net.L == 2 && net.dims[1] > 64);
+// splitting the weights and padding the rows, unless those are most of a large batch's
+// traffic.  us fused / layer by layer, 16k and 400k queries: 256-256 41 / 18 and 682 /
+// 480; 64-64-64 16 / 15 and 159 / 117; 6-64-35 15.6 / 14.7 and 108 / 100; 6-32-3 15.5 /
+// 14.1 and 74 / 72; 6-64-3 15.5 / 14.0, but 78 / 87; 6-48-8 15.6 / 14.2, but 81 / 95;
+// 6-128-3 15.6 / 16.3 and 94 / 152; 6-32-32-3 15.5 / 19.3 and 93 / 107.
+bool fuse_forward_pays(const Net& net, int64_t n) {
+  if (net.L != 2) return net.L > 2;
+  const int hidden = net.dims[1];
+  return hidden > 64 ||
+         (hidden > 32 && net.dims[0] <= 16 && net.dims[2] <= 16 && n >= 64 * 1024);
 }
 
 // y = net(x), or (post.on) the surrogate's table rows from it.
@@ -976,7 +980,7 @@ int forward_any(gm_ctx* ctx, const Net& net, int64_t n, const float* params, con
   gm::FuseNet f;
   size_t slot;
   *posted = false;
-  if (fuse_forward_pays(net) && fuse_net(net, terms, f)) {
+  if (fuse_forward_pays(net, n) && fuse_net(net, terms, f)) {
     if ((rc = ctx->reserve(ctx->mlp_ws, (size_t)f.n_frag * 64 * terms * sizeof(uint4)))) return rc;
     uint4* frag = (uint4*)ctx->mlp_ws.ptr;
     ctx->mark_begin(gm::kKMlp, s, &slot);

@@ -476,7 +476,8 @@ int gm_surrogate_post(gm_ctx* ctx, int64_t n, int n_out, const float* q, double 
 /* gm_mlp_forward followed by gm_surrogate_post: table rows [n][dims[n_layers]]
  * of network features x (gm_surrogate_prep) and their queries q, in one pass
  * where the network is at most 256 wide and runs fused (three layers or more, or two
- * with more than 64 features between them). */
+ * with more than 64 features between them; a large batch with few inputs and outputs
+ * with more than 32). */
 int gm_surrogate_rows(gm_ctx* ctx, int n_layers, const int* dims, int64_t n, const float* params,
                       const float* x, const float* q, double m_water_re, const float* tgt_mean,
                       const float* tgt_std, float* rows, gm_stream stream);

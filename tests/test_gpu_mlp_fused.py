@@ -25,10 +25,12 @@ def _setup(dims, n):
 
 # rows around one and two 64-row blocks; widths at and past the 16-, 32-, 64- and
 # 128-feature splits of the wavefronts; 257 (layer by layer), and one layer and two
-# with 33 or 64 features between them (forward layer by layer, gradients fused)
+# with 33, 48 or 64 features between them (forward layer by layer but for the large
+# batch with few inputs and outputs, gradients fused)
 @pytest.mark.parametrize("dims,n", [((6, 256, 35), 63), ((6, 256, 35), 64), ((32, 33, 16), 65),
                                     ((33, 128, 129, 3), 128), ((256, 65, 256), 129),
                                     ((5, 7), 200), ((256, 256), 70), ((6, 64, 35), 65),
+                                    ((6, 48, 8), 65535), ((6, 48, 8), 65536),
                                     ((32, 33, 20, 16), 65), ((5, 7, 7, 7), 200),
                                     ((6, 257, 4), 65)])
 def test_tile_edges_vs_oracle(gpu, dims, n):
