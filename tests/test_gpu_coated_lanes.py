@@ -185,3 +185,26 @@ def _both(n, y_lo, y_hi, skew):
     h, ref = _lib.private_ctx(), _lib.private_ctx()
     set_knob(ref, "coated_lanes", 1)
     return _run(h, x, y, m1, m2, True), _run(ref, x, y, m1, m2, True)
+
+
+# the lanes per point set by hand, on a batch that runs one per lane by itself
+@pytest.mark.parametrize("lanes", [16, 32, 64])
+def test_lanes_set_by_hand(gpu, lanes):
+    from geosmie_amd import _lib
+    from geosmie_amd.autotune import get, set_knob
+    n = 30001
+    rng = np.random.default_rng(lanes)
+    y = np.exp(rng.uniform(np.log(0.02), np.log(60.0), n))
+    x = y * rng.uniform(0.3, 0.9, n)
+    m1, m2 = np.full(n, 1.95 + 0.79j), np.full(n, 1.4 + 0j)
+    h, ref = _lib.private_ctx(), _lib.private_ctx()
+    set_knob(h, "coated_lanes", lanes)
+    set_knob(ref, "coated_lanes", 1)
+    assert get(h, "coated_lanes") == lanes
+    got, want = _run(h, x, y, m1, m2, True), _run(ref, x, y, m1, m2, True)
+    for a, b in zip(got[:2], want[:2]):
+        assert _torch().equal(_torch().isnan(a), _torch().isnan(b))
+        assert float(_torch().nan_to_num(a - b).abs().max()) <= 2e-9
+    for q in (0, 1, 4):
+        rel = _torch().nan_to_num((got[2][q] - want[2][q]) / want[2][q])
+        assert float(rel.abs().max()) <= 2e-9, q
